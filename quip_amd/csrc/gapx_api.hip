@@ -507,7 +507,14 @@ static int model_upload(gapx_model *m) {
                               xp.begin() + (size_t)r * dp);
                 CHK(upload(c->d_XsP, xp.data(), xp.size() * 8));
             }
-            CHK(upload(c->d_rb, c->rb.data(), c->rb.size() * 8));
+            std::vector<double> rb(c->rb);   // and the radial tables of soap_dev
+            rb.resize(c->n + 24, 0.0);
+            const double alpha = 0.5 / (c->sigma * c->sigma);
+            for (int k = 1; k < std::min(c->n, 12); k++) {
+                rb[c->n + k] = 0.5 * exp(-alpha * c->rb[k] * c->rb[k]);
+                rb[c->n + 12 + k] = 1.0 / k;
+            }
+            CHK(upload(c->d_rb, rb.data(), rb.size() * 8));
             CHK(upload(c->d_T, c->T.data(), c->T.size() * 8));
             CHK(upload(c->d_qmap, c->qmap.data(), c->qmap.size() * 4));
             const size_t need = soap_lds_bytes(soap_dev(*c));
@@ -1262,6 +1269,9 @@ static SoapDev soap_dev(const Coord &c) {
     sp.rc = c.rc; sp.ctw = c.ctw; sp.alpha = 0.5 / (c.sigma * c.sigma); sp.cw = c.cw; sp.u00 = c.u00;
     sp.n = c.n; sp.S = c.S; sp.K = c.S * c.n; sp.L = c.L; sp.LM = (c.L + 1) * (c.L + 1); sp.dim = c.dim;
     for (int s = 0; s < kMaxSpecies; s++) sp.species_Z[s] = s < c.S ? c.species[s] : -1;
+    sp.dr = c.n > 1 ? c.rb[1] : 0.0;
+    sp.a2dr = 2.0 * sp.alpha * sp.dr; sp.ia2dr = 1.0 / sp.a2dr; sp.ictw = 1.0 / sp.ctw;
+    sp.rt = c.d_rb.as<double>() + c.n;
     sp.rb = c.d_rb.as<double>(); sp.T = c.d_T.as<double>(); sp.qmap = c.d_qmap.as<int>();
     return sp;
 }
@@ -1852,6 +1862,19 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
             const size_t zn[3] = {(size_t)P * 3, (size_t)N, (size_t)P};
             launch_zero_f64_multi(has_d2b_var ? 3 : 2, zp, zn, s);
         }
+        // whether an earlier coordinate writes forces on coordinate k's pairs too: a pair
+        // descriptor, or one with a centre species in common (0 is every species).  Otherwise the
+        // adjoint stores its forces without reading the cleared ones (batch512: 100 MB less).
+        auto shared_pairs = [&](size_t k) {
+            for (size_t j = 0; j < k; j++) {
+                if (skipped(j)) continue;
+                if (m->coords[j]->kind != 1) return true;
+                for (int za : m->coords[j]->centreZ)
+                    for (int zb : m->coords[k]->centreZ)
+                        if (za == zb || za == 0 || zb == 0) return true;
+            }
+            return false;
+        };
         for (size_t k = 0; k < NCOORD; k++) {
             Coord &c = *m->coords[k];
             if (skipped(k)) continue;
@@ -1883,7 +1906,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
             SoapDev sp = soap_dev(c);
             const int t0 = marks ? tm.mark(s) : -1;
             launch_soap_fwd(sp, nc, centres, w.Z.as<int>(), w.nb_off.as<int>(), w.nb_j.as<int>(), w.nb_r.as<double>(),
-                            w.nb_d.as<double>(), w.X.as<double>(), w.norm.as<double>(), w.cbuf.as<double>(), s);
+                            w.nb_d.as<double>(), w.X.as<double>(), w.norm.as<double>(), w.cbuf.as<double>(), want_var, s);
             const int t1 = marks ? tm.mark(s) : -1;
             int ntile = 0;
             const bool f64fused = m->precision == GAPX_PREC_FP64 && grad && tu.f64parts > 0;
@@ -1935,7 +1958,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
                     launch_var_self_grad(nc, c.dim, w.X.as<double>(), d2, c.zeta, w.Gv.as<double>(), s);
                     launch_soap_bwd(sp, nc, centres, w.Z.as<int>(), w.nb_off.as<int>(), w.nb_j.as<int>(),
                                     w.nb_r.as<double>(), w.nb_d.as<double>(), w.X.as<double>(), w.Gv.as<double>(),
-                                    w.norm.as<double>(), w.cbuf.as<double>(), w.pairFv.as<double>(), s);
+                                    w.norm.as<double>(), w.cbuf.as<double>(), w.pairFv.as<double>(), shared_pairs(k), s);
                 }
             }
             if (grad) {
@@ -1954,7 +1977,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
                 const int t3 = marks ? tm.mark(s) : -1;
                 launch_soap_bwd(sp, nc, centres, w.Z.as<int>(), w.nb_off.as<int>(), w.nb_j.as<int>(),
                                 w.nb_r.as<double>(), w.nb_d.as<double>(), w.X.as<double>(), w.G.as<double>(),
-                                w.norm.as<double>(), w.cbuf.as<double>(), w.pairF.as<double>(), s);
+                                w.norm.as<double>(), w.cbuf.as<double>(), w.pairF.as<double>(), shared_pairs(k), s);
                 if (marks) { tm.stage(3, t2, t3); tm.stage(4, t3, tm.mark(s)); }
             }
         }
@@ -2481,7 +2504,7 @@ extern "C" int gapx_descriptors(gapx_model *m, int coord, int N, const double *p
     CHK(w.cbuf.ensure((size_t)nc * KLM * 8));
     launch_soap_fwd(soap_dev(c), nc, w.centres[coord].as<int>(), w.Z.as<int>(), w.nb_off.as<int>(),
                     w.nb_j.as<int>(), w.nb_r.as<double>(), w.nb_d.as<double>(), w.X.as<double>(), w.norm.as<double>(),
-                    w.cbuf.as<double>(), s);
+                    w.cbuf.as<double>(), false, s);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(X, w.X.p, (size_t)nc * c.dim * 8, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));

@@ -24,7 +24,9 @@ struct SoapDev {
     double rc, ctw, alpha, cw, u00;
     int n, S, K, LM, dim, L;
     int species_Z[kMaxSpecies];
-    const double *rb;    // n grid points
+    const double *rb;    // n grid points r_a = a dr
+    const double *rt;    // exp(-alpha r_a^2) / 2 and 1/a of a < 12 (zero for a = 0 and a >= n): 2 x 12
+    double dr, a2dr, ia2dr, ictw;   // grid spacing, 2 alpha dr, its inverse, 1 / ctw
     const double *T;     // n x n transform, T[a*n+b]
     const int *qmap;     // dim-1 entries: (ia<<16)|(jb<<8)|l
 };
@@ -103,6 +105,8 @@ void launch_zero_step(double *pairF, double *pairE, double *esite, int N, const 
 // device; done at model load so that no launch sequence contains an upload)
 hipError_t soap_constants_init();
 hipError_t soap_fast_constants_init();
+hipError_t soap_lane_constants_init();
+void soap_coefficient_order(int l, int m, int *place, double *factor);
 int soap_supported(int n, int L);
 int soap_fast_supported(int n, int L);
 // LDS bytes per block the descriptor kernels of this shape use (largest launch variant)
@@ -111,15 +115,21 @@ size_t soap_fast_lds_bytes(const SoapDev &sp);
 bool launch_soap_fwd_fast(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
                           const int *nb_j, const double *nb_r, const double *nb_d, double *X, double *norm,
                           double *cbuf, hipStream_t s);
+// the adjoint: add = false stores the pair forces (pairF is zero or another centre's rows), true adds to them
 bool launch_soap_bwd_fast(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
                           const int *nb_j, const double *nb_r, const double *nb_d, const double *X, const double *G,
-                          const double *norm, const double *cbuf, double *pairF, hipStream_t s);
+                          const double *norm, const double *cbuf, double *pairF, bool add, hipStream_t s);
+bool launch_soap_fwd_lane(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
+                          const int *nb_j, const double *nb_r, const double *nb_d, double *X, double *norm,
+                          double *cbuf, hipStream_t s);
+size_t soap_lane_lds_bytes(const SoapDev &sp);
+// for_variance: the forward whose summation order the GAP variance's digits belong to
 void launch_soap_fwd(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
                      const int *nb_j, const double *nb_r, const double *nb_d, double *X, double *norm,
-                     double *cbuf, hipStream_t s);
+                     double *cbuf, bool for_variance, hipStream_t s);
 void launch_soap_bwd(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
                      const int *nb_j, const double *nb_r, const double *nb_d, const double *X, const double *G,
-                     const double *norm, const double *cbuf, double *pairF, hipStream_t s);
+                     const double *norm, const double *cbuf, double *pairF, bool add, hipStream_t s);
 
 // GEMMs
 // Tile configuration `cfg` in [0, kGemmTiles): (WM, WN, k tile) = (4,2,16), (2,2,16),

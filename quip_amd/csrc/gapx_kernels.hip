@@ -53,7 +53,8 @@ static hipError_t ensure_constants() {
 
 hipError_t soap_constants_init() {
     hipError_t e = ensure_constants();
-    return e != hipSuccess ? e : soap_fast_constants_init();
+    if (e == hipSuccess) e = soap_fast_constants_init();
+    return e != hipSuccess ? e : soap_lane_constants_init();
 }
 
 static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
@@ -1524,7 +1525,8 @@ size_t soap_lds_bytes(const SoapDev &sp) {
 
 void launch_soap_fwd(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
                      const int *nb_j, const double *nb_r, const double *nb_d, double *X, double *norm,
-                     double *cbuf, hipStream_t s) {
+                     double *cbuf, bool for_variance, hipStream_t s) {
+    if (for_variance && launch_soap_fwd_lane(sp, nc, centres, Z, nb_off, nb_j, nb_r, nb_d, X, norm, cbuf, s)) return;
     if (launch_soap_fwd_fast(sp, nc, centres, Z, nb_off, nb_j, nb_r, nb_d, X, norm, cbuf, s)) return;
     ensure_constants();
     if (nc <= 0) return;
@@ -1546,8 +1548,8 @@ void launch_soap_fwd(const SoapDev &sp, int nc, const int *centres, const int *Z
 
 void launch_soap_bwd(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
                      const int *nb_j, const double *nb_r, const double *nb_d, const double *X, const double *G,
-                     const double *norm, const double *cbuf, double *pairF, hipStream_t s) {
-    if (launch_soap_bwd_fast(sp, nc, centres, Z, nb_off, nb_j, nb_r, nb_d, X, G, norm, cbuf, pairF, s)) return;
+                     const double *norm, const double *cbuf, double *pairF, bool add, hipStream_t s) {
+    if (launch_soap_bwd_fast(sp, nc, centres, Z, nb_off, nb_j, nb_r, nb_d, X, G, norm, cbuf, pairF, add, s)) return;
     ensure_constants();
     if (nc <= 0) return;
     size_t sh = bwd_generic_lds(sp);

@@ -1,32 +1,45 @@
-// SOAP descriptor kernels specialised on (n_max, l_max).
+// SOAP descriptor kernels specialised on (n_max, l_max), on the FP64 matrix cores.
 //
-// One wavefront per centre atom.  The radial transform T (n x n) and the
-// radial grid live in LDS; an empty asm with a memory clobber closes every
-// l step so the compiler re-reads T from LDS instead of pinning n^2 doubles in
-// VGPRs.  All loops over b, a, l and m are unrolled at compile time, so the
-// per-lane recursion state (radial: F_l, F_(l+1), 1/x per grid point;
-// Legendre: two previous levels) stays in registers with no scratch.
+// Every contraction of the descriptor is a batch of small products: the density
+// coefficients c'_l = sum_k F_l(a, k) Y_lm(k) over the neighbours k, the radial
+// transform T, the power spectrum c_l c_l^T, and in the adjoint dE/dc_l = P_l c_l and the
+// products of dE/dc' with the neighbours' radial functions.  They run on
+// v_mfma_f64_4x4x4: four independent 4x4 blocks of a k of 4, at the same rate per
+// operation as 16x16x4 (measured 16 and 64 cycles), so levels of 1 to 17 harmonics waste
+// little.  The recursions and the products' operands meet in registers: the lane that
+// holds an operand element computes it, so neighbour data never pass through LDS except
+// for a small table of per-neighbour scalars.
 //
-//  forward: per l, lanes = neighbours stage fc F_l(a) and Y_l,m in LDS, lanes
-//           = (a, m) accumulate c' in the primitive radial basis; c = T^T c'
-//           once per centre; lanes = power-spectrum entries form p, a wave
-//           reduction gives |p|.
-//  adjoint: dE/dp -> dE/dc per level as a small product staged in LDS ->
-//           dE/dc' = T dE/dc, then lanes = neighbours re-evaluate F_l, Y and
-//           grad Y and contract them with dE/dc'.
+// Lane roles of the 4x4x4 product (lane = 16 k + 4 b + i): A holds row i, inner index k
+// of block b; B holds inner index k, column i of block b; D holds row k, column i of block b.
+//
+// Harmonics of a level come in groups of four: group v = 0 holds cos(m phi) terms of
+// m = 0..3, v = 1 sin terms of m = 0..3 (m = 0 is empty), v = 2, 3 the same for m = 4..7 and
+// v = 4, 5 for m = 8 (empty beyond it).  Empty slots meet zeros.
 #include "gapx_kernels.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace gapx {
 
 #define GAPX_PI_S 3.14159265358979323846264338327950288
 
-// N_lm of the real spherical harmonics (x sqrt 2 for m > 0) and (2m-1)!!
-static __constant__ double c_ynorm[(kMaxL + 1) * (kMaxL + 2) / 2];
-static __constant__ double c_dfact[kMaxL + 2];
-static __constant__ double c_rinv[2 * kMaxL + 4];   // 1/k (k = 0 unused)
-static __constant__ double c_isq[kMaxL + 1];        // 1/sqrt(2l+1)
+__host__ __device__ constexpr int lev_groups(int l) { return l == 0 ? 1 : l < 4 ? 2 : l < 8 ? 4 : 6; }
+__host__ __device__ constexpr int lev_base(int l) { return l == 0 ? 0 : l <= 4 ? 2 * l - 1 : l <= 8 ? 4 * l - 9 : 29; }
+__host__ __device__ constexpr int soap_groups(int L) { return lev_base(L) + lev_groups(L); }
+
+constexpr int kSoapMaxL = 8;                             // of the specialised shapes
+constexpr int kSoapGroups = soap_groups(kSoapMaxL);      // 29
+
+// per group: its level; per (group, slot): the place of the harmonic within the (L+1)^2
+// coefficients of a radial row (-1: empty) and the factor between the monic Legendre
+// recursion used here and the real harmonic
+static __constant__ int c_glev[kSoapGroups + 3];
+static __constant__ int c_gpos[4 * kSoapGroups + 12];
+static __constant__ double c_gnorm[4 * kSoapGroups + 12];
+static __constant__ double c_ginv[4 * kSoapGroups + 12];   // 1 / c_gnorm (0: empty)
+static __constant__ double c_isq[kSoapMaxL + 1];         // 1/sqrt(2l+1)
 
 static bool g_soap_const_ready[64] = {};   // per device
 static hipError_t ensure_soap_constants() {
@@ -35,630 +48,937 @@ static hipError_t ensure_soap_constants() {
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
     if (g_soap_const_ready[dev]) return hipSuccess;
-    double yn[(kMaxL + 1) * (kMaxL + 2) / 2], df[kMaxL + 2];
-    for (int l = 0; l <= kMaxL; l++)
-        for (int m = 0; m <= l; m++) {
-            double r = 1.0;   // (l-m)!/(l+m)!
-            for (int k = l - m + 1; k <= l + m; k++) r /= (double)k;
-            double v = sqrt((2.0 * l + 1.0) / (4.0 * GAPX_PI_S) * r);
-            if (m > 0) v *= sqrt(2.0);
-            yn[l * (l + 1) / 2 + m] = v;
+    int lev[kSoapGroups + 3] = {}, pos[4 * kSoapGroups + 12];
+    double nrm[4 * kSoapGroups + 12] = {}, inv[4 * kSoapGroups + 12] = {}, isq[kSoapMaxL + 1];
+    std::fill(pos, pos + 4 * kSoapGroups + 12, -1);
+    for (int l = 0; l <= kSoapMaxL; l++) {
+        isq[l] = 1.0 / sqrt(2.0 * l + 1.0);
+        for (int v = 0; v < lev_groups(l); v++) {
+            const int g = lev_base(l) + v;
+            lev[g] = l;
+            for (int j = 0; j < 4; j++) {
+                const int m = 4 * (v / 2) + j;
+                if (m > l || (m == 0 && (v & 1))) continue;
+                soap_coefficient_order(l, v & 1 ? -m : m, pos + 4 * g + j, nrm + 4 * g + j);
+                inv[4 * g + j] = 1.0 / nrm[4 * g + j];
+            }
         }
-    df[0] = 1.0;
-    for (int m = 1; m < kMaxL + 2; m++) df[m] = df[m - 1] * (2.0 * m - 1.0);
-    double ri[2 * kMaxL + 4];
-    ri[0] = 0.0;
-    for (int k = 1; k < 2 * kMaxL + 4; k++) ri[k] = 1.0 / (double)k;
-    double isq[kMaxL + 1];
-    for (int l = 0; l <= kMaxL; l++) isq[l] = 1.0 / sqrt(2.0 * l + 1.0);
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_rinv), ri, sizeof(ri))) != hipSuccess) return e;
+    }
+    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_glev), lev, sizeof(lev))) != hipSuccess) return e;
+    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_gpos), pos, sizeof(pos))) != hipSuccess) return e;
+    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_gnorm), nrm, sizeof(nrm))) != hipSuccess) return e;
+    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_ginv), inv, sizeof(inv))) != hipSuccess) return e;
     if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_isq), isq, sizeof(isq))) != hipSuccess) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_ynorm), yn, sizeof(yn))) != hipSuccess) return e;
-    if ((e = hipMemcpyToSymbol(HIP_SYMBOL(c_dfact), df, sizeof(df))) != hipSuccess) return e;
     g_soap_const_ready[dev] = true;
     return hipSuccess;
 }
 
 hipError_t soap_fast_constants_init() { return ensure_soap_constants(); }
 
-#define RELOAD_BARRIER() __asm__ volatile("" ::: "memory")
-
-// neighbours staged per pass of the forward kernel (one lane each)
-constexpr int kSoapChunk = 32;
-
-__device__ __forceinline__ double fc_s(double r, double rc, double w) {
-    if (r > rc) return 0.0;
-    if (r > rc - w) return 0.5 * (cos(GAPX_PI_S * (r - rc + w) / w) + 1.0);
-    return 1.0;
+// The real harmonic (l, m) (m < 0: sin) in a radial row of the coefficient buffer: its place
+// and the factor it is stored with.
+void soap_coefficient_order(int l, int m, int *place, double *factor) {
+    const int a = m < 0 ? -m : m, v = 2 * (a / 4) + (m < 0);
+    int next = l * l;   // of group v's first slot
+    for (int u = 0; u < v; u++) next += std::min(l + 1 - 4 * (u / 2), 4) - (u == 1);
+    *place = next + a % 4 - (v == 1);
+    double r = 1.0, lead = 1.0;   // (l-a)!/(l+a)!; the a-th derivative of P_l over its monic form
+    for (int k = l - a + 1; k <= l + a; k++) r /= (double)k;
+    for (int k = 1; k <= l; k++) lead *= 2.0 * k - 1.0;
+    for (int k = 2; k <= l - a; k++) lead /= (double)k;
+    *factor = sqrt((2.0 * l + 1.0) / (4.0 * GAPX_PI_S) * r) * (a > 0 ? sqrt(2.0) : 1.0) * lead;
 }
-// fc and dfc/dr together: one sincos for the transition region
-__device__ __forceinline__ void fc_dfc_s(double r, double rc, double w, double &fc, double &dfc) {
-    fc = 0.0;
-    dfc = 0.0;
-    if (r > rc) return;
-    if (r > rc - w) {
-        double sn, cs;
-        sincos(GAPX_PI_S * (r - rc + w) / w, &sn, &cs);
-        fc = 0.5 * (cs + 1.0);
-        dfc = -0.5 * GAPX_PI_S * sn / w;
-        return;
-    }
-    fc = 1.0;
+
+__device__ __forceinline__ double mfma4(double a, double b, double c) {
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+// orders this wavefront's LDS writes before its reads of other lanes' data
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// orders the block's LDS accesses: a barrier that waits for LDS only (memory accesses stay
+// in flight), or within a lone wavefront the fence only
+template <int NW>
+__device__ __forceinline__ void block_lds_sync() {
+    if constexpr (NW > 1) __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else wave_lds_sync();
+}
+// the lane number anew: what follows from it is recomputed here instead of being kept in
+// registers across a loop over centres
+__device__ __forceinline__ int fresh_lane() {
+    int l = threadIdx.x & 63;
+    __asm__ volatile("" : "+v"(l));
+    return l;
 }
 __device__ __forceinline__ double wave_sum_s(double v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
 }
-__device__ __forceinline__ int species_s(const SoapDev &sp, int z) {
-    for (int s = 0; s < sp.S; s++)
+__device__ __forceinline__ int species_s(const SoapDev &sp, int S, int z) {
+    for (int s = 0; s < S; s++)
         if (sp.species_Z[s] == z || sp.species_Z[s] == 0) return s;
     return -1;
 }
 
-// Associated Legendre values P_l^m (m = 0..l) of one neighbour, level by level,
-// in two LDS rows: on entry cur holds P_(l-2), prev P_(l-1); on exit cur holds P_l.
-__device__ __forceinline__ void legendre_level(int l, double uz, const double *prev, double *cur) {
-    for (int m = 0; m <= l; m++) {
-        double pc;
-        if (m == l) pc = c_dfact[m];
-        else if (m == l - 1) pc = (2.0 * l - 1.0) * uz * prev[m];
-        else pc = ((2.0 * l - 1.0) * uz * prev[m] - (double)(l + m - 1) * cur[m]) * c_rinv[l - m];
-        cur[m] = pc;
+// The neighbour table in LDS: one row per field, one slot per neighbour.  A pass covers
+// kSoapPass neighbours (one per lane); the slots of each species start at a multiple of
+// 16, the neighbours of one tile.
+constexpr int kSoapPass = 64;
+enum { kUx, kUy, kUz, kIxq, kE0, kQ, kQi, kFwdFields, kFc = kFwdFields, kDfc, kIr, kR, kBwdFields };
+
+// A wavefront's neighbours of one pass, one per lane, on their way from memory.
+struct SoapNb {
+    int j, z;
+    double r, dx, dy, dz;
+    __device__ __forceinline__ void load(int p0, int nk, const int *__restrict__ nb_j, const double *__restrict__ nb_r,
+                                         const double *__restrict__ nb_d) {
+        const int lane = threadIdx.x & 63;
+        if (lane < nk) {
+            const int p = p0 + lane;
+            j = nb_j[p];
+            r = nb_r[p];
+            dx = nb_d[3 * p]; dy = nb_d[3 * p + 1]; dz = nb_d[3 * p + 2];
+        }
+    }
+    __device__ __forceinline__ void species(int nk, const int *__restrict__ Z) {
+        if ((int)(threadIdx.x & 63) < nk) z = Z[j];
+    }
+};
+
+// One wavefront writes the table of nk <= 64 neighbours from pair p0 on, the first slot
+// (sb) and the number (sc) of each species' slots, and (adjoint) the pair of each slot.
+// Radial functions of grid point r_a = a dr: exp(-alpha (r -+ r_a)^2) = e0 gA[a] q^(+-a)
+// with e0 = exp(-alpha r^2), gA = exp(-alpha r_a^2), q = exp(2 alpha r dr).  Outside the range
+// where these stay finite q = 0 marks the slot and its exponentials are formed directly (r in the
+// place of 1/q).  The forward's e0 carries the cutoff function.
+template <int N, bool BWD>
+__device__ __forceinline__ void soap_stage(const SoapDev &sp, int S, const SoapNb &nb, int p0, int nk, double *tab,
+                                           int slots, int *sb, int *sc, int *pair) {
+    const int lane = threadIdx.x & 63;
+    const double r = nb.r;
+    int s = -1;
+    if (lane < nk && !(r > sp.rc)) s = species_s(sp, S, nb.z);
+    int slot = 0, base = 0;
+    for (int si = 0; si < S; si++) {
+        const unsigned long long mk = __ballot(s == si);
+        const int n = __popcll(mk);
+        if (s == si) slot = base + __popcll(mk & ((1ull << lane) - 1ull));
+        if (lane == 0) { sb[si] = base; sc[si] = n; }
+        base += (n + 15) & ~15;
+    }
+    if (s < 0) return;
+    double fc = 1.0, dfc = 0.0;
+    if (r > sp.rc - sp.ctw) {
+        double sn, cs;
+        sincospi((r - sp.rc + sp.ctw) * sp.ictw, &sn, &cs);
+        fc = 0.5 * (cs + 1.0);
+        dfc = -0.5 * GAPX_PI_S * sp.ictw * sn;
+    }
+    const double ir = 1.0 / r, xq = sp.a2dr * r, rmax = (N - 1) * sp.dr;
+    double e0 = 1.0, q = 0.0, qi = r;
+    if (xq > 0.0 && xq * (4 * ((N + 3) / 4) - 1) < 600.0 && sp.alpha * (r * r + rmax * rmax) < 600.0) {
+        e0 = exp(-sp.alpha * r * r);
+        q = exp(xq);
+        qi = 1.0 / q;
+    }
+    if (!BWD) e0 *= fc;
+    tab[kUx * slots + slot] = nb.dx * ir;
+    tab[kUy * slots + slot] = nb.dy * ir;
+    tab[kUz * slots + slot] = nb.dz * ir;
+    tab[kIxq * slots + slot] = ir * sp.ia2dr;
+    tab[kE0 * slots + slot] = e0;
+    tab[kQ * slots + slot] = q;
+    tab[kQi * slots + slot] = qi;
+    if constexpr (BWD) {
+        tab[kFc * slots + slot] = fc;
+        tab[kDfc * slots + slot] = dfc;
+        tab[kIr * slots + slot] = ir;
+        tab[kR * slots + slot] = r;
+        pair[slot] = p0 + lane;
     }
 }
 
-// i_l recursion state for all grid points: F0 = f_l, F1 = f_(l+1).  The
-// recursion factor 1/x_a = 1/(2 alpha r r_a) is ixq / a with ixq = 1/(2 alpha r dr)
-// (r_a = a dr), formed from ixq when used (no per-point array: fewer registers).
-// rbs: grid r_a = a * dr; gA[a] = exp(-alpha r_a^2); iA[a] = 1/a.
-// exp(-alpha (r -+ r_a)^2) = exp(-alpha r^2) gA[a] q^(+-a) with q = exp(2 alpha r dr):
-// two exponentials and one division per neighbour.  Outside the range where the
-// powers stay finite, every point is direct.
+// The constant tables of a block in LDS (a table in memory would queue behind the neighbour
+// data on their way): the transform, the radial tables, per (group, slot) the harmonics' factor
+// and the place and level of the harmonic, per level 1/sqrt(2l+1).
+template <int N, int L>
+struct SoapTables {
+    static constexpr int NA = (N + 3) / 4, NQ4 = (soap_groups(L) + 3) / 4 * 4;
+    double *T, *rt, *gn, *isq;
+    int *pos;   // place (0xffff: an empty slot) | level << 16
+    __device__ __forceinline__ SoapTables(double *p) : T(p), rt(T + N * N), gn(rt + 24), isq(gn + 4 * NQ4), pos((int *)(isq + L + 1)) {}
+    __device__ __forceinline__ void fill(const SoapDev &sp, int nthr) {
+        for (int e = threadIdx.x; e < N * N; e += nthr) T[e] = sp.T[e];
+        for (int e = threadIdx.x; e < 24; e += nthr) rt[e] = sp.rt[e];
+        for (int e = threadIdx.x; e < L + 1; e += nthr) isq[e] = c_isq[e];
+        for (int e = threadIdx.x; e < 4 * NQ4; e += nthr) {
+            const bool in = e < 4 * soap_groups(L);
+            gn[e] = in ? c_gnorm[e] : 0.0;
+            pos[e] = in ? (c_gpos[e] & 0xffff) | c_glev[e / 4] << 16 : 0xffff;
+        }
+    }
+    // T[a][b], zero beyond the basis
+    __device__ __forceinline__ double t(int a, int b) const {
+        return N % 4 == 0 || (a < N && b < N) ? T[min(a, N - 1) * N + min(b, N - 1)] : 0.0;
+    }
+};
+
+// recursion coefficient of the monic m-th derivatives of P_l: p_l = z p_(l-1) - beta p_(l-2),
+// beta = ((l-1)^2 - m^2) / ((2l-1)(2l-3)); zero states below l = m keep p_(m+1) = z p_m
+__device__ __forceinline__ double leg_beta(int l, double m2) {
+    const double rl = 1.0 / ((2.0 * l - 1.0) * (2.0 * l - 3.0));
+    return fma(-m2, rl, (l - 1.0) * (l - 1.0) * rl);
+}
+
+// One lane's share of a neighbour: the radial functions of grid points a = g + 4u and the
+// harmonics of m = g and g + 4 (and m = 8 in lane group 0).
 template <int N>
-struct Rad {
-    double F0[N], F1[N], ixq;
-    __device__ __forceinline__ void init(const double *rbs, const double *gA, const double *iA, double alpha,
-                                         double r) {
-        const double xq = N > 1 ? 2.0 * alpha * r * rbs[1] : 0.0;
-        const double rmax = rbs[N - 1];
-        ixq = 1.0 / xq;
-        if (xq > 0.0 && xq * (N - 1) < 600.0 && alpha * (r * r + rmax * rmax) < 600.0) {
-            const double e0 = exp(-alpha * r * r);
-            const double q = exp(xq), qi = 1.0 / q;
-            double qa = 1.0, qia = 1.0;
-            F0[0] = e0;
-            F1[0] = 0.0;
+struct SoapLane {
+    static constexpr int NA = (N + 3) / 4;
+    // per lane group: exp(-alpha r_a^2) / 2 and 1/a (0 for a = 0 and a >= N)
+    double hg[NA], ia[NA];
+    // recursion state F_l, F_(l+1), 1/x_a; the a = 0 value of l = 0
+    double F0[NA], F1[NA], iv[NA], z0;
+    double z, mA2, mB2, pA, pA1, pB, pB1;   // monic Legendre values of levels l, l - 1
+    double start[4];                        // 1 in the group whose m starts at this level
+
+    __device__ __forceinline__ void setup(const double *rt, int g) {
 #pragma unroll
-            for (int a = 1; a < N; a++) {
-                qa *= q;
-                qia *= qi;
-                const double eg = e0 * gA[a];
-                const double em = eg * qa, ep = eg * qia;
-                const double iv = ixq * iA[a];
-                F0[a] = 0.5 * (em - ep) * iv;
-                F1[a] = 0.5 * (em + ep) * iv - F0[a] * iv;
+        for (int u = 0; u < NA; u++) {
+            hg[u] = rt[g + 4 * u];
+            ia[u] = rt[12 + g + 4 * u];
+        }
+        mA2 = (double)(g * g);
+        mB2 = (double)((g + 4) * (g + 4));
+#pragma unroll
+        for (int l = 0; l < 4; l++) start[l] = g == l ? 1.0 : 0.0;
+    }
+    // monic m-th derivative of P_l, m = g + m0 (zero below l = m), from the states of l-1 and l-2
+    __device__ __forceinline__ double legendre(int l, int m0, double m2, double p1, double p2) const {
+        const int k = l - m0;
+        if (k == 0) return start[0];
+        const double t = k < 4 ? fma(z, p1, start[k < 4 ? k : 0]) : z * p1;
+        return k == 1 ? t : t - leg_beta(l, m2) * p2;
+    }
+    // i_l recursion from i_(-1) = cosh(x)/x, i_0 = sinh(x)/x, x_a = 2 alpha r r_a; ixq = 1/x_1
+    __device__ __forceinline__ void radial(const SoapDev &sp, int g, double ixq, double e0, double q,
+                                           double qi) {
+        const double q2 = q * q, i2 = qi * qi;
+        double ep = g == 0 ? 1.0 : g == 1 ? q : g == 2 ? q2 : q2 * q;
+        double em = g == 0 ? 1.0 : g == 1 ? qi : g == 2 ? i2 : i2 * qi;
+        const double q4 = q2 * q2, i4 = i2 * i2;
+        const bool direct = q == 0.0;
+        z0 = g == 0 ? e0 : 0.0;
+        if (__any(direct)) {
+            const double r = qi;
+            if (direct && g == 0) z0 = e0 * exp(-sp.alpha * r * r);
+#pragma unroll
+            for (int u = 0; u < NA; u++) {
+                const int a = g + 4 * u;
+                const double ra = a * sp.dr;
+                iv[u] = ixq * ia[u];
+                double m_ = e0 * hg[u] * ep, p_ = e0 * hg[u] * em;
+                if (direct) {
+                    m_ = a < N ? 0.5 * e0 * exp(-sp.alpha * (r - ra) * (r - ra)) : 0.0;
+                    p_ = a < N ? 0.5 * e0 * exp(-sp.alpha * (r + ra) * (r + ra)) : 0.0;
+                    if (a == 0 || a >= N) iv[u] = 0.0;
+                }
+                F0[u] = (m_ - p_) * iv[u];
+                F1[u] = (m_ + p_) * iv[u] - F0[u] * iv[u];
+                ep *= q4;
+                em *= i4;
             }
             return;
         }
 #pragma unroll
-        for (int a = 0; a < N; a++) {
-            const double ra = rbs[a];
-            if (a == 0) {
-                F0[a] = exp(-alpha * (ra * ra + r * r));
-                F1[a] = 0.0;
-            } else {
-                const double ep = exp(-alpha * (r + ra) * (r + ra)), em = exp(-alpha * (r - ra) * (r - ra));
-                const double iv = ixq * (1.0 / (double)a);
-                F0[a] = 0.5 * (em - ep) * iv;
-                F1[a] = 0.5 * (em + ep) * iv - F0[a] * iv;
+        for (int u = 0; u < NA; u++) {
+            iv[u] = ixq * ia[u];
+            const double eg = e0 * hg[u];
+            const double m_ = eg * ep, p_ = eg * em;
+            F0[u] = (m_ - p_) * iv[u];
+            F1[u] = (m_ + p_) * iv[u] - F0[u] * iv[u];
+            if (u + 1 < NA) {
+                ep *= q4;
+                em *= i4;
             }
-            __builtin_amdgcn_sched_barrier(0);   // one grid point's exponentials at a time
         }
     }
-    // Scaled form (the adjoint): F1 holds a f_(l+1)(a), so that the sum over grid points
-    // of r_a f_(l+1)(a) v_a is dr times the sum of F1[a] v_a, with no product by r_a.
-    // Starting from the state init leaves, step_scaled keeps this form:
-    // a f_(l+2) = a f_l - (2l+3) ixq f_(l+1) and f_(l+1) = F1[a] / a.
-    __device__ __forceinline__ void scale_f1() {
-#pragma unroll
-        for (int a = 0; a < N; a++) F1[a] *= (double)a;
-    }
-    __device__ __forceinline__ void step_scaled(int l) {
-        const double c = (2.0 * l + 3.0) * ixq;
-        F0[0] = 0.0;   // grid point 0 (r_a = 0): f_(l+1) = 0 for every l
-#pragma unroll
-        for (int a = 1; a < N; a++) {
-            const double t = F1[a] * (1.0 / (double)a);
-            F1[a] = (double)a * F0[a] - c * t;
-            F0[a] = t;
-        }
-    }
+    __device__ __forceinline__ double f(int l, int u) const { return l == 0 && u == 0 ? F0[0] + z0 : F0[u]; }
     __device__ __forceinline__ void step(int l) {
-        F0[0] = F1[0];   // grid point 0 (r_a = 0): f_(l+1) = 0 for every l
-        F1[0] = 0.0;
 #pragma unroll
-        for (int a = 1; a < N; a++) {
-            const double n2 = F0[a] - (2.0 * l + 3.0) * (ixq * (1.0 / (double)a)) * F1[a];
-            F0[a] = F1[a];
-            F1[a] = n2;
+        for (int u = 0; u < NA; u++) {
+            const double n2 = F0[u] - ((2.0 * l + 3.0) * iv[u]) * F1[u];
+            F0[u] = F1[u];
+            F1[u] = n2;
         }
     }
 };
 
-// Forward.  With g_b(r) = fc(r) sum_a F_l(a, r) T[a][b] (F = the i_l recursion
-// values of grid point a), c[b][lm] = sum_a T[a][b] c'[a][lm] where
-// c'[a][lm] = sum_k fc F_l(a, r_k) Y_lm(k) is accumulated in the primitive
-// (Gaussian) radial basis and transformed once per centre.
-// Per neighbour chunk: the chunk's neighbours are listed per species (wave
-// ballot); per l, lanes = neighbours stage fc F_l(a) and Y_l,m in LDS and
-// lanes = (a, m) accumulate c' of each species over that species' list only.
-// One level of a chunk: stage fc F_l and Y_l of the neighbours, then accumulate
-// c' of level l.  A macro so that both level loops (rolled and unrolled) inline it.
-#define SOAP_FWD_LEVEL(l, cur, prv)                                                                                  \
-            __syncthreads();   /* the previous level's reads of Rl / Yl are done */                                  \
-            if (lane < 32 * CPW) {   /* rows of neighbours outside every list stay zero for the dense loop */        \
-_Pragma("unroll")                                                                                                    \
-                for (int a = 0; a < N; a++) Rh[a * RT + kl] = s >= 0 ? fc * rs.F0[a] : 0.0;                          \
-            }                                                                                                        \
-            if (s >= 0) {                                                                                            \
-                rs.step(l);                                                                                          \
-                legendre_level(l, uz, prv, cur);                                                                     \
-                double A = 1.0, B = 0.0;                                                                             \
-                double *Yr = Yh + kl;   /* slot m of this neighbour at Yr[m * RT] */                                 \
-                for (int m = 0; m <= l; m++) {                                                                       \
-                    if (m > 0) {                                                                                     \
-                        const double An = A * ux - B * uy;                                                           \
-                        B = A * uy + B * ux;                                                                         \
-                        A = An;                                                                                      \
-                    }                                                                                                \
-                    const double Nn = c_ynorm[l * (l + 1) / 2 + m] * cur[m];                                         \
-                    if (m == 0) Yr[l * RT] = Nn;                                                                     \
-                    else {                                                                                           \
-                        Yr[(l + m) * RT] = Nn * A;                                                                   \
-                        Yr[(l - m) * RT] = Nn * B;                                                                   \
-                    }                                                                                                \
-                }                                                                                                    \
-            } else if (lane < 32 * CPW) {                                                                            \
-                for (int m = 0; m < 2 * l + 1; m++) Yh[m * RT + kl] = 0.0;                                           \
-            }                                                                                                        \
-            __syncthreads();                                                                                         \
-            const int W = 2 * l + 1;                                                                                 \
-            for (int it = lane; it < CPW * N * W; it += 64) {                                                        \
-                const int hh = CPW == 1 ? 0 : it / (N * W), r_ = it - hh * (N * W);                                 \
-                const int a = r_ / W, mi = r_ - a * W;                                                               \
-                const double *Rc = Rl + hh * (N * RT), *Yc = Yl + hh * (YW * RT);                                   \
-                double *cPc = cP + hh * KLMp;                                                                        \
-                if (S == 1) {   /* one species: every row of the chunk in pairs, zero rows included */            \
-                    const double2 *R2 = (const double2 *)(Rc + a * RT), *Y2 = (const double2 *)(Yc + mi * RT);      \
-                    double acc0 = 0.0, acc1 = 0.0;                                                                   \
-_Pragma("unroll 4")                                                                                                  \
-                    for (int k2 = 0; k2 < NB / 2; k2++) {                                                            \
-                        const double2 rv = R2[k2], yv = Y2[k2];                                                      \
-                        acc0 += rv.x * yv.x;                                                                         \
-                        acc1 += rv.y * yv.y;                                                                         \
-                    }                                                                                                \
-                    cPc[a * LM + l * l + mi] += acc0 + acc1;                                                         \
-                    continue;                                                                                        \
-                }                                                                                                    \
-                for (int si = 0; si < S; si++) {                                                                     \
-                    const int n = ns[hh * S + si];                                                                   \
-                    const int *ki = kidx + (hh * S + si) * NB;                                                       \
-                    double acc0 = 0.0, acc1 = 0.0;                                                                   \
-                    int q = 0;                                                                                       \
-_Pragma("unroll 2")                                                                                                  \
-                    for (; q + 1 < n; q += 2) {                                                                      \
-                        const int k0 = ki[q], k1 = ki[q + 1];                                                        \
-                        acc0 += Rc[a * RT + k0] * Yc[mi * RT + k0];                                                  \
-                        acc1 += Rc[a * RT + k1] * Yc[mi * RT + k1];                                                  \
-                    }                                                                                                \
-                    if (q < n) {                                                                                     \
-                        const int k0 = ki[q];                                                                        \
-                        acc0 += Rc[a * RT + k0] * Yc[mi * RT + k0];                                                  \
-                    }                                                                                                \
-                    cPc[(si * N + a) * LM + l * l + mi] += acc0 + acc1;                                              \
-                }                                                                                                    \
-            }
+// Which groups a forward wavefront accumulates: 1 the groups of m < 4, 2 those of m >= 4, 3 all.
+template <int L, int SETS>
+struct FwdGroups {
+    static constexpr int count = SETS == 1 ? 2 * L + 1 : SETS == 2 ? 2 * (L - 3) + (L >= 8 ? 2 : 0) : soap_groups(L);
+    __host__ __device__ static constexpr int index(int l, int v) {   // place of (level, group) in this wavefront's list
+        return SETS == 1 ? (l == 0 ? 0 : 2 * l - 1 + v) : SETS == 2 ? 2 * (l - 4) + v - 2 : lev_base(l) + v;
+    }
+    __device__ static __forceinline__ int group(int idx) {           // and back, to the group number
+        if (SETS == 3) return idx;
+        if (SETS == 1) {
+            const int l = (idx + 1) >> 1;
+            return idx == 0 ? 0 : lev_base(l) + ((idx + 1) & 1);
+        }
+        const int l = 4 + (idx >> 1);
+        return l > 8 ? lev_base(8) + 4 + (idx & 1) : lev_base(l) + 2 + (idx & 1);
+    }
+};
 
-// PREG: each lane's Legendre levels in registers, with the level loop unrolled (no
-// LDS rows, more registers: two wavefronts per SIMD); otherwise two LDS rows per
-// lane and a rolled level loop (three wavefronts per SIMD).
-// CPW: centres per wavefront.  A centre's chunk of 32 neighbours occupies 32 lanes,
-// so with two centres lanes 0-31 and 32-63 stage the neighbours of one centre each
-// and every staging instruction serves two centres.
-template <int N, int L, bool PREG, int CPW>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PREG ? 2 : WPE_FWD, 8))) void k_soap_fwd_x(
-    SoapDev sp, int nc, const int *__restrict__ centres, const int *__restrict__ Z, const int *__restrict__ nb_off,
-    const int *__restrict__ nb_j, const double *__restrict__ nb_r, const double *__restrict__ nb_d, double *X,
-    double *norm_out, double *cbuf) {
+// LDS layout of the forward kernel, in doubles (shared by the kernel and its launcher)
+struct FwdLds {
+    int slots, gs, rs, cs, p_off, c_off, tab_off, tail, total;   // total in bytes
+    __host__ __device__ FwdLds(int NA, int L, int S, int nw, int dim, bool p_lds, bool c_lds) {
+        slots = kSoapPass + 16 * (S - 1);
+        gs = 64 * NA + 4;                       // partial sums of one group; 4 apart so that groups fall on distinct banks
+        rs = 4 * gs;                            // four groups at a time per wavefront
+        cs = 4 * soap_groups(L) + 1;            // odd: rows on distinct banks
+        const int tab = kFwdFields * slots;
+        // a single wavefront is done with the table before it reduces: they share their place
+        const int red = nw * rs, front = nw == 1 && S == 1 ? (tab > red ? tab : red) : tab + red;
+        tab_off = 0;
+        p_off = nw == 1 && S == 1 ? 0 : tab;    // the reduction area, later the power spectrum
+        const int p_need = p_lds ? dim : 0;
+        const int room = front - p_off;
+        c_off = p_off + (p_need > room ? p_need : room);
+        c_off = (c_off + 1) & ~1;
+        tail = c_off + (c_lds ? S * NA * 4 * cs : 0);
+        total = (tail + nw) * 8 + 2 * S * 4;   // followed by the constant tables
+        total = (total + 7) & ~7;
+    }
+};
+
+// Forward: a block of NW wavefronts takes cpb centres in turn; a centre's neighbours are
+// fetched while the one before is worked on.  A wavefront takes the neighbours of one
+// species (and, SPLIT, the harmonics of m < 4 or m >= 4) in tiles of 16: lane 4 n + g
+// evaluates neighbour n's radial functions of a = g, g+4, .. and its harmonics of m = g, g+4,
+// which are the operands of 4x4x4 products whose four blocks are four quarters of the tile.
+// The quarters are summed through LDS once per centre, T and the power spectrum follow as
+// further 4x4x4 products.  135612 Si centres at 8/6: 1.10 -> 0.46 ms against lanes accumulating
+// c' from levels staged in LDS (700 MB of X and c written at 1.5 TB/s; VALU issue 47% and the
+// matrix pipe 21% of it); 32768 SiC centres at 12/8: 3.19 -> 0.77 ms.  SP: the number of species where it is fixed at compile time, else 0.
+template <int N, int L, int NW, bool SPLIT, int SP>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(N <= 8 && L <= 6 ? 3 : 2, 8))) void k_soap_fwd_x(
+    SoapDev sp, int nc, int cpb, const int *__restrict__ centres, const int *__restrict__ Z,
+    const int *__restrict__ nb_off, const int *__restrict__ nb_j, const double *__restrict__ nb_r,
+    const double *__restrict__ nb_d, double *X, double *norm_out, double *cbuf, int p_lds_, int c_lds_) {
     extern __shared__ double lds[];
-    constexpr int LM = (L + 1) * (L + 1);
-    constexpr int YW = 2 * L + 1;
-    constexpr int NB = kSoapChunk;
-    const int K = sp.K, KLM = K * LM, S = sp.S;
-    const int KLMp = (KLM + 1) & ~1;   // per-centre c' rows, 16-byte aligned
-    double *Ts = lds;              // N*N
-    double *rbs = Ts + N * N;      // N grid points, then exp(-alpha r_a^2) and 1/a (N each)
-    double *gA = rbs + N, *iA = gA + N;
-    double *cP = rbs + 3 * N;      // CPW x K*LM: c' during accumulation, c after the transform
-    // The staged levels are stored one row per radial point a (Rl) and per m slot (Yl),
-    // neighbours along the row: the writes of 32 lanes are consecutive, and the dense
-    // accumulation reads two neighbours per 16-byte access.  The row stride RT = NB + 2
-    // keeps rows 16-byte aligned (N (N + 3) and KLMp are even) and puts successive rows
-    // 16 bytes apart in the bank cycle.
-    constexpr int RT = NB + 2;     // row stride of Rl and Yl
-    constexpr int PR = (2 * (L + 2)) | 1;   // row stride of a lane's two Legendre rows (odd: distinct banks)
-    double *Rl = cP + CPW * KLMp;  // CPW x N x RT: fc F_l(a) of neighbour k of centre h at Rl[(h N + a) RT + k]
-    double *Yl = Rl + CPW * N * RT;   // CPW x YW x RT: Y_l,m of neighbour k at Yl[(h YW + slot) RT + k]
-    double *Pq0 = Yl + CPW * YW * RT; // 32 CPW x PR: the staging lanes' Legendre rows (not PREG)
-    int *kidx = (int *)(Pq0 + (PREG ? 0 : 32 * CPW * PR));   // CPW x S x NB: the chunk's neighbours of each species
-    int *ns = kidx + CPW * S * NB; // their counts
-    const int lane = threadIdx.x;
-    const int h = CPW == 2 ? lane >> 5 : 0, kl = lane & 31;   // this lane's centre and neighbour slot
-    const int desc = CPW * blockIdx.x + h;
-    const bool valid = desc < nc;   // this lane's centre exists (the same for all lanes with CPW 1)
-    const int ci = valid ? centres[desc] : 0;
-    double *Rh = Rl + h * (N * RT), *Yh = Yl + h * (YW * RT);
-    for (int e = lane; e < N * N; e += 64) Ts[e] = sp.T[e];
-    if (lane < N) {
-        rbs[lane] = sp.rb[lane];
-        gA[lane] = exp(-sp.alpha * sp.rb[lane] * sp.rb[lane]);
-        iA[lane] = lane > 0 ? 1.0 / (double)lane : 0.0;
+    constexpr int NA = (N + 3) / 4, LM = (L + 1) * (L + 1);
+    const int S = SP ? SP : sp.S, K = S * N, KLM = K * LM, d = K * (K + 1) / 2 * (L + 1) + 1;
+    const bool p_lds = SP || p_lds_, c_lds = SP || c_lds_;
+    const FwdLds lo(NA, L, S, NW, d, p_lds, c_lds);
+    double *tab = lds + lo.tab_off, *red = lds + lo.p_off, *pL = red, *cL = lds + lo.c_off, *ssw = lds + lo.tail;
+    int *sb = (int *)(ssw + NW), *sc = sb + S;
+    SoapTables<N, L> tb(lds + lo.total / 8);
+    tb.fill(sp, 64 * NW);
+    const int lane = threadIdx.x & 63;
+    const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int d0 = blockIdx.x * cpb, dn = min(d0 + cpb, nc);
+    int ci = centres[d0], cn = centres[min(d0 + 1, dn - 1)];
+    int p0 = nb_off[ci], np = nb_off[ci + 1] - p0;
+    SoapNb nb;
+    if (w == NW - 1) {
+        nb.load(p0, min(kSoapPass, np), nb_j, nb_r, nb_d);
+        nb.species(min(kSoapPass, np), Z);
     }
-    for (int e = lane; e < CPW * KLMp; e += 64) cP[e] = 0.0;
     __syncthreads();
-    const int p0 = valid ? nb_off[ci] : 0, np = valid ? nb_off[ci + 1] - p0 : 0;
-    int npmax = np;   // chunks of the wave (uniform): those of its larger centre
-    if (CPW == 2) npmax = max(np, __shfl_xor(np, 32, 64));
-    for (int c0 = 0; c0 < npmax; c0 += NB) {
-        const int nk = max(0, min(NB, np - c0));
-        __syncthreads();   // the previous chunk's reads of the lists are done
-        int s = -1;
-        double fc = 0.0, ux = 0.0, uy = 0.0, uz = 0.0;
-        Rad<N> rs;
-        if (kl < nk && lane < 32 * CPW) {
-            const int p = p0 + c0 + kl;
-            const double r = nb_r[p];
-            s = species_s(sp, Z[nb_j[p]]);
-            if (r > sp.rc) s = -1;
-            if (s >= 0) {
-                fc = fc_s(r, sp.rc, sp.ctw);
-                rs.init(rbs, gA, iA, sp.alpha, r);
-                const double ir = 1.0 / r;
-                ux = nb_d[3 * p] * ir; uy = nb_d[3 * p + 1] * ir; uz = nb_d[3 * p + 2] * ir;
+    for (int desc = d0; desc < dn; desc++) {
+        // the next centre's pairs and the index of the one after it
+        const int pn = nb_off[cn], nn = nb_off[cn + 1] - pn;
+        const int c2 = centres[min(desc + 2, dn - 1)];
+        const int csp = species_s(sp, S, Z[ci]);
+        double *co = cbuf + (size_t)desc * KLM;
+
+        auto unit = [&](auto sets_tag, int s, bool first_pass, bool last_pass) {
+            constexpr int SETS = decltype(sets_tag)::value;
+            using FG = FwdGroups<L, SETS>;
+            constexpr int NGS = FG::count;
+            const int ln0 = fresh_lane(), i4 = ln0 & 3;
+            SoapLane<N> rl;
+            rl.setup(tb.rt, i4);
+            double acc[NGS][NA];
+#pragma unroll
+            for (int i = 0; i < NGS; i++)
+#pragma unroll
+                for (int u = 0; u < NA; u++) acc[i][u] = 0.0;
+            for (int c0 = 0; c0 < np; c0 += kSoapPass) {
+                const int nk = min(kSoapPass, np - c0);
+                if (first_pass || np > kSoapPass) {   // a single pass of neighbours stays staged for every unit
+                    block_lds_sync<NW>();
+                    if (w == NW - 1) {
+                        if (!first_pass || c0 > 0) {
+                            nb.load(p0 + c0, nk, nb_j, nb_r, nb_d);
+                            nb.species(nk, Z);
+                        }
+                        soap_stage<N, false>(sp, S, nb, p0 + c0, nk, tab, lo.slots, sb, sc, nullptr);
+                    }
+                    block_lds_sync<NW>();
+                }
+                if (s < 0) continue;
+                const int base = sb[s], cnt = sc[s];
+                for (int t = 0; t < cnt; t += 16) {
+                    const int off = t + (lane >> 2);
+                    const int sl = base + min(off, cnt - 1);
+                    const double x = tab[kUx * lo.slots + sl], y = tab[kUy * lo.slots + sl];
+                    rl.z = tab[kUz * lo.slots + sl];
+                    const double e0 = off < cnt ? tab[kE0 * lo.slots + sl] : 0.0;
+                    rl.radial(sp, i4, tab[kIxq * lo.slots + sl], e0, tab[kQ * lo.slots + sl], tab[kQi * lo.slots + sl]);
+                    // (x + i y)^m of m = i4 and i4 + 4
+                    const double x2 = x * x - y * y, y2 = 2.0 * x * y;
+                    const double x3 = x2 * x - y2 * y, y3 = x2 * y + y2 * x;
+                    const double Aa = i4 == 0 ? 1.0 : i4 == 1 ? x : i4 == 2 ? x2 : x3;
+                    const double Ba = i4 == 0 ? 0.0 : i4 == 1 ? y : i4 == 2 ? y2 : y3;
+                    const double x4 = x2 * x2 - y2 * y2, y4 = 2.0 * x2 * y2;
+                    const double Ab = Aa * x4 - Ba * y4, Bb = Aa * y4 + Ba * x4;
+                    rl.pA = rl.pA1 = rl.pB = rl.pB1 = 0.0;
+#pragma unroll
+                    for (int l = 0; l <= L; l++) {
+                        double F[NA];
+#pragma unroll
+                        for (int u = 0; u < NA; u++) F[u] = rl.f(l, u);
+                        if constexpr (SETS & 1) {
+                            const double p = rl.legendre(l, 0, rl.mA2, rl.pA, rl.pA1);
+                            rl.pA1 = rl.pA;
+                            rl.pA = p;
+                            const double ya = p * Aa, yb = p * Ba;
+#pragma unroll
+                            for (int u = 0; u < NA; u++) {
+                                acc[FG::index(l, 0)][u] = mfma4(F[u], ya, acc[FG::index(l, 0)][u]);
+                                if (l > 0) acc[FG::index(l, 1)][u] = mfma4(F[u], yb, acc[FG::index(l, 1)][u]);
+                            }
+                        }
+                        if constexpr (SETS & 2) {
+                            if (l >= 4) {
+                                const double p = rl.legendre(l, 4, rl.mB2, rl.pB, rl.pB1);
+                                rl.pB1 = rl.pB;
+                                rl.pB = p;
+                                const double ya = p * Ab, yb = p * Bb;
+#pragma unroll
+                                for (int u = 0; u < NA; u++) {
+                                    acc[FG::index(l, 2)][u] = mfma4(F[u], ya, acc[FG::index(l, 2)][u]);
+                                    acc[FG::index(l, 3)][u] = mfma4(F[u], yb, acc[FG::index(l, 3)][u]);
+                                }
+                            }
+                            if (l >= 8) {   // m = 8 in slot 0; the other slots' factor is zero
+                                const double ya = x4 * x4 - y4 * y4, yb = 2.0 * x4 * y4;
+                                constexpr int v4 = L >= 8 ? 4 : 2, v5 = L >= 8 ? 5 : 3;
+#pragma unroll
+                                for (int u = 0; u < NA; u++) {
+                                    acc[FG::index(l, v4)][u] = mfma4(F[u], ya, acc[FG::index(l, v4)][u]);
+                                    acc[FG::index(l, v5)][u] = mfma4(F[u], yb, acc[FG::index(l, v5)][u]);
+                                }
+                            }
+                        }
+                        if (l < L) rl.step(l);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            if (last_pass && desc + 1 < dn && w == NW - 1)   // the next centre's neighbours set out
+                nb.load(pn, min(kSoapPass, nn), nb_j, nb_r, nb_d);
+            if (s < 0) return;
+            // sum the four quarters, four groups at a time, transform, and store c (times the
+            // harmonics' factor, as the adjoint takes it)
+            const int ln = fresh_lane(), k4 = ln >> 4, b4 = (ln >> 2) & 3;
+            double TA[NA][NA];   // T[a = 4u + k][b = 4v + i] of the transform's operand
+#pragma unroll
+            for (int u = 0; u < NA; u++)
+#pragma unroll
+                for (int v = 0; v < NA; v++) {
+                    const int a = 4 * u + k4, b = 4 * v + i4;
+                    TA[v][u] = tb.t(a, b);
+                }
+            double *rw = red + w * lo.rs;
+            constexpr int NQ = (NGS + 3) / 4;
+#pragma unroll
+            for (int t = 0; t < NQ; t++) {
+                wave_lds_sync();
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (4 * t + i < NGS)
+#pragma unroll
+                        for (int u = 0; u < NA; u++)
+                            rw[i * lo.gs + 64 * u + lane] = acc[4 * t + i < NGS ? 4 * t + i : 0][u];
+                wave_lds_sync();
+                const bool ok = 4 * t + 3 < NGS || 4 * t + b4 < NGS;
+                const int g = FG::group(ok ? 4 * t + b4 : 0);
+                const double nk = ok ? tb.gn[4 * g + i4] : 0.0;
+                const int pos = ok ? tb.pos[4 * g + i4] & 0xffff : 0xffff;
+                double Bv[NA];
+#pragma unroll
+                for (int u = 0; u < NA; u++) {
+                    const double *q = rw + (ok ? b4 : 0) * lo.gs + 64 * u + 16 * k4 + i4;
+                    Bv[u] = ((q[0] + q[4]) + (q[8] + q[12])) * nk;
+                }
+#pragma unroll
+                for (int v = 0; v < NA; v++) {
+                    double D = 0.0;
+#pragma unroll
+                    for (int u = 0; u < NA; u++) D = mfma4(TA[v][u], Bv[u], D);
+                    const int row = 4 * v + k4;
+                    if (v == 0 && k4 == 0 && i4 == 0 && ok && g == 0 && s == csp) D += sp.cw * sp.u00 * nk;
+                    if (c_lds && ok) cL[(s * NA * 4 + row) * lo.cs + 4 * g + i4] = D;
+                    if (pos != 0xffff && (N % 4 == 0 || row < N)) co[(s * N + row) * LM + pos] = D * nk;
+                }
+            }
+        };
+        const int nunits = SPLIT ? 2 * S : S;
+        for (int u0 = 0; u0 < nunits; u0 += NW) {
+            const int un = u0 + w;
+            const int s = un < nunits ? (SPLIT ? un >> 1 : un) : -1;
+            if constexpr (SPLIT) {
+                if (un & 1) unit(std::integral_constant<int, 2>{}, s, u0 == 0, u0 + NW >= nunits);
+                else unit(std::integral_constant<int, 1>{}, s, u0 == 0, u0 + NW >= nunits);
+            } else {
+                unit(std::integral_constant<int, 3>{}, s, u0 == 0, u0 + NW >= nunits);
             }
         }
-        for (int si = 0; S > 1 && si < S; si++) {   // neighbours beyond the cutoff are in no list
-            const bool mine = lane < 32 * CPW && s == si;
-            const unsigned long long mk = __ballot(mine);
-            const unsigned long long mh = (mk >> (32 * h)) & 0xffffffffull;   // this centre's half
-            if (mine) kidx[(h * S + si) * NB + __popcll(mh & ((1ull << kl) - 1ull))] = kl;
-            if (kl == 0 && lane < 32 * CPW) ns[h * S + si] = __popcll(mh);
-        }
-        if constexpr (PREG) {
-            double P0[L + 2], P1[L + 2];
+        if (c_lds) block_lds_sync<NW>();
+        else __syncthreads();
+        // power spectrum: blocks of 4 x 4 row pairs (gi >= gj), four pairs per product
+        const int R = S * NA, npair = R * (R + 1) / 2;
+        double *xo = X + (size_t)desc * d;
+        double ss = 0.0;
+        for (int q0 = 4 * w; q0 < npair; q0 += 4 * NW) {
+            const int ln = fresh_lane(), k4 = ln >> 4, b4 = (ln >> 2) & 3, i4 = ln & 3;
+            const int pi = min(q0 + b4, npair - 1);
+            int gi = (int)((sqrtf(8.0f * (float)pi + 1.0f) - 1.0f) * 0.5f);
+            while ((gi + 1) * (gi + 2) / 2 <= pi) gi++;
+            while (gi * (gi + 1) / 2 > pi) gi--;
+            const int gj = pi - gi * (gi + 1) / 2;
+            const int ri = 4 * gi + k4, rj = 4 * gj + i4;   // rows of this lane's result
+            const int ai = ri % (4 * NA), aj = rj % (4 * NA);
+            const int ia = ri / (4 * NA) * N + ai, jb = rj / (4 * NA) * N + aj;
+            const bool ok = q0 + b4 < npair && ai < N && aj < N && ia >= jb;
+            const double f = ia != jb ? 1.4142135623730950488 : 1.0;
+            const int q = (ia * (ia + 1) / 2 + jb) * (L + 1);
+            if (c_lds) {
+                const double *ca = cL + (4 * gi + i4) * lo.cs + k4, *cb = cL + (4 * gj + i4) * lo.cs + k4;
 #pragma unroll
-            for (int l = 0; l <= L; l++) {
-                double *cur = (l & 1) ? P1 : P0;
-                const double *prv = (l & 1) ? P0 : P1;
-                SOAP_FWD_LEVEL(l, cur, prv);
+                for (int l = 0; l <= L; l++) {
+                    double D = 0.0;
+#pragma unroll
+                    for (int v = 0; v < lev_groups(l); v++)
+                        D = mfma4(ca[4 * (lev_base(l) + v)], cb[4 * (lev_base(l) + v)], D);
+                    const double p = D * (f * tb.isq[l]);
+                    if (ok) {
+                        if (p_lds) pL[q + l] = p;
+                        else xo[q + l] = p;
+                        ss += p * p;
+                    }
+                }
+            } else {   // many species: c is read back from memory
+                const int ra = 4 * gi + i4, rb = 4 * gj + i4;
+                const bool oa = ra % (4 * NA) < N, ob = rb % (4 * NA) < N;
+                const double *ca = co + (size_t)(ra / (4 * NA) * N + ra % (4 * NA)) * LM;
+                const double *cb = co + (size_t)(rb / (4 * NA) * N + rb % (4 * NA)) * LM;
+                for (int l = 0; l <= L; l++) {
+                    double D = 0.0;
+                    for (int v = 0; v < lev_groups(l); v++) {
+                        const int pos = c_gpos[4 * (lev_base(l) + v) + k4];
+                        const double f1 = c_ginv[4 * (lev_base(l) + v) + k4];
+                        D = mfma4(oa && pos >= 0 ? ca[pos] * f1 : 0.0, ob && pos >= 0 ? cb[pos] * f1 : 0.0, D);
+                    }
+                    const double p = D * (f * tb.isq[l]);
+                    if (ok) {
+                        if (p_lds) pL[q + l] = p;
+                        else xo[q + l] = p;
+                        ss += p * p;
+                    }
+                }
             }
-        } else {
-            double *Pq = Pq0 + lane * PR;   // this lane's two Legendre rows
-#pragma unroll 1
-            for (int l = 0; l <= L; l++) {
-                double *cur = Pq + (l & 1) * (L + 2);
-                const double *prv = Pq + ((l + 1) & 1) * (L + 2);
-                SOAP_FWD_LEVEL(l, cur, prv);
-            }
         }
-    }
-    __syncthreads();
-    // c = T^T c', one (centre, species, lm) column per lane, in place
-    for (int it = lane; it < CPW * S * LM; it += 64) {
-        const int hh = CPW == 1 ? 0 : it / (S * LM), r_ = it - hh * (S * LM), si = r_ / LM, lm = r_ - si * LM;
-        double *cc = cP + hh * KLMp;
-        RELOAD_BARRIER();   // T is re-read from LDS for every column
-        double cp[N];
+        if (desc + 1 < dn && w == NW - 1) nb.species(min(kSoapPass, nn), Z);
+        ss = wave_sum_s(ss);
+        if (NW > 1 && lane == 0) ssw[w] = ss;
+        if (p_lds) block_lds_sync<NW>();
+        else __syncthreads();
+        if (NW > 1) {
+            ss = ssw[0];
 #pragma unroll
-        for (int a = 0; a < N; a++) cp[a] = cc[(si * N + a) * LM + lm];
-#pragma unroll
-        for (int b = 0; b < N; b++) {
-            double acc = 0.0;
-#pragma unroll
-            for (int a = 0; a < N; a++) acc += Ts[a * N + b] * cp[a];
-            cc[(si * N + b) * LM + lm] = acc;
-            RELOAD_BARRIER();   // one column of T in registers at a time
+            for (int i = 1; i < NW; i++) ss += ssw[i];
         }
-    }
-    __syncthreads();
-    if (kl == 0 && valid && lane < 32 * CPW) {   // centre atom term
-        const int sc = species_s(sp, Z[ci]);
-        if (sc >= 0) cP[h * KLMp + (sc * N) * LM] += sp.cw * sp.u00 * c_ynorm[0];
-    }
-    __syncthreads();
-    // power spectrum, written unnormalised and rescaled in place by the same lanes
-    const int d = sp.dim;
-    const int d0 = CPW * blockIdx.x;
-    double ss[CPW];
-#pragma unroll
-    for (int hh = 0; hh < CPW; hh++) ss[hh] = 0.0;
-    for (int it = lane; it < CPW * (d - 1); it += 64) {
-        const int hh = CPW == 1 ? 0 : it / (d - 1), q = it - hh * (d - 1);
-        if (d0 + hh >= nc) continue;
-        const double *cc = cP + hh * KLMp;
-        const int code = sp.qmap[q];
-        const int ia = code >> 16, jb = (code >> 8) & 0xff, l = code & 0xff;
-        double v = 0.0;
-        for (int m = -l; m <= l; m++) v += cc[ia * LM + l * l + l + m] * cc[jb * LM + l * l + l + m];
-        v *= (ia != jb ? 1.4142135623730950488 : 1.0) / sqrt(2.0 * l + 1.0);
-        X[(size_t)(d0 + hh) * d + q] = v;
-#pragma unroll
-        for (int g2 = 0; g2 < CPW; g2++)
-            if (g2 == hh) ss[g2] += v * v;
-    }
-    double inv[CPW];
-#pragma unroll
-    for (int hh = 0; hh < CPW; hh++) {
-        const double nrm = sqrt(wave_sum_s(ss[hh]));
-        inv[hh] = nrm > 0.0 ? 1.0 / nrm : 0.0;
-        if (lane == 0 && d0 + hh < nc) {
-            X[(size_t)(d0 + hh) * d + d - 1] = 0.0;
-            norm_out[d0 + hh] = nrm;
+        const double nrm = sqrt(ss);
+        const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
+        for (int q = threadIdx.x; q < d - 1; q += 64 * NW) xo[q] = (p_lds ? pL[q] : xo[q]) * inv;
+        if (threadIdx.x == 0) {
+            xo[d - 1] = 0.0;
+            norm_out[desc] = nrm;
         }
-    }
-    for (int it = lane; it < CPW * (d - 1); it += 64) {
-        const int hh = CPW == 1 ? 0 : it / (d - 1), q = it - hh * (d - 1);
-        if (d0 + hh >= nc) continue;
-        double sc = inv[0];
-#pragma unroll
-        for (int g2 = 1; g2 < CPW; g2++)
-            if (g2 == hh) sc = inv[g2];
-        X[(size_t)(d0 + hh) * d + q] *= sc;
-    }
-    for (int hh = 0; hh < CPW; hh++) {
-        if (d0 + hh >= nc) break;
-        double *co = cbuf + (size_t)(d0 + hh) * KLM;
-        for (int e = lane; e < KLM; e += 64) co[e] = cP[hh * KLMp + e];
+        ci = cn;
+        cn = c2;
+        p0 = pn;
+        np = nn;
+        if (NW > 1) block_lds_sync<NW>();   // the power spectrum's place is free again
     }
 }
 
-// Adjoint.  dE/dc in the orthonormal basis is transformed once per centre to
-// the primitive basis, dc'[a][lm] = sum_b T[a][b] dc[b][lm], so that per
-// neighbour and (l, m): sum_b dc g_b = fc S0 and sum_b dc dg_b/dr =
-// fc (cl S0 + 2 alpha S1) + dfc S0 with S0 = sum_a F_l(a) dc'[a], S1 =
-// sum_a r_a F_(l+1)(a) dc'[a] and cl = -2 alpha r + l / r.
-// OCC: the occupancy the register budget is cut for.  The higher one pays off when
-// there are many more wavefronts than SIMDs; a small launch runs faster with the
-// larger budget.
-template <int N, int L, int OCC>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(OCC, 8))) void k_soap_bwd_x(
+// LDS layout of the adjoint kernel, in doubles: the neighbour table, dE/dc' of SB species as
+// operands, dE/dp (p_lds), a wave sum per wavefront, then the slot tables
+struct BwdLds {
+    int slots, a_off, p_off, w_off, total;
+    __host__ __device__ BwdLds(int NA, int L, int S, int SB, int nw, int dim, bool p_lds) {
+        slots = kSoapPass + 16 * (S - 1);
+        a_off = kBwdFields * slots;
+        p_off = a_off + SB * soap_groups(L) * NA * 16;
+        w_off = p_off + (p_lds ? dim : 0);
+        total = (w_off + nw) * 8 + (2 * S + slots) * 4;   // followed by the constant tables
+        total = (total + 7) & ~7;
+    }
+};
+
+// Adjoint: a block of NW wavefronts takes cpb centres in turn; a centre's neighbours (and
+// where they fit the registers X and G) are fetched while the one before is worked on.
+// dE/dp = (G - x (x.G)) / |p| is staged in LDS; dE/dc_l = P_l c_l and dE/dc' = T dE/dc follow as
+// chained 4x4x4 products, four harmonic groups at a time, the result of the first being the
+// operand of the second as it stands.  Then tiles of 16 neighbours: lane 16 g + n holds
+// neighbour n's radial functions of a = g, g+4, .. and their r derivatives, which multiply
+// dE/dc' from LDS; the products come out in the lanes that hold the harmonics they belong
+// to (m = g, g+4).  With S0_lm = sum_a F_l(a) dc'[a][lm] and S1_lm = sum_a F_l'(a) dc'[a][lm]
+// the pair's force is (fc sum S1 Y + dfc sum S0 Y) u + fc (V - u (u.V)) / r, V = sum S0 gradY.
+// The sums over l are kept per m with the Legendre factors only; (x + i y)^m enters once at
+// the end, and a last product with unit rows sums the lanes of a neighbour.  135612 Si
+// centres at 8/6: 1.09 -> 0.63 ms against a lane per neighbour reading dE/dc' from LDS (VALU issue
+// 44%, matrix pipe 26% of it); 32768 SiC centres at 12/8: 3.80 -> 0.90 ms.  A wavefront per centre and
+// 2 wavefronts per SIMD: with spills at 3 the reloads queue behind the data on their way (1.07 ms).
+// SP: the number of species where it is fixed at compile time, else 0.
+template <int N, int L, int NW, int SP>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_soap_bwd_x(
     SoapDev sp, int nc, int cpb, const int *__restrict__ centres, const int *__restrict__ Z,
     const int *__restrict__ nb_off, const int *__restrict__ nb_j, const double *__restrict__ nb_r,
     const double *__restrict__ nb_d, const double *__restrict__ X, const double *__restrict__ G,
-    const double *__restrict__ norm, const double *__restrict__ cbuf, double *pairF, int whole) {
-    // cpb centres per wavefront: a centre has ~30 neighbours, so one lane per
-    // neighbour over 64/cpb lanes keeps the wavefront busy.
-    // LDS: T, the grid tables, dE/dc (then dE/dc') of each centre, the centre
-    // scalars, and one staging region used first for the per-l blocks of the
-    // dE/dc product and then for the lanes' Legendre rows.
+    const double *__restrict__ norm, const double *__restrict__ cbuf, double *pairF, int p_lds_, int SB_, int add) {
     extern __shared__ double lds[];
-    constexpr int LM = (L + 1) * (L + 1);
-    constexpr int PR = (2 * (L + 2)) | 1;   // odd: a lane's rows on distinct banks
-    const int K = sp.K, KLM = K * LM, d = sp.dim, S = sp.S;
-    double *Ts = lds;              // N*N
-    double *rbs = Ts + N * N;      // N grid points, then exp(-alpha r_a^2) and 1/a (N each)
-    double *gA = rbs + N, *iA = gA + N;
-    double *dcs_all = rbs + 3 * N; // cpb x K*LM
-    double *csc = dcs_all + cpb * KLM;   // cpb x (dot, 1/|p|)
-    double *stg = csc + 2 * cpb;   // max(K*K + K*(2L+1), 64*PR), or with whole max(cpb*(L+1)*(K*K+2) | cpb*d, 64*PR)
-    const int lane = threadIdx.x;
-    const int d0 = cpb * blockIdx.x;
-    const int nh = min(cpb, nc - d0);
-    for (int e = lane; e < N * N; e += 64) Ts[e] = sp.T[e];
-    if (lane < N) {
-        rbs[lane] = sp.rb[lane];
-        gA[lane] = exp(-sp.alpha * sp.rb[lane] * sp.rb[lane]);
-        iA[lane] = lane > 0 ? 1.0 / (double)lane : 0.0;
-    }
-    for (int h = 0; h < nh; h++) {
-        const int desc = d0 + h;
+    constexpr int NA = (N + 3) / 4, LM = (L + 1) * (L + 1), NG = soap_groups(L), NQ = (NG + 3) / 4;
+    constexpr int DC = SP * N * (SP * N + 1) / 2 * (L + 1);            // components (less the last, zero one)
+    constexpr int QR = SP ? (DC + 64 * NW - 1) / (64 * NW) : 1;        // of them per lane
+    constexpr bool AHEAD = SP && QR <= 4;                              // X and G of the next centre in registers
+    constexpr int UN = SP ? (NQ * SP + NW - 1) / NW : 1;               // quads of groups per wavefront (one species each)
+    constexpr bool CAHEAD = SP && UN * SP * NA <= 12;                  // the next centre's c likewise
+    static_assert(SP <= 1 || NW == 2 * SP, "wavefronts are dealt evenly to the species");
+    const int S = SP ? SP : sp.S, KLM = S * N * LM, d = SP ? DC + 1 : sp.dim;
+    const int SB = SP ? SP : SB_;
+    const bool p_lds = SP || p_lds_;
+    const BwdLds lo(NA, L, S, SB, NW, d, p_lds);
+    double *tab = lds, *Aop = lds + lo.a_off, *P = lds + lo.p_off, *ws = lds + lo.w_off;
+    int *sb = (int *)(ws + NW), *sc = sb + S, *pair = sc + S;
+    SoapTables<N, L> tb(lds + lo.total / 8);
+    tb.fill(sp, 64 * NW);
+    const int lane = threadIdx.x & 63;
+    const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int d0 = blockIdx.x * cpb, dn = min(d0 + cpb, nc);
+    double xr[QR], gr[QR];   // X and G of this lane's components
+    auto load_xg = [&](int desc) {
         const double *x = X + (size_t)desc * d, *gg = G + (size_t)desc * d;
-        double dot = 0.0;
-        for (int q = lane; q < d; q += 64) dot += x[q] * gg[q];
-        dot = wave_sum_s(dot);
-        if (lane == 0) {
-            const double nrm = norm[desc];
-            csc[2 * h] = dot;
-            csc[2 * h + 1] = nrm > 0.0 ? 1.0 / nrm : 0.0;
+#pragma unroll
+        for (int i = 0; i < QR; i++) {
+            const int q = threadIdx.x + 64 * NW * i;
+            xr[i] = q < d - 1 ? x[q] : 0.0;
+            gr[i] = q < d - 1 ? gg[q] : 0.0;
         }
-        const double nrm = norm[desc];
-        const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
-        if (whole == 1) {   // dE/dp of every centre staged together; c is read from cbuf
-            double *dpL = stg + h * d;
-            for (int q = lane; q < d; q += 64) dpL[q] = (gg[q] - x[q] * dot) * inv;
-        } else if (whole == 2) {   // the level blocks P_l (below) of every centre, all levels
-            // level blocks K*K + 2 doubles apart: rows of different levels read by one group
-            // of lanes then fall on different bank groups
-            const int KKp = K * K + 2;
-            double *Ph = stg + h * (L + 1) * KKp;
-            for (int e = lane; e < (L + 1) * K * K; e += 64) {
-                const int l = e / (K * K), r = e - l * K * K, ia = r / K, jb = r - ia * K;
-                const int hi = ia > jb ? ia : jb, lo = ia > jb ? jb : ia;
-                const int q = (hi * (hi + 1) / 2 + lo) * (L + 1) + l;
-                Ph[l * KKp + r] = (gg[q] - x[q] * dot) * inv * (ia == jb ? 2.0 : 1.4142135623730950488) * c_isq[l];
-            }
-        }
+    };
+    if (SP) load_xg(d0);
+    int ci = centres[d0], cn = centres[min(d0 + 1, dn - 1)];
+    int p0 = nb_off[ci], np = nb_off[ci + 1] - p0;
+    SoapNb nb;
+    if (w == NW - 1) {
+        nb.load(p0, min(kSoapPass, np), nb_j, nb_r, nb_d);
+        nb.species(min(kSoapPass, np), Z);
     }
     __syncthreads();
-    if (whole == 2) {   // dE/dc in one pass over (centre, ia, lm): row ia of P_l times column lm of c
-        for (int it = lane; it < nh * KLM; it += 64) {
-            const int h = it / KLM, e = it - h * KLM;
-            const int ia = e / LM, lm = e - ia * LM;
-            const int l = (int)sqrtf((float)lm);   // exact: lm < (l+1)^2 is far from a rounding step
-            const double *Pr = stg + h * (L + 1) * (K * K + 2) + l * (K * K + 2) + ia * K;
-            const double *cL = cbuf + (size_t)(d0 + h) * KLM + lm;
-            double acc = 0.0;
-            if (S == 1) {
-#pragma unroll
-                for (int jb = 0; jb < N; jb++) acc += Pr[jb] * cL[jb * LM];
-            } else {
-                for (int jb = 0; jb < K; jb++) acc += Pr[jb] * cL[jb * LM];
-            }
-            dcs_all[h * KLM + e] = acc;
-        }
-        __syncthreads();
-    }
-    if (whole == 1) {   // dE/dc in one pass over (centre, ia, lm)
-        for (int it = lane; it < nh * KLM; it += 64) {
-            const int h = it / KLM, e = it - h * KLM;
-            const double *dpL = stg + h * d, *cL = cbuf + (size_t)(d0 + h) * KLM;
-            const int ia = e / LM, lm = e - ia * LM;
-            int l = (int)sqrt((double)lm + 0.5);
-            if (l * l > lm) l--;
-            double acc = 0.0;
-            for (int jb = 0; jb < K; jb++) {
-                const int hi = ia > jb ? ia : jb, lo = ia > jb ? jb : ia;
-                const int q = (hi * (hi + 1) / 2 + lo) * (L + 1) + l;
-                acc += dpL[q] * (ia == jb ? 2.0 : 1.4142135623730950488) * cL[jb * LM + lm];
-            }
-            dcs_all[h * KLM + e] = acc / sqrt(2.0 * l + 1.0);
-        }
-        __syncthreads();
-    }
-    // otherwise dE/dc per centre and level l: dc_l (K x 2l+1) = P_l (K x K) c_l (K x 2l+1) with
-    // P_l[ia][jb] = dE/dp_(ia,jb),l x (2 if ia = jb else sqrt 2) / sqrt(2l+1) and
-    // dE/dp = (G - x (x.G)) / |p|; both blocks are staged in LDS one level at a time.
-    for (int h = 0; h < (whole ? 0 : nh); h++) {
-        const int desc = d0 + h;
-        const double *x = X + (size_t)desc * d, *gg = G + (size_t)desc * d;
+    // columns of c of this wavefront's quads of groups (times the harmonics' factor)
+    const int ws_ = SP > 1 ? w / (NW / SP) : 0, tw = SP > 1 ? w % (NW / SP) : w;
+    constexpr int TS = SP > 1 ? NW / SP : NW;
+    double cB[UN][SP ? SP * NA : 1];
+    auto load_c = [&](int desc) {
         const double *cg = cbuf + (size_t)desc * KLM;
-        const double dot = csc[2 * h], inv = csc[2 * h + 1];
-        double *dcL = dcs_all + h * KLM;
-        for (int l = 0; l <= L; l++) {
-            const int W = 2 * l + 1;
-            const double il = 1.0 / sqrt(2.0 * l + 1.0);
-            double *Pl = stg, *Cl = stg + K * K;
-            for (int e = lane; e < K * K; e += 64) {
-                const int ia = e / K, jb = e - ia * K;
-                const int hi = ia > jb ? ia : jb, lo = ia > jb ? jb : ia;
-                const int q = (hi * (hi + 1) / 2 + lo) * (L + 1) + l;
-                Pl[e] = (gg[q] - x[q] * dot) * inv * (ia == jb ? 2.0 : 1.4142135623730950488) * il;
+        const int ln = fresh_lane(), k4 = ln >> 4;
+#pragma unroll
+        for (int i = 0; i < UN; i++) {
+            const int g4 = 16 * (tw + TS * i) + (ln & 15);   // 4 group + slot
+            const int pos = g4 < 4 * NG ? tb.pos[g4] & 0xffff : 0xffff;
+#pragma unroll
+            for (int k = 0; k < SP * NA; k++) {
+                const int aj = 4 * (k % NA) + k4;
+                cB[i][k] = pos != 0xffff && (N % 4 == 0 || aj < N) ? cg[(k / NA * N + aj) * LM + pos] : 0.0;
             }
-            for (int e = lane; e < K * W; e += 64) {
-                const int jb = e / W, m = e - jb * W;
-                Cl[e] = cg[jb * LM + l * l + m];
-            }
-            __syncthreads();
-            for (int e = lane; e < K * W; e += 64) {
-                const int ia = e / W, m = e - ia * W;
-                double acc = 0.0;
-                for (int jb = 0; jb < K; jb++) acc += Pl[ia * K + jb] * Cl[jb * W + m];
-                dcL[ia * LM + l * l + m] = acc;
-            }
-            __syncthreads();
         }
-    }
-    // dc -> dc' in place, one (centre, species, lm) column per lane
-    for (int it = lane; it < nh * S * LM; it += 64) {
-        const int h = it / (S * LM), rem = it - h * S * LM, si = rem / LM, lm = rem - si * LM;
-        double *col = dcs_all + h * KLM + si * N * LM + lm;
-        RELOAD_BARRIER();   // T is re-read from LDS for every column
-        double v[N];
+    };
+    if (CAHEAD) load_c(d0);
+    for (int desc = d0; desc < dn; desc++) {
+        const int pn = nb_off[cn], nn = nb_off[cn + 1] - pn;
+        const int c2 = centres[min(desc + 2, dn - 1)];
+        const double *x = X + (size_t)desc * d, *gg = G + (size_t)desc * d, *cg = cbuf + (size_t)desc * KLM;
+        const double nrm = norm[desc];
+        const int ln = fresh_lane(), k4 = ln >> 4, b4 = (ln >> 2) & 3, i4 = ln & 3;
+        double dot = 0.0;
+        if (SP) {
+            if (!AHEAD && desc > d0) load_xg(desc);
+            if (!CAHEAD) load_c(desc);
 #pragma unroll
-        for (int b = 0; b < N; b++) v[b] = col[b * LM];
-#pragma unroll
-        for (int a = 0; a < N; a++) {
-            double acc = 0.0;
-#pragma unroll
-            for (int b = 0; b < N; b++) acc += Ts[a * N + b] * v[b];
-            col[a * LM] = acc;
-            RELOAD_BARRIER();   // one row of T in registers at a time
+            for (int i = 0; i < QR; i++) dot += xr[i] * gr[i];
+        } else {
+            for (int q = threadIdx.x; q < d; q += 64 * NW) dot += x[q] * gg[q];
         }
-    }
-    __syncthreads();
-    const int lanes_per = 64 / cpb;
-    const int h = lane / lanes_per, sub = lane - h * lanes_per;
-    if (h >= nh) return;
-    const int ci = centres[d0 + h];
-    const double *dcP = dcs_all + h * KLM;
-    double *Pq = stg + lane * PR;   // this lane's two Legendre rows
-    const int p0 = nb_off[ci], np = nb_off[ci + 1] - p0;
-    const double al2 = 2.0 * sp.alpha;
-    const double dr = rbs[1];   // grid spacing: r_a = a dr
-    for (int k = sub; k < np; k += lanes_per) {
-        const int p = p0 + k;
-        const double r = nb_r[p];
-        const int s = species_s(sp, Z[nb_j[p]]);
-        if (r > sp.rc || s < 0) continue;
-        double fc, dfc;
-        fc_dfc_s(r, sp.rc, sp.ctw, fc, dfc);
-        const double ir = 1.0 / r;
-        const double ux = nb_d[3 * p] * ir, uy = nb_d[3 * p + 1] * ir, uz = nb_d[3 * p + 2] * ir;
-        const double *dcs = dcP + s * N * LM;
-        Rad<N> rs;
-        rs.init(rbs, gA, iA, sp.alpha, r);
-        rs.scale_f1();
-        // Per (l, m): S0 = sum_a f_l(a) dc'[a], S1 = sum_a r_a f_(l+1)(a) dc'[a] (dr times the
-        // scaled sum), s2 = fc S0 and s1 = fc (cl S0 + 2 alpha S1) + dfc S0 with cl = -2 alpha r + l / r;
-        // the force on the pair is sum (s1 Y - s2 (u.gY) / r) u + sum s2 gY / r over (l, m), gY the
-        // angular gradient of Y.  Only the sums T0 = sum S0 Y, T0L = sum l S0 Y, T1 = sum S1 Y and
-        // V = sum S0 gY are kept; a pair of real harmonics (m and -m) is handled together.
-        double T0 = 0.0, T0L = 0.0, T1 = 0.0, Vx = 0.0, Vy = 0.0, Vz = 0.0;
-#pragma unroll 1
-        for (int l = 0; l <= L; l++) {
-            double *cur = Pq + (l & 1) * (L + 2);
-            legendre_level(l, uz, Pq + ((l + 1) & 1) * (L + 2), cur);
-            cur[l + 1] = 0.0;
-            double A = 1.0, B = 0.0, Am = 0.0, Bm = 0.0;
-            double t0 = 0.0;
-            for (int m = 0; m <= l; m++) {
-                if (m > 0) {
-                    Am = A;
-                    Bm = B;
-                    const double An = A * ux - B * uy;
-                    B = A * uy + B * ux;
-                    A = An;
-                }
-                const double Nn = c_ynorm[l * (l + 1) / 2 + m];
-                const double NnP = Nn * cur[m], NnPz = Nn * cur[m + 1];
-                const double *dca = dcs + l * l + l + m, *dcb = dcs + l * l + l - m;
-                double S0a = 0.0, S1a = 0.0, S0b = 0.0, S1b = 0.0;
+        dot = wave_sum_s(dot);
+        if (NW > 1) {
+            if (lane == 0) ws[w] = dot;
+            block_lds_sync<NW>();
+            dot = ws[0];
 #pragma unroll
-                for (int a = 0; a < N; a++) {
-                    const double x = dca[a * LM];
-                    S0a += rs.F0[a] * x;
-                    S1a += rs.F1[a] * x;
-                }
-                if (m > 0) {
+            for (int i = 1; i < NW; i++) dot += ws[i];
+        }
+        const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
+        if (SP) {
 #pragma unroll
-                    for (int a = 0; a < N; a++) {
-                        const double x = dcb[a * LM];
-                        S0b += rs.F0[a] * x;
-                        S1b += rs.F1[a] * x;
+            for (int i = 0; i < QR; i++) {
+                const int q = threadIdx.x + 64 * NW * i;
+                if (q < d - 1) P[q] = gr[i] - xr[i] * dot;
+            }
+        } else if (p_lds) {
+            for (int q = threadIdx.x; q < d - 1; q += 64 * NW) P[q] = gg[q] - x[q] * dot;
+        }
+        block_lds_sync<NW>();
+        // dE/dc = P_l c with P_l[ia][jb] = (G - x (x.G))_(ia,jb),l / |p| x (2 if ia = jb else sqrt 2) / sqrt(2l+1):
+        // the diagonal's factor enters with the operand, the columns' factor with the result
+        const double dg = i4 == k4 ? 1.4142135623730950488 : 1.0;
+        const double invs = 1.4142135623730950488 * inv;
+        double TA[NA][NA];   // T[a = 4v + i][b = 4u + k]
+#pragma unroll
+        for (int u = 0; u < NA; u++)
+#pragma unroll
+            for (int v = 0; v < NA; v++) TA[v][u] = tb.t(4 * v + i4, 4 * u + k4);
+        bool staged_first = false;
+        for (int s0 = 0; s0 < S; s0 += SB) {
+            const int ns = min(SB, S - s0);
+            if (s0 > 0) block_lds_sync<NW>();   // the previous species' operands are done with
+            if constexpr (SP > 0) {
+                int qi[SP * NA][NA];   // place of P_0[ia = (s, 4u + i)][jb = (sj, 4kk + k)], -1: none
+#pragma unroll
+                for (int k = 0; k < SP * NA; k++)
+#pragma unroll
+                    for (int u = 0; u < NA; u++) {
+                        const int ai = 4 * u + i4, aj = 4 * (k % NA) + k4;
+                        const int ia = ws_ * N + ai, jb = k / NA * N + aj;
+                        const int hi = max(ia, jb), lw = min(ia, jb);
+                        qi[k][u] = N % 4 == 0 || (ai < N && aj < N) ? (__umul24(hi, hi + 1) / 2 + lw) * (L + 1) : -1;
+                    }
+#pragma unroll
+                for (int i = 0; i < UN; i++) {
+                    const int g = 4 * (tw + TS * i) + b4;
+                    if (4 * (tw + TS * i) >= NG) continue;
+                    const int l = tb.pos[4 * g + i4] >> 16;
+                    const double cf = invs * tb.isq[l];
+                    double D1[NA];
+#pragma unroll
+                    for (int u = 0; u < NA; u++) D1[u] = 0.0;
+#pragma unroll
+                    for (int k = 0; k < SP * NA; k++)
+#pragma unroll
+                        for (int u = 0; u < NA; u++) {
+                            double a = N % 4 == 0 || qi[k][u] >= 0 ? P[qi[k][u] + l] : 0.0;
+                            if (k == ws_ * NA + u) a *= dg;
+                            D1[u] = mfma4(a, cB[i][k], D1[u]);
+                        }
+                    double *ao = Aop + ((ws_ * NG + g) * NA) * 16 + 4 * k4 + i4;
+#pragma unroll
+                    for (int v = 0; v < NA; v++) {
+                        double D = 0.0;
+#pragma unroll
+                        for (int u = 0; u < NA; u++) D = mfma4(TA[v][u], D1[u], D);
+                        if (g < NG) ao[16 * v] = D * cf;
                     }
                 }
-                // Y = NnP (A, B), gY_z = NnPz (A, B), (gY_x, gY_y) = m NnP (Am, -Bm) and (Bm, Am)
-                const double u0 = S0a * A + S0b * B, u1 = S1a * A + S1b * B;
-                t0 += NnP * u0;
-                T1 += NnP * u1;
-                Vz += NnPz * u0;
-                if (m > 0) {
-                    const double NnPm = NnP * (double)m;
-                    Vx += NnPm * (S0a * Am + S0b * Bm);
-                    Vy += NnPm * (S0b * Am - S0a * Bm);
+            } else {
+                for (int un = w; un < NQ * ns; un += NW) {
+                    const int sr = un / NQ, t = un - sr * NQ, s = s0 + sr;
+                    const int g = min(4 * t + b4, NG - 1);
+                    const int pos = tb.pos[4 * g + i4] & 0xffff, l = tb.pos[4 * g + i4] >> 16;
+                    double D1[NA];
+#pragma unroll
+                    for (int u = 0; u < NA; u++) D1[u] = 0.0;
+                    for (int sj = 0; sj < S; sj++) {
+#pragma unroll
+                        for (int kk = 0; kk < NA; kk++) {
+                            const int aj = 4 * kk + k4, jb = sj * N + aj;
+                            const bool okj = N % 4 == 0 || aj < N;
+                            const double cb = okj && pos != 0xffff ? cg[jb * LM + pos] : 0.0;
+#pragma unroll
+                            for (int u = 0; u < NA; u++) {
+                                const int ai = 4 * u + i4, ia = s * N + ai;
+                                const int hi = max(ia, jb), lw = min(ia, jb);
+                                const int q = (hi * (hi + 1) / 2 + lw) * (L + 1) + l;
+                                double a = 0.0;
+                                if (okj && (N % 4 == 0 || ai < N)) {
+                                    a = p_lds ? P[q] : gg[q] - x[q] * dot;
+                                    if (ia == jb) a *= 1.4142135623730950488;
+                                }
+                                D1[u] = mfma4(a, cb, D1[u]);
+                            }
+                        }
+                    }
+                    double *ao = Aop + ((sr * NG + g) * NA) * 16 + 4 * k4 + i4;
+#pragma unroll
+                    for (int v = 0; v < NA; v++) {
+                        double D = 0.0;
+#pragma unroll
+                        for (int u = 0; u < NA; u++) D = mfma4(TA[v][u], D1[u], D);
+                        if (4 * t + b4 < NG) ao[16 * v] = D * (invs * tb.isq[l]);
+                    }
                 }
             }
-            T0 += t0;
-            T0L += (double)l * t0;
-            rs.step_scaled(l);
+            for (int c0 = 0; c0 < np; c0 += kSoapPass) {
+                const int nk = min(kSoapPass, np - c0);
+                if (!staged_first || np > kSoapPass) {   // a single pass of neighbours stays staged
+                    if (staged_first) block_lds_sync<NW>();
+                    if (w == NW - 1) {
+                        if (staged_first) {
+                            nb.load(p0 + c0, nk, nb_j, nb_r, nb_d);
+                            nb.species(nk, Z);
+                        }
+                        soap_stage<N, true>(sp, S, nb, p0 + c0, nk, tab, lo.slots, sb, sc, pair);
+                    }
+                    staged_first = true;
+                }
+                block_lds_sync<NW>();
+                if (s0 + SB >= S && c0 + kSoapPass >= np && desc + 1 < dn) {   // the next centre's data set out
+                    if (w == NW - 1) nb.load(pn, min(kSoapPass, nn), nb_j, nb_r, nb_d);
+                    if (AHEAD) load_xg(desc + 1);
+                    if (CAHEAD) load_c(desc + 1);
+                }
+                const int lt = fresh_lane(), k4 = lt >> 4, i4 = lt & 3;
+                SoapLane<N> rl;
+                rl.setup(tb.rt, k4);
+                int tile = 0;   // tiles are dealt to the wavefronts in turn
+                for (int sr = 0; sr < ns; sr++) {
+                    const int base = sb[s0 + sr], cnt = sc[s0 + sr];
+                    const double *as = Aop + sr * NG * NA * 16 + 4 * k4 + i4;
+                    for (int t = 0; t < cnt; t += 16, tile++) {
+                        if (NW > 1 && tile % NW != w) continue;
+                        const int off = t + (lane & 15);
+                        const int sl = base + min(off, cnt - 1);
+                        // an earlier descriptor's force on the pair (add), fetched before it is needed
+                        const double old = add && k4 < 3 ? pairF[3 * (size_t)pair[sl] + k4] : 0.0;
+                        const double ux = tab[kUx * lo.slots + sl], uy = tab[kUy * lo.slots + sl];
+                        const double uz = tab[kUz * lo.slots + sl];
+                        rl.radial(sp, k4, tab[kIxq * lo.slots + sl], tab[kE0 * lo.slots + sl], tab[kQ * lo.slots + sl],
+                                  tab[kQi * lo.slots + sl]);
+                        rl.z = uz;
+                        double ca[NA];   // 2 alpha r_a
+#pragma unroll
+                        for (int u = 0; u < NA; u++) ca[u] = (k4 + 4 * u) * sp.a2dr;
+                        const double ir = tab[kIr * lo.slots + sl];
+                        const double m2ar = -2.0 * sp.alpha * tab[kR * lo.slots + sl];
+                        double pA = 0.0, pA1 = 0.0, dA = 0.0, dA1 = 0.0, pB = 0.0, pB1 = 0.0, dB = 0.0, dB1 = 0.0;
+                        // per m: sums over l of S0 p, S1 p, S0 p' for the cos (a) and sin (b) harmonics
+                        double a0 = 0.0, a1 = 0.0, az = 0.0, b0 = 0.0, b1 = 0.0, bz = 0.0;
+                        double e0 = 0.0, e1 = 0.0, ez = 0.0, f0 = 0.0, f1 = 0.0, fz = 0.0;
+                        double h0 = 0.0, h1 = 0.0, i0 = 0.0, i1 = 0.0;
+#pragma unroll
+                        for (int l = 0; l <= L; l++) {
+                            double F[NA], Fd[NA];
+                            const double cl = fma((double)l, ir, m2ar);
+#pragma unroll
+                            for (int u = 0; u < NA; u++) {
+                                F[u] = rl.f(l, u);
+                                Fd[u] = fma(cl, F[u], ca[u] * rl.F1[u]);
+                            }
+                            double S0[6], S1[6];
+#pragma unroll
+                            for (int v = 0; v < lev_groups(l); v++) {
+                                S0[v] = S1[v] = 0.0;
+#pragma unroll
+                                for (int u = 0; u < NA; u++) {
+                                    const double a = as[((lev_base(l) + v) * NA + u) * 16];
+                                    S0[v] = mfma4(a, F[u], S0[v]);
+                                    S1[v] = mfma4(a, Fd[u], S1[v]);
+                                }
+                            }
+                            {
+                                const double p = rl.legendre(l, 0, rl.mA2, pA, pA1);
+                                double dp = 0.0;
+                                if (l == 1) dp = pA;
+                                if (l > 1) dp = pA + (uz * dA - leg_beta(l, rl.mA2) * dA1);
+                                pA1 = pA; pA = p;
+                                dA1 = dA; dA = dp;
+                                a0 += S0[0] * p; a1 += S1[0] * p; az += S0[0] * dp;
+                                if (l > 0) { b0 += S0[1] * p; b1 += S1[1] * p; bz += S0[1] * dp; }
+                            }
+                            if (l >= 4) {
+                                const double p = rl.legendre(l, 4, rl.mB2, pB, pB1);
+                                double dp = 0.0;
+                                if (l == 5) dp = pB;
+                                if (l > 5) dp = pB + (uz * dB - leg_beta(l, rl.mB2) * dB1);
+                                pB1 = pB; pB = p;
+                                dB1 = dB; dB = dp;
+                                constexpr int va = 2, vb = 3;
+                                e0 += S0[va] * p; e1 += S1[va] * p; ez += S0[va] * dp;
+                                f0 += S0[vb] * p; f1 += S1[vb] * p; fz += S0[vb] * dp;
+                            }
+                            if (l >= 8) { h0 = S0[4]; h1 = S1[4]; i0 = S0[5]; i1 = S1[5]; }
+                            if (l < L) rl.step(l);
+                            __builtin_amdgcn_sched_barrier(0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        }
+                        const double x2 = ux * ux - uy * uy, y2 = 2.0 * ux * uy;
+                        const double x3 = x2 * ux - y2 * uy, y3 = x2 * uy + y2 * ux;
+                        const double x4 = x2 * x2 - y2 * y2, y4 = 2.0 * x2 * y2;
+                        // (x + i y)^g and ^(g-1) (which meets the factor m = 0 in group 0)
+                        const double Aa = k4 == 0 ? 1.0 : k4 == 1 ? ux : k4 == 2 ? x2 : x3;
+                        const double Ba = k4 == 0 ? 0.0 : k4 == 1 ? uy : k4 == 2 ? y2 : y3;
+                        const double Am = k4 <= 1 ? 1.0 : k4 == 2 ? ux : x2;
+                        const double Bm = k4 <= 1 ? 0.0 : k4 == 2 ? uy : y2;
+                        const double m = (double)k4;
+                        double T0 = Aa * a0 + Ba * b0, T1 = Aa * a1 + Ba * b1, Vz = Aa * az + Ba * bz;
+                        double Vx = m * (a0 * Am + b0 * Bm), Vy = m * (b0 * Am - a0 * Bm);
+                        {
+                            const double Ab = Aa * x4 - Ba * y4, Bb = Aa * y4 + Ba * x4;
+                            const double An = Aa * x3 - Ba * y3, Bn = Aa * y3 + Ba * x3, mm = m + 4.0;
+                            T0 += Ab * e0 + Bb * f0;
+                            T1 += Ab * e1 + Bb * f1;
+                            Vz += Ab * ez + Bb * fz;
+                            Vx += mm * (e0 * An + f0 * Bn);
+                            Vy += mm * (f0 * An - e0 * Bn);
+                        }
+                        if constexpr (L >= 8) {   // group 0 only: the others' operands are zero
+                            const double A8 = x4 * x4 - y4 * y4, B8 = 2.0 * x4 * y4;
+                            const double A7 = x4 * x3 - y4 * y3, B7 = x4 * y3 + y4 * x3;
+                            T0 += A8 * h0 + B8 * i0;
+                            T1 += A8 * h1 + B8 * i1;
+                            Vx += 8.0 * (h0 * A7 + i0 * B7);
+                            Vy += 8.0 * (i0 * A7 - h0 * B7);
+                        }
+                        const double fc = tab[kFc * lo.slots + sl], dfc = tab[kDfc * lo.slots + sl];
+                        Vx *= fc; Vy *= fc; Vz *= fc;
+                        const double rad = (fc * T1 + dfc * T0) - (ux * Vx + uy * Vy + uz * Vz) * ir;
+                        // row c of the product: component c summed over the neighbour's four lanes
+                        double D = mfma4(i4 == 0 ? 1.0 : 0.0, rad * ux + Vx * ir, 0.0);
+                        D = mfma4(i4 == 1 ? 1.0 : 0.0, rad * uy + Vy * ir, D);
+                        D = mfma4(i4 == 2 ? 1.0 : 0.0, rad * uz + Vz * ir, D);
+                        if (k4 < 3 && off < cnt) pairF[3 * (size_t)pair[sl] + k4] = add ? old + D : D;
+                    }
+                }
+            }
         }
-        const double sY = (dfc - al2 * r * fc) * T0 + fc * ir * T0L + al2 * fc * dr * T1;
-        const double gx = fc * Vx, gy = fc * Vy, gz = fc * Vz;
-        const double a1 = sY - (ux * gx + uy * gy + uz * gz) * ir;
-        const double fx = a1 * ux + gx * ir, fy = a1 * uy + gy * ir, fz = a1 * uz + gz * ir;
-        pairF[3 * p] += fx;
-        pairF[3 * p + 1] += fy;
-        pairF[3 * p + 2] += fz;
+        if (np == 0 && desc + 1 < dn) {
+            if (w == NW - 1) nb.load(pn, min(kSoapPass, nn), nb_j, nb_r, nb_d);
+            if (AHEAD) load_xg(desc + 1);
+            if (CAHEAD) load_c(desc + 1);
+        }
+        if (desc + 1 < dn && w == NW - 1) nb.species(min(kSoapPass, nn), Z);
+        ci = cn;
+        cn = c2;
+        p0 = pn;
+        np = nn;
+        block_lds_sync<NW>();   // the table and the operands are free again
     }
 }
 
@@ -671,68 +991,61 @@ int soap_fast_supported(int n, int L) {
     return 0;
 }
 
-// Two centres per wave: single-species models with n <= 8, l <= 6 whose register
-// state fits without spilling (n l >= 32: 8/4, 6/6, 8/6).
-static constexpr bool fwd_pair_ok(int n, int L) { return n <= 8 && L <= 6 && n * L >= 32; }
-// Only the variants the launcher can pick are instantiated.
-template <int N, int L>
-static void fwd_go(bool preg, int cpw, int nblk, size_t sh, hipStream_t s, const SoapDev &sp, int nc,
-                   const int *centres, const int *Z, const int *nb_off, const int *nb_j, const double *nb_r,
-                   const double *nb_d, double *X, double *norm, double *cbuf) {
-    if constexpr (fwd_pair_ok(N, L)) {
-        if (cpw == 2) {
-            hipLaunchKernelGGL((k_soap_fwd_x<N, L, true, 2>), dim3(nblk), dim3(64), sh, s, sp, nc, centres, Z,
-                               nb_off, nb_j, nb_r, nb_d, X, norm, cbuf);
-            return;
-        }
-    }
-    if constexpr (N < 10 && L < 8) {
-        if (!preg) {
-            hipLaunchKernelGGL((k_soap_fwd_x<N, L, false, 1>), dim3(nblk), dim3(64), sh, s, sp, nc, centres, Z,
-                               nb_off, nb_j, nb_r, nb_d, X, norm, cbuf);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((k_soap_fwd_x<N, L, true, 1>), dim3(nblk), dim3(64), sh, s, sp, nc, centres, Z, nb_off,
-                       nb_j, nb_r, nb_d, X, norm, cbuf);
+// What a block may take: within it the power spectrum, c and dE/dp are kept in LDS where
+// they fit, so that at least two blocks share a CU; many species go through memory.
+constexpr int kSoapLdsCap = 60 * 1024;   // without the constant tables (at most 4 KB)
+
+struct FwdPlan {
+    bool split, p_lds, c_lds;
+    int nw;
+    size_t lds;
+};
+static size_t table_lds(const SoapDev &sp) {
+    const int nq4 = (soap_groups(sp.L) + 3) / 4 * 4;
+    return (size_t)(sp.n * sp.n + 24 + 4 * nq4 + sp.L + 1) * 8 + 4 * nq4 * 4;
+}
+static FwdPlan fwd_plan(const SoapDev &sp, bool split) {
+    FwdPlan f;
+    const int NA = (sp.n + 3) / 4;
+    f.split = split || sp.S > 1;
+    f.nw = sp.S > 1 ? 4 : split ? 2 : 1;
+    f.p_lds = f.c_lds = true;
+    if (FwdLds(NA, sp.L, sp.S, f.nw, sp.dim, true, true).total > kSoapLdsCap) f.p_lds = false;
+    if (FwdLds(NA, sp.L, sp.S, f.nw, sp.dim, f.p_lds, true).total > kSoapLdsCap) f.c_lds = false;
+    f.lds = FwdLds(NA, sp.L, sp.S, f.nw, sp.dim, f.p_lds, f.c_lds).total + table_lds(sp);
+    return f;
+}
+struct BwdPlan {
+    bool p_lds;
+    int nw, SB;
+    size_t lds;
+};
+static BwdPlan bwd_plan(const SoapDev &sp, bool split) {
+    BwdPlan b;
+    const int NA = (sp.n + 3) / 4;
+    b.nw = sp.S > 1 ? 4 : split ? 2 : 1;
+    b.p_lds = true;
+    b.SB = sp.S;
+    if (BwdLds(NA, sp.L, sp.S, sp.S, b.nw, sp.dim, true).total > kSoapLdsCap) b.p_lds = false;
+    while (b.SB > 1 && BwdLds(NA, sp.L, sp.S, b.SB, b.nw, sp.dim, b.p_lds).total > kSoapLdsCap) b.SB--;
+    b.lds = BwdLds(NA, sp.L, sp.S, b.SB, b.nw, sp.dim, b.p_lds).total + table_lds(sp);
+    return b;
 }
 
-// LDS bytes of the forward block: transform, radial grid, c' accumulators, the staged
-// neighbour chunk and (without registers for the Legendre levels) their LDS rows
-static size_t fwd_fast_lds(const SoapDev &sp, int cpw, bool preg) {
-    const int LM = (sp.L + 1) * (sp.L + 1), KLM = sp.K * LM, NB = kSoapChunk;
-    return (size_t)(sp.n * sp.n + 3 * sp.n + cpw * ((KLM + 1) & ~1) + cpw * (NB + 2) * (sp.n + 2 * sp.L + 1) +
-                    (preg ? 0 : 32 * cpw * ((2 * (sp.L + 2)) | 1))) * 8 +
-           (size_t)cpw * sp.S * (NB + 1) * 4;
-}
-
-// LDS bytes of the adjoint block, with its staging choice: whole = 2 stages the level
-// blocks P_l of all its centres, 1 dE/dp, 0 one level at a time; cpb centres per wave
-static size_t bwd_fast_lds(const SoapDev &sp, int *cpb_out, int *whole_out) {
-    const int LM = (sp.L + 1) * (sp.L + 1);
-    const int KLM = sp.K * LM, PR = (2 * (sp.L + 2)) | 1;
-    const size_t stg0 = std::max((size_t)sp.K * sp.K + (size_t)sp.K * (2 * sp.L + 1), (size_t)64 * PR);
-    const size_t pl = (size_t)(sp.L + 1) * (sp.K * sp.K + 2);
-    auto stg = [&](int cpb, int whole) {
-        return whole == 2 ? std::max(stg0, cpb * pl) : whole == 1 ? std::max(stg0, (size_t)cpb * sp.dim) : stg0;
-    };
-    auto need = [&](int cpb, int whole) {
-        return ((size_t)sp.n * sp.n + 3 * sp.n + (size_t)cpb * (KLM + 2) + stg(cpb, whole)) * 8;
-    };
-    const int whole = need(2, 2) <= 24 * 1024 ? 2 : need(2, 1) <= 24 * 1024 ? 1 : 0;
-    const int cpb = need(2, whole) <= 24 * 1024 ? 2 : 1;   // two centres per wave when LDS stays small
-    if (cpb_out) *cpb_out = cpb;
-    if (whole_out) *whole_out = whole;
-    return need(cpb, whole);
-}
-
+// What a model's descriptors are admitted by (the size a level-by-level adjoint with its
+// coefficients and one K x K level in LDS would take, and the variance's forward); the kernels
+// here stay within kSoapLdsCap and their tables for every shape admitted.
 size_t soap_fast_lds_bytes(const SoapDev &sp) {
     if (!soap_fast_supported(sp.n, sp.L)) return 0;
-    const int cpw = sp.S == 1 && fwd_pair_ok(sp.n, sp.L) ? 2 : 1;
-    size_t f = fwd_fast_lds(sp, cpw, true);
-    if (cpw == 1 && sp.n < 10 && sp.L < 8) f = std::max(f, fwd_fast_lds(sp, 1, false));
-    return std::max(f, bwd_fast_lds(sp, nullptr, nullptr));
+    const size_t KLM = (size_t)sp.K * (sp.L + 1) * (sp.L + 1), level = (size_t)sp.K * sp.K + (size_t)sp.K * (2 * sp.L + 1);
+    const size_t adjoint = sp.n * sp.n + 3 * sp.n + KLM + 2 + std::max(level, (size_t)64 * ((2 * (sp.L + 2)) | 1));
+    return std::max(soap_lane_lds_bytes(sp), adjoint * 8);
 }
+
+// Centres a block takes in turn: several once the launch has many more blocks than the GPU
+// holds (2048 to 3072 wavefronts), so that a centre's data arrive while the one before is
+// worked on (batch512 adjoint: 1.73 ms without, 0.63 ms with; the tables then in LDS).
+static int centres_per_block(int nc) { return nc >= 65536 ? 8 : nc >= 16384 ? 4 : 1; }
 
 bool launch_soap_fwd_fast(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
                           const int *nb_j, const double *nb_r, const double *nb_d, double *X, double *norm,
@@ -740,69 +1053,50 @@ bool launch_soap_fwd_fast(const SoapDev &sp, int nc, const int *centres, const i
     if (!soap_fast_supported(sp.n, sp.L)) return false;
     ensure_soap_constants();
     if (nc <= 0) return true;
-    const int LM = (sp.L + 1) * (sp.L + 1);
-    const int KLM = sp.K * LM;
-    // neighbour chunk of 32: covers a centre's neighbours within 5 A in one pass
-    // for covalent solids and keeps the block's LDS small
-    const int NB = kSoapChunk;
-    // Two centres per wave with the Legendre levels in registers for single-species
-    // models up to n 8, l 6 (measured on the 8/6 model: batch512 1.22 -> 1.11 ms,
-    // si4096 0.049 -> 0.043 ms); one centre per wave otherwise (the two-species 12/8
-    // model runs 3.4 ms with one and 5.6 ms with two, its LDS per wave doubling).
-    const int cpw = sp.S == 1 && fwd_pair_ok(sp.n, sp.L) ? 2 : 1;
-    const bool preg = cpw == 2 || sp.n >= 10 || sp.L >= 8 || nc < 16384;
-    const size_t sh = fwd_fast_lds(sp, cpw, preg);
-    (void)KLM; (void)NB;
-    const int nblk = (nc + cpw - 1) / cpw;
-#define LAUNCH(NN, LL)                                                                                          \
-    if (sp.n == NN && sp.L == LL) {                                                                             \
-        fwd_go<NN, LL>(preg, cpw, nblk, sh, s, sp, nc, centres, Z, nb_off, nb_j, nb_r, nb_d, X, norm, cbuf);     \
-        return true;                                                                                            \
+    // Two wavefronts per centre (m < 4, m >= 4) while a wavefront per centre would not fill the
+    // GPU (si4055: 44 -> 30 us), and where the accumulators of all groups (2 x 29 x 3 registers
+    // at 12/8) leave too few registers; one otherwise (no recursion is run twice).
+    const FwdPlan f = fwd_plan(sp, sp.n > 8 || sp.L > 6 || nc < 4096);
+    const int cpb = centres_per_block(nc), nblk = (nc + cpb - 1) / cpb;
+#define GO(NN, LL, NW, SPLIT, SP)                                                                                  \
+    hipLaunchKernelGGL((k_soap_fwd_x<NN, LL, NW, SPLIT, SP>), dim3(nblk), dim3(64 * NW), f.lds, s, sp, nc, cpb,    \
+                       centres, Z, nb_off, nb_j, nb_r, nb_d, X, norm, cbuf, (int)f.p_lds, (int)f.c_lds)
+#define LAUNCH(NN, LL)                                                                                             \
+    if (sp.n == NN && sp.L == LL) {                                                                                \
+        if (sp.S > 2 || !f.p_lds || !f.c_lds) GO(NN, LL, 4, true, 0);                                              \
+        else if (sp.S == 2) GO(NN, LL, 4, true, 2);                                                                \
+        else if (f.split) GO(NN, LL, 2, true, 1);                                                                  \
+        else if constexpr (NN <= 8 && LL <= 6) GO(NN, LL, 1, false, 1);                                            \
+        return true;                                                                                               \
     }
     SOAP_FAST(LAUNCH)
 #undef LAUNCH
+#undef GO
     return false;
-}
-#undef SOAP_FWD_LEVEL
-
-template <int N, int L>
-static void bwd_go(bool occ3, int nblk, size_t sh, hipStream_t s, const SoapDev &sp, int nc, int cpb,
-                   const int *centres, const int *Z, const int *nb_off, const int *nb_j, const double *nb_r,
-                   const double *nb_d, const double *X, const double *G, const double *norm, const double *cbuf,
-                   double *pairF, int whole) {
-    if constexpr (N <= 8) {
-        if (occ3) {
-            hipLaunchKernelGGL((k_soap_bwd_x<N, L, WPE_BWD + 1>), dim3(nblk), dim3(64), sh, s, sp, nc, cpb, centres,
-                               Z, nb_off, nb_j, nb_r, nb_d, X, G, norm, cbuf, pairF, whole);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((k_soap_bwd_x<N, L, WPE_BWD>), dim3(nblk), dim3(64), sh, s, sp, nc, cpb, centres, Z, nb_off,
-                       nb_j, nb_r, nb_d, X, G, norm, cbuf, pairF, whole);
 }
 
 bool launch_soap_bwd_fast(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
                           const int *nb_j, const double *nb_r, const double *nb_d, const double *X, const double *G,
-                          const double *norm, const double *cbuf, double *pairF, hipStream_t s) {
+                          const double *norm, const double *cbuf, double *pairF, bool add, hipStream_t s) {
     if (!soap_fast_supported(sp.n, sp.L)) return false;
     ensure_soap_constants();
     if (nc <= 0) return true;
-    // whole: all centres of the block staged at once (small descriptors): 2, the level blocks
-    // P_l (K x K each); 1, dE/dp; 0, one level at a time
-    int cpb = 1, whole = 0;
-    const size_t sh = bwd_fast_lds(sp, &cpb, &whole);
-    const int nblk = (nc + cpb - 1) / cpb;
-    // three wavefronts per SIMD for n <= 8 (161 VGPRs without spills) once the launch has
-    // at least four per SIMD to schedule
-    const bool occ3 = sp.n <= 8 && nblk >= 4 * 1024;
-#define LAUNCH(NN, LL)                                                                                          \
-    if (sp.n == NN && sp.L == LL) {                                                                             \
-        bwd_go<NN, LL>(occ3, nblk, sh, s, sp, nc, cpb, centres, Z, nb_off, nb_j, nb_r, nb_d, X, G, norm,   \
-                       cbuf, pairF, whole);                                                                     \
-        return true;                                                                                            \
+    const BwdPlan b = bwd_plan(sp, sp.n > 8 || sp.L > 6 || nc < 4096);
+    const int cpb = centres_per_block(nc), nblk = (nc + cpb - 1) / cpb;
+#define GO(NN, LL, NW, SP)                                                                                         \
+    hipLaunchKernelGGL((k_soap_bwd_x<NN, LL, NW, SP>), dim3(nblk), dim3(64 * NW), b.lds, s, sp, nc, cpb, centres,  \
+                       Z, nb_off, nb_j, nb_r, nb_d, X, G, norm, cbuf, pairF, (int)b.p_lds, b.SB, (int)add)
+#define LAUNCH(NN, LL)                                                                                             \
+    if (sp.n == NN && sp.L == LL) {                                                                                \
+        if (sp.S > 2 || !b.p_lds || b.SB < sp.S) GO(NN, LL, 4, 0);                                                 \
+        else if (sp.S == 2) GO(NN, LL, 4, 2);                                                                      \
+        else if (b.nw == 2) GO(NN, LL, 2, 1);                                                                      \
+        else if constexpr (NN <= 8 && LL <= 6) GO(NN, LL, 1, 1);                                                   \
+        return true;                                                                                               \
     }
     SOAP_FAST(LAUNCH)
 #undef LAUNCH
+#undef GO
     return false;
 }
 
