@@ -287,7 +287,7 @@ int gapx_model_set_autotune(gapx_model *model, int on);
  * times the fused GP kernel (descriptors up to 256 components) with 1, 2, 4 and 8
  * sparse-point parts and with the stream-K schedule (every block of a CU-filling grid
  * takes an equal run of (centre block, sparse chunk) units), or the split GEMMs (larger
- * descriptors) with 64 x 64 and 128 x 128 LDS tiles, and keeps the fastest.
+ * descriptors) with 64 x 64 and LDS tiles (128 x 128 or 256 x 256 by their number), and keeps the fastest.
  * gapx_model_tuning_split lists the choices: fused_parts (-1 the stream-K schedule,
  * 0 where the GEMMs are used), gemm1_lds / gemm2_lds (-1 where the fused
  * kernel is used) and the measured milliseconds of one launch (fused kernel with its

@@ -418,11 +418,12 @@ __global__ __launch_bounds__(256) void k_gemm2_split_lds(int nc, int d, int Mpad
 }
 
 // 128 x 128 tiles when they alone fill the GPU (two per CU); 64 x 64 tiles otherwise
-// (lds_mode: -1 this rule, 0 the 64 x 64 tiles, 1 the 128 x 128 tiles)
+// (lds_mode: -1 this rule, 0 the 64 x 64 tiles, 1 the LDS tiles)
 static bool use_lds_tiles(int rows, int cols, int lds_mode = -1) {
     if (lds_mode >= 0) return lds_mode == 1;
     return (long)cdivm(rows, kLT) * cdivm(cols, kLT) >= 512;
 }
+static bool use_big_tiles(int rows, int cols, int ldk, int per_round);
 
 
 // LDS rows of the fused split kernel: no padding; 16-byte vectors XOR-swizzled, vector c
@@ -922,11 +923,265 @@ __global__ void k_sum_parts_f32(size_t n, int parts, const float *P, double inv_
     G[i] = s * inv_wscale;
 }
 
+
+// ---------------------------------------------------------------------------
+// The same GEMMs on 256 x 256 block tiles: 8 wavefronts of 128 x 64 (8 x 4 MFMA tiles),
+// k steps of 32.  A step's slices (256 rows of A and of B, hi and lo, 64 KB) stream into one
+// of two LDS buffers by buffer loads while the other is used, with one wait and one
+// barrier per step and no registers held for the prefetch.  Against the 128 x 128 tiles
+// (staged through registers, two barriers a step) each staged byte feeds twice the MFMAs
+// and each LDS fragment read 4/3 as many.  16384 centres x 2000 points x 2701 components: GEMM 1
+// 626 -> 444 us and GEMM 2 668 -> 486 us, 1196 and 1093 TFLOP/s executed, what a large bf16
+// product reaches on this card (1152); the same loop on a quarter of the CUs runs 16% faster
+// per tile, and starting each step on fewer fragments changes nothing, so the rest is the
+// card's clock under load.  16-byte vector c of a 32-element row r sits at c ^ (r / 2 % 4), so that
+// the 8 rows a group of lanes reads fall on distinct 16-byte bank groups.  An element's MFMA
+// passes run in the same order as in the smaller tiles: results are bitwise the same.
+// Rows past the matrix are clamped to its last one (their results are not written).
+// ---------------------------------------------------------------------------
+constexpr int kBT = 256;                   // tile edge
+constexpr int kBSlice = kBT * 32;          // elements of one staged slice
+constexpr unsigned kBBytes = 1u << 31;     // tile rows x leading dimension stay below it
+
+template <int PREC>
+struct BigTile {
+    typedef Half<PREC> H;
+    typedef typename H::T T;
+    typedef typename H::V V;
+    __amdgpu_buffer_rsrc_t ah, al, bh, bl;
+    unsigned ao[2], bo[2];   // byte offsets of this lane's vectors of the wavefront's two loads per slice
+    int wv, ra, rb;          // wavefront; this lane's fragment places in the A and B slices
+
+    __device__ __forceinline__ void init(const T *Ahi, const T *Alo, const T *Bhi, const T *Blo, int ldk, int m0,
+                                         int amax, int n0, int bmax) {
+        const int t = threadIdx.x, lane = t & 63;
+        wv = __builtin_amdgcn_readfirstlane(t >> 6);
+        const int arows = min(kBT, amax - m0), brows = min(kBT, bmax - n0);
+        ah = mat_rsrc(Ahi + (size_t)m0 * ldk, (unsigned)arows * ldk * 2);
+        al = mat_rsrc(Alo + (size_t)m0 * ldk, (unsigned)arows * ldk * 2);
+        bh = mat_rsrc(Bhi + (size_t)n0 * ldk, (unsigned)brows * ldk * 2);
+        bl = mat_rsrc(Blo + (size_t)n0 * ldk, (unsigned)brows * ldk * 2);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int row = 16 * (wv + 8 * i) + (lane >> 2), c = (lane & 3) ^ ((row >> 1) & 3);
+            ao[i] = (unsigned)((min(row, arows - 1) * ldk + 8 * c) * 2);
+            bo[i] = (unsigned)((min(row, brows - 1) * ldk + 8 * c) * 2);
+        }
+        const int r16 = lane & 15, c = (lane >> 4) ^ ((r16 >> 1) & 3);
+        ra = ((wv >> 2) * 128 + r16) * 32 + 8 * c;
+        rb = ((wv & 3) * 64 + r16) * 32 + 8 * c;
+    }
+    // the slices of k step k0 into a buffer [A hi, A lo, B hi, B lo]
+    __device__ __forceinline__ void stage(int k0, T *buf) const {
+        const unsigned so = (unsigned)k0 * 2;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            T *d = buf + 512 * (wv + 8 * i);
+            dma16(ah, ao[i], so, d);
+            dma16(al, ao[i], so, d + kBSlice);
+            dma16(bh, bo[i], so, d + 2 * kBSlice);
+            dma16(bl, bo[i], so, d + 3 * kBSlice);
+        }
+    }
+    __device__ __forceinline__ void step(int knext, int ldk, const T *__restrict__ cur, T *__restrict__ next,
+                                         float4_t (&acc)[8][4]) const {
+        if (knext < ldk) stage(knext, next);
+        V fbh[4], fbl[4], fah, fal, nah, nal;
+        fah = *(const V *)(cur + ra);
+        fal = *(const V *)(cur + kBSlice + ra);
+        fbh[0] = *(const V *)(cur + 2 * kBSlice + rb);
+        fbl[0] = *(const V *)(cur + 3 * kBSlice + rb);
+        // every wavefront leaves the barrier at once and LDS serves them in turn: the first row
+        // tile starts on its first column tile's fragments, each next one's read before it
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j < 3) {
+                fbh[j + 1] = *(const V *)(cur + 2 * kBSlice + rb + 512 * (j + 1));
+                fbl[j + 1] = *(const V *)(cur + 3 * kBSlice + rb + 512 * (j + 1));
+            } else {
+                nah = *(const V *)(cur + ra + 512);
+                nal = *(const V *)(cur + kBSlice + ra + 512);
+            }
+            acc[0][j] = H::mfma(fal, fbh[j], acc[0][j]);
+            acc[0][j] = H::mfma(fah, fbl[j], acc[0][j]);
+            acc[0][j] = H::mfma(fah, fbh[j], acc[0][j]);
+            if (j == 0) __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 1; i < 8; i++) {
+            fah = nah;
+            fal = nal;
+            if (i < 7) {
+                nah = *(const V *)(cur + ra + 512 * (i + 1));
+                nal = *(const V *)(cur + kBSlice + ra + 512 * (i + 1));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = H::mfma(fal, fbh[j], acc[i][j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = H::mfma(fah, fbl[j], acc[i][j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = H::mfma(fah, fbh[j], acc[i][j]);
+            if (i < 7) {   // the next row tile's reads before this one's MFMAs
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 12, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0);   // this wavefront's loads into the next buffer have landed
+        __syncthreads();
+    }
+    __device__ __forceinline__ void run(int ldk, T *buf0, T *buf1, float4_t (&acc)[8][4]) const {
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
+        stage(0, buf0);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        for (int k0 = 0; k0 < ldk; k0 += 64) {
+            step(k0 + 32, ldk, buf0, buf1, acc);
+            if (k0 + 32 < ldk) step(k0 + 64, ldk, buf1, buf0, acc);
+        }
+    }
+};
+
+__device__ __forceinline__ unsigned dpp_xor1(unsigned x) { return (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xf, 0xf, true); }
+__device__ __forceinline__ unsigned dpp_xor2(unsigned x) { return (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xf, 0xf, true); }
+
+// K = X Xs^T with the epilogue of k_gemm1_split (e_part has one column per tile column)
+template <int PREC, bool INTZ>
+__global__ __launch_bounds__(512) void k_gemm1_split_big(int nc, int M, int dpad, int Mpad, int ntn,
+                                                          const typename Half<PREC>::T *Xhi,
+                                                          const typename Half<PREC>::T *Xlo,
+                                                          const typename Half<PREC>::T *Shi,
+                                                          const typename Half<PREC>::T *Slo, const double *wvec,
+                                                          double zeta, int izeta, double wscale,
+                                                          typename Half<PREC>::T *Whi, typename Half<PREC>::T *Wlo,
+                                                          double *e_part) {
+    typedef Half<PREC> H;
+    typedef typename H::T T;
+    __shared__ __attribute__((aligned(16))) T buf0[4 * kBSlice], buf1[4 * kBSlice];
+    __shared__ double red[4][kBT];
+    int tm, tn;
+    lds_tile_coords(ntn, tm, tn);
+    const int m0 = tm * kBT, n0 = tn * kBT;
+    float4_t acc[8][4];
+    BigTile<PREC> bt;
+    bt.init(Xhi, Xlo, Shi, Slo, dpad, m0, nc, n0, M);
+    bt.run(dpad, buf0, buf1, acc);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3, c = lane & 3;
+    double wv[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int col = n0 + wn * 64 + j * 16 + (lane & 15);
+        wv[j] = col < M ? wvec[col] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        double rowsum[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            unsigned p[4];   // (hi, lo) of W at rows 4 (lane/16) + v, this lane's column
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const double kv = (double)acc[i][j][v];
+                double kz1, kz;
+                if constexpr (INTZ) {
+                    kz1 = 1.0;
+                    for (int q = 1; q < izeta; q++) kz1 *= kv;
+                    kz = kz1 * kv;
+                } else {
+                    kz1 = pow(kv, zeta - 1.0);
+                    kz = pow(kv, zeta);
+                }
+                rowsum[v] += wv[j] * kz;
+                const double wk = n0 + wn * 64 + j * 16 + (lane & 15) < M ? wv[j] * zeta * kz1 * wscale : 0.0;
+                const T h = H::from(wk), l = H::from(wk - H::to(h));
+                p[v] = (unsigned)__builtin_bit_cast(unsigned short, h) | (unsigned)__builtin_bit_cast(unsigned short, l) << 16;
+            }
+            // 4 x 4 transpose within the quad: lane c gets row 4 (lane/16) + c of the quad's four columns
+            const bool odd = c & 1, hi2 = c & 2;
+            const unsigned a0 = odd ? p[1] : p[0], b0 = odd ? p[3] : p[2];
+            const unsigned a1 = dpp_xor1(odd ? p[0] : p[1]), b1 = dpp_xor1(odd ? p[2] : p[3]);
+            const unsigned x0 = odd ? a1 : a0, x1 = odd ? a0 : a1, y0 = odd ? b1 : b0, y1 = odd ? b0 : b1;
+            const unsigned r0 = dpp_xor2(hi2 ? x0 : y0), r1 = dpp_xor2(hi2 ? x1 : y1);
+            const unsigned q0 = hi2 ? r0 : x0, q1 = hi2 ? r1 : x1, q2 = hi2 ? y0 : r0, q3 = hi2 ? y1 : r1;
+            const int row = m0 + wm * 128 + i * 16 + 4 * (lane >> 4) + c;
+            const int col = n0 + wn * 64 + j * 16 + 4 * ((lane >> 2) & 3);
+            if (row < nc && col < Mpad) {
+                uint2 vh, vl;
+                vh.x = (q0 & 0xffffu) | q1 << 16; vh.y = (q2 & 0xffffu) | q3 << 16;
+                vl.x = q0 >> 16 | (q1 & 0xffff0000u); vl.y = q2 >> 16 | (q3 & 0xffff0000u);
+                *(uint2 *)(Whi + (size_t)row * Mpad + col) = vh;
+                *(uint2 *)(Wlo + (size_t)row * Mpad + col) = vl;
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            double x = rowsum[v];
+            for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+            if ((lane & 15) == 0) red[wn][wm * 128 + i * 16 + 4 * (lane >> 4) + v] = x;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < kBT) {
+        const int row = m0 + threadIdx.x;
+        if (row < nc)
+            e_part[(size_t)row * ntn + tn] = (red[0][threadIdx.x] + red[1][threadIdx.x]) +
+                                             (red[2][threadIdx.x] + red[3][threadIdx.x]);
+    }
+}
+
+// G = W Xs (FP64 output, unscaled)
+template <int PREC>
+__global__ __launch_bounds__(512) void k_gemm2_split_big(int nc, int d, int Mpad, int ntn,
+                                                          const typename Half<PREC>::T *Whi,
+                                                          const typename Half<PREC>::T *Wlo,
+                                                          const typename Half<PREC>::T *Thi,
+                                                          const typename Half<PREC>::T *Tlo, double inv_wscale,
+                                                          double *G) {
+    typedef typename Half<PREC>::T T;
+    __shared__ __attribute__((aligned(16))) T buf0[4 * kBSlice], buf1[4 * kBSlice];
+    int tm, tn;
+    lds_tile_coords(ntn, tm, tn);
+    const int m0 = tm * kBT, n0 = tn * kBT;
+    float4_t acc[8][4];
+    BigTile<PREC> bt;
+    bt.init(Whi, Wlo, Thi, Tlo, Mpad, m0, nc, n0, d);
+    bt.run(Mpad, buf0, buf1, acc);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int row = m0 + wm * 128 + i * 16 + 4 * (lane >> 4) + v;
+            if (row >= nc) continue;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int col = n0 + wn * 64 + j * 16 + (lane & 15);
+                if (col < d) G[(size_t)row * d + col] = (double)acc[i][j][v] * inv_wscale;
+            }
+        }
+}
+
 static int int_zeta_m(double z) {
     double r = floor(z + 0.5);
     return (fabs(z - r) == 0.0 && r >= 1.0 && r <= 16.0) ? (int)r : 0;
 }
 
+
+// 256 x 256 tiles (one block per CU, rounds of 256) against the 128 x 128 ones, whose time
+// grows with their number: 600 (GEMM 1) or 430 (GEMM 2) of those take as long as a round.
+// Measured at 2720 and 2016 k: GEMM 1 256 tiles 193-210 us a full round (167 us from 64 tiles on),
+// 128 tiles 102-124 (256 of them), 152-164 (512), 228-270 (720), 298-319 us (1008); GEMM 2
+// 119-155 (132 tiles), 129-152 (253) against 156-170 (528), 220-230 us (990).
+static bool use_big_tiles(int rows, int cols, int ldk, int per_round) {
+    const long big = (long)cdivm(rows, kBT) * cdivm(cols, kBT), small = (long)cdivm(rows, kLT) * cdivm(cols, kLT);
+    return small >= per_round * ((big + 255) / 256) && (size_t)kBT * ldk * 2 < kBBytes;
+}
 
 void launch_gemm1_split(int prec, int nc, int M, int d, int dpad, int lds_mode, const double *X, const void *Xs_hi,
                         const void *Xs_lo, const double *wvec, double zeta, double wscale, float *Wf,
@@ -934,7 +1189,9 @@ void launch_gemm1_split(int prec, int nc, int M, int d, int dpad, int lds_mode, 
     const int Mpad = (M + 31) / 32 * 32;
     dim3 grid(cdivm(nc, 64), cdivm(M, 64));
     const bool lds = use_lds_tiles(nc, M, lds_mode);
-    const int ntn = cdivm(M, kLT), nblk = cdivm(nc, kLT) * ntn;
+    const bool big = lds && use_big_tiles(nc, M, dpad, 600);
+    const int edge = big ? kBT : kLT;
+    const int ntn = cdivm(M, edge), nblk = cdivm(nc, edge) * ntn;
     *ntile_out = lds ? ntn : (int)grid.y;
     if (nc <= 0) return;
     const size_t xsz = (size_t)((nc + 63) / 64 * 64) * dpad;
@@ -944,6 +1201,16 @@ void launch_gemm1_split(int prec, int nc, int M, int d, int dpad, int lds_mode, 
     char *wf = (char *)Wf;
     void *Whi = wf, *Wlo = wf + (size_t)nc * Mpad * 2;
     const int iz = int_zeta_m(zeta);
+#define G1B(P, T, IZ)                                                                                            \
+    hipLaunchKernelGGL((k_gemm1_split_big<P, IZ>), dim3(nblk), dim3(512), 0, s, nc, M, dpad, Mpad, ntn,          \
+                       (const T *)Xhi, (const T *)Xlo, (const T *)Xs_hi, (const T *)Xs_lo, wvec, zeta, iz, wscale, \
+                       (T *)Whi, (T *)Wlo, e_part)
+    if (big) {
+        if (prec == 1) { if (iz > 0) G1B(1, __bf16, true); else G1B(1, __bf16, false); }
+        else { if (iz > 0) G1B(2, _Float16, true); else G1B(2, _Float16, false); }
+        return;
+    }
+#undef G1B
 #define G1L(P, T, IZ)                                                                                            \
     hipLaunchKernelGGL((k_gemm1_split_lds<P, IZ>), dim3(nblk), dim3(256), 0, s, nc, M, dpad, Mpad, ntn,          \
                        (const T *)Xhi, (const T *)Xlo, (const T *)Xs_hi, (const T *)Xs_lo, wvec, zeta, iz, wscale, \
@@ -1087,6 +1354,18 @@ void launch_gemm2_split(int prec, int nc, int M, int d, int dpad, int Mpad, int 
     const char *wf = (const char *)Wf;
     const void *Whi = wf, *Wlo = wf + (size_t)nc * Mpad * 2;
     const double inv = 1.0 / wscale;
+    if (use_lds_tiles(nc, d, lds_mode) && use_big_tiles(nc, d, Mpad, 430)) {
+        const int ntn = cdivm(d, kBT), nblk = cdivm(nc, kBT) * ntn;
+        if (prec == 1)
+            hipLaunchKernelGGL(k_gemm2_split_big<1>, dim3(nblk), dim3(512), 0, s, nc, d, Mpad, ntn,
+                               (const __bf16 *)Whi, (const __bf16 *)Wlo, (const __bf16 *)XsT_hi,
+                               (const __bf16 *)XsT_lo, inv, G);
+        else
+            hipLaunchKernelGGL(k_gemm2_split_big<2>, dim3(nblk), dim3(512), 0, s, nc, d, Mpad, ntn,
+                               (const _Float16 *)Whi, (const _Float16 *)Wlo, (const _Float16 *)XsT_hi,
+                               (const _Float16 *)XsT_lo, inv, G);
+        return;
+    }
     if (use_lds_tiles(nc, d, lds_mode)) {
         const int ntn = cdivm(d, kLT), nblk = cdivm(nc, kLT) * ntn;
         if (prec == 1)
