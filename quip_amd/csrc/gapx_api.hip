@@ -1916,7 +1916,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
                                     w.e_part.as<double>(), &ntile, s);
             } else if (m->precision == GAPX_PREC_FP64) {
                 launch_gemm1_f64(tu.g1, nc, c.M, c.dim, w.X.as<double>(), c.d_Xs.as<double>(), c.d_w.as<double>(),
-                                 c.zeta, w.W.as<double>(), w.e_part.as<double>(), &ntile, s);
+                                 c.zeta, grad ? w.W.as<double>() : nullptr, w.e_part.as<double>(), &ntile, s);
             } else if (fused[k]) {   // split forms: K -> W -> G in one kernel
                 launch_gp_fused_split(m->precision, nc, c.M, c.dim, c.dpad, c.Mpad, tu.fparts, w.X.as<double>(),
                                       c.d_Xs_hi.p, c.d_Xs_lo.p, c.d_w.as<double>(), c.zeta, c.wscale,
@@ -2160,7 +2160,7 @@ int gapx::calc_host(gapx_model *m, Engine &eg, int S, const int *atom_off, const
         HIPCHK(hipMemcpyAsync(w.pos.p, h, bpos, hipMemcpyHostToDevice, s));
     }
     CHK(eval_batch(m, eg, S, atom_off, w.pos.as<double>(), pos, Z, lats, pbcs, nl_cutoff,
-                   want | GAPX_WANT_E | GAPX_WANT_V | GAPX_WANT_F | GAPX_WANT_LOCAL_E | GAPX_WANT_LOCAL_V,
+                   want | GAPX_WANT_E | GAPX_WANT_LOCAL_E,   // no gradient unless one of its outputs is asked for
                    w.e.as<double>(), w.le.as<double>(), w.f.as<double>(), w.vir.as<double>(), w.lv.as<double>(),
                    ext, opt ? &o2 : nullptr));
     CHK(resolve_pending(m, eg));   // a speculative call that overflowed is redone before its results are read

@@ -1600,6 +1600,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GBK == 16 ?
     const int wm = w >> 1, wn = w & 1;
     const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
     const int kbeg = blockIdx.z * kchunk, kend = min(Kd, kbeg + kchunk);
+    const bool store = C != nullptr;   // energies alone need no W (17553 x 2000: 281 MB)
     C += (size_t)blockIdx.z * Mr * Nc;
     double4_t acc[WM][WN];
 #pragma unroll
@@ -1691,7 +1692,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GBK == 16 ?
                     rowsum[i][v] += wv * kz;
                     kv = wv * zeta * kz1;
                 }
-                if (row < Mr && col < Nc) C[(size_t)row * Nc + col] = kv;
+                if ((!EPI || store) && row < Mr && col < Nc) C[(size_t)row * Nc + col] = kv;
             }
         }
     if (EPI) {
