@@ -496,6 +496,8 @@ static int model_upload(gapx_model *m) {
         Coord *c = cp.get();
         std::vector<double> w(c->M);
         for (int s = 0; s < c->M; s++) w[s] = c->alpha[s] * c->delta * c->delta * c->scut[s];
+        // the FP64 products read pairs of columns: the last pair of an odd row ends past the matrix
+        CHK(c->d_Xs.ensure(c->Xs.size() * 8 + 16));
         CHK(upload(c->d_Xs, c->Xs.data(), c->Xs.size() * 8));
         CHK(upload(c->d_w, w.data(), w.size() * 8));
         if (c->kind == 1) {
@@ -1295,8 +1297,8 @@ int gapx::check_batch(int S, const int *atom_off, const int *Z, const double *la
 // first evaluation times every GEMM 1 tile and every GEMM 2 tile x split-K factor
 // (fastest of three launches after a warm-up) with HIP events on the engine's stream, on the
 // call's own operands (X is already computed), and keeps the fastest.  Later
-// calls in the bucket reuse the choice.  Without autotuning: GEMM 1 (4,2),
-// GEMM 2 (2,2) with the default split-K factor.
+// calls in the bucket reuse the choice.  Without autotuning: 64 x 64 tiles,
+// GEMM 2 with the default split-K factor.
 static int gemm_tune(gapx_model *m, Engine &eg, Coord &c, int nc, GemmTune &out, bool cached_only = false) {
     out = GemmTune();
     out.parts = gemm2_parts(nc, c.dim);
@@ -1947,14 +1949,12 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
             if (want_var) {   // FP64 whatever the GEMM precision
                 launch_gemm_nt_f64(nc, c.M, c.dim, w.X.as<double>(), c.d_Xs.as<double>(), w.vK.as<double>(), s);
                 launch_var_cov(nc, c.M, w.vK.as<double>(), d2, c.zeta, w.vk.as<double>(), s);
-                launch_gemm2_f64(1, 1, nc, c.M, c.M, w.vk.as<double>(), c.d_Cinv.as<double>(), w.vV.as<double>(),
-                                 nullptr, s);
+                launch_gemm_nn_f64(nc, c.M, c.M, w.vk.as<double>(), c.d_Cinv.as<double>(), w.vV.as<double>(), s);
                 launch_var_rows(nc, c.M, c.dim, w.X.as<double>(), w.vK.as<double>(), w.vk.as<double>(),
                                 w.vV.as<double>(), d2, c.zeta, centres, w.var_inst[k].as<double>(),
                                 w.varsite.as<double>(), s);
                 if (want_vgrad) {
-                    launch_gemm2_f64(1, 1, nc, c.M, c.dim, w.vV.as<double>(), c.d_Xs.as<double>(), w.Gv.as<double>(),
-                                     nullptr, s);
+                    launch_gemm_nn_f64(nc, c.M, c.dim, w.vV.as<double>(), c.d_Xs.as<double>(), w.Gv.as<double>(), s);
                     launch_var_self_grad(nc, c.dim, w.X.as<double>(), d2, c.zeta, w.Gv.as<double>(), s);
                     launch_soap_bwd(sp, nc, centres, w.Z.as<int>(), w.nb_off.as<int>(), w.nb_j.as<int>(),
                                     w.nb_r.as<double>(), w.nb_d.as<double>(), w.X.as<double>(), w.Gv.as<double>(),

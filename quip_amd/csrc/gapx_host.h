@@ -108,7 +108,7 @@ struct DBuf {
 // model
 // ---------------------------------------------------------------------------
 struct GemmTune {
-    int g1 = 0, g2 = 1, parts = 1;   // GEMM 1 tile, GEMM 2 tile, GEMM 2 split-K factor
+    int g1 = 2, g2 = 2, parts = 1;   // GEMM 1 tile, GEMM 2 tile, GEMM 2 split-K factor
     float g1_ms = 0, g2_ms = 0;      // measured times of the chosen configurations
     // split forms: sparse-point parts of the fused kernel (0 = its default rule), and the
     // split GEMMs' tiles (-1 = the default rule, 0 = 64 x 64, 1 = 128 x 128 LDS tiles)

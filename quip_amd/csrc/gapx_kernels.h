@@ -132,11 +132,17 @@ void launch_soap_bwd(const SoapDev &sp, int nc, const int *centres, const int *Z
                      const double *norm, const double *cbuf, double *pairF, bool add, hipStream_t s);
 
 // GEMMs
-// Tile configuration `cfg` in [0, kGemmTiles): (WM, WN, k tile) = (4,2,16), (2,2,16),
-// (2,4,16), (4,2,32), (2,2,32), (2,4,32); block tile (32 WM) x (32 WN) of 4 wavefronts.
-constexpr int kGemmTiles = 6;
+// Tile configuration `cfg` in [0, kGemmTiles): 128 x 128, 64 x 128, 64 x 64 (gapx_gemm64.hip); a product
+// whose byte offsets pass 31 bits (gemm_stream_ok) and those of the GAP variance, whose digits
+// depend on the order of summation, run on 64 x 64 tiles staged through registers.
+constexpr int kGemmTiles = 3;
+bool gemm_stream_ok(int M, int d);
+int gemm_stream_ntile(int cfg, int M);
+void launch_gemm1_f64_stream(int cfg, int nc, int M, int d, const double *X, const double *Xs, const double *wvec,
+                             double zeta, double *W, double *e_part, hipStream_t s);
+void launch_gemm2_f64_stream(int cfg, int parts, int nc, int M, int d, const double *W, const double *Xs, double *out,
+                             hipStream_t s);
 // gemm1: K = X (nc x d) . Xs^T (M x d); W = w_s zeta K^(zeta-1) (not stored if W is null); e_part[i*ntile + t]
-int gemm1_ntile(int cfg, int M);
 void launch_gemm1_f64(int cfg, int nc, int M, int d, const double *X, const double *Xs, const double *wvec,
                       double zeta, double *W, double *e_part, int *ntile_out, hipStream_t s);
 // gemm2: G = W (nc x M) . Xs (M x d); with parts > 1 the k range is split and the
@@ -205,7 +211,8 @@ void launch_d2b(int N, const int *Z, int Z1, int Z2, double rc, double ctw, int 
 void launch_sum_fixed(size_t n, const double *v, double *out, hipStream_t s);
 
 // GAP variance (projected-process estimate), FP64.
-// C = A (rows x kd) . B^T (cols x kd), no epilogue
+// C = A (rows x kd) . B^T (cols x kd), and C = A (rows x kd) . B (kd x cols), no epilogue
+void launch_gemm_nn_f64(int rows, int kd, int cols, const double *A, const double *B, double *C, hipStream_t s);
 void launch_gemm_nt_f64(int rows, int cols, int kd, const double *A, const double *B, double *C, hipStream_t s);
 // kv[i][s] = delta2 K[i][s]^zeta
 void launch_var_cov(int nc, int M, const double *K, double delta2, double zeta, double *kv, hipStream_t s);

@@ -1578,18 +1578,19 @@ constexpr int GPAD = 1;   // odd: the 16 k-rows one stash write touches fall on 
 
 // C = A . B (+ fused GP epilogue).  A is row-major (rows x K, k contiguous);
 // B is row-major (cols x K) when BT, else (K x cols).  4 wavefronts in a 2x2
-// grid, each owning (16 WM) x (16 WN) outputs, block tile (32 WM) x (32 WN).
+// grid, each owning 32 x 32 outputs, block tile 64 x 64, k tiles of 16.
 // The next k tile is fetched into registers while the current one feeds the
 // MFMAs from LDS.  blockIdx.z selects a k range (split-K) whose partial result
-// goes to C + z * rows * cols.
+// goes to C + z * rows * cols.  For the GAP variance, whose digits depend on this order of
+// summation, and for products whose byte offsets pass 31 bits; gapx_gemm64.hip otherwise.
 // The occupancy hint keeps the accumulators in ordinary VGPRs for the whole kernel:
 // without it the compiler places them in AGPRs and copies all of them out and back
 // around every k tile.
-template <bool BT, bool EPI, int WM, int WN, int GBK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GBK == 16 ? 3 : 2))) void k_gemm_f64(int Mr, int Nc, int Kd, int kchunk, const double *__restrict__ A,
-                                                  const double *__restrict__ B, double *__restrict__ C,
-                                                  const double *__restrict__ wvec, double zeta, int izeta,
-                                                  double *__restrict__ e_part) {
+template <bool BT, bool EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_gemm_f64(
+    int Mr, int Nc, int Kd, int kchunk, const double *__restrict__ A, const double *__restrict__ B,
+    double *__restrict__ C, const double *__restrict__ wvec, double zeta, int izeta, double *__restrict__ e_part) {
+    constexpr int WM = 2, WN = 2, GBK = 16;
     constexpr int BM = 32 * WM, BN = 32 * WN;
     constexpr int AL = BM * GBK / 256;   // A elements per thread per k tile
     constexpr int BL = BN * GBK / 256;
@@ -1722,32 +1723,17 @@ static int int_zeta(double z) {
     return (fabs(z - r) == 0.0 && r >= 1.0 && r <= 16.0) ? (int)r : 0;
 }
 
-// Tile shapes the autotuner chooses between: (WM, WN, k tile) per block of 4
-// wavefronts, block tile (32 WM) x (32 WN).
-static const int kTiles[kGemmTiles][3] = {{4, 2, 16}, {2, 2, 16}, {2, 4, 16}, {4, 2, 32}, {2, 2, 32}, {2, 4, 32}};
-
-int gemm1_ntile(int cfg, int M) { return cdiv(M, 32 * kTiles[cfg][1]); }
-
-template <int WM, int WN, int BK>
-static void gemm1_go(int nc, int M, int d, const double *X, const double *Xs, const double *wvec, double zeta,
-                     double *W, double *e_part, hipStream_t s) {
-    dim3 grid(cdiv(nc, 32 * WM), cdiv(M, 32 * WN), 1);
-    hipLaunchKernelGGL((k_gemm_f64<true, true, WM, WN, BK>), grid, dim3(256), 0, s, nc, M, d, d, X, Xs, W, wvec,
-                       zeta, int_zeta(zeta), e_part);
-}
-
 void launch_gemm1_f64(int cfg, int nc, int M, int d, const double *X, const double *Xs, const double *wvec,
                       double zeta, double *W, double *e_part, int *ntile_out, hipStream_t s) {
-    *ntile_out = gemm1_ntile(cfg, M);
+    const bool stream = gemm_stream_ok(M, d);
+    *ntile_out = stream ? gemm_stream_ntile(cfg, M) : cdiv(M, 64);
     if (nc <= 0) return;
-    switch (cfg) {
-        case 0: gemm1_go<4, 2, 16>(nc, M, d, X, Xs, wvec, zeta, W, e_part, s); break;
-        case 1: gemm1_go<2, 2, 16>(nc, M, d, X, Xs, wvec, zeta, W, e_part, s); break;
-        case 2: gemm1_go<2, 4, 16>(nc, M, d, X, Xs, wvec, zeta, W, e_part, s); break;
-        case 3: gemm1_go<4, 2, 32>(nc, M, d, X, Xs, wvec, zeta, W, e_part, s); break;
-        case 4: gemm1_go<2, 2, 32>(nc, M, d, X, Xs, wvec, zeta, W, e_part, s); break;
-        default: gemm1_go<2, 4, 32>(nc, M, d, X, Xs, wvec, zeta, W, e_part, s); break;
+    if (stream) {
+        launch_gemm1_f64_stream(cfg, nc, M, d, X, Xs, wvec, zeta, W, e_part, s);
+        return;
     }
+    hipLaunchKernelGGL((k_gemm_f64<true, true>), dim3(cdiv(nc, 64), cdiv(M, 64)), dim3(256), 0, s, nc, M, d, d, X, Xs, W,
+                       wvec, zeta, int_zeta(zeta), e_part);
 }
 
 // split-K partial sums, reduced in a fixed order
@@ -1767,26 +1753,16 @@ int gemm2_parts(int nc, int d) {
     return parts;
 }
 
-template <int WM, int WN, int BK>
-static void gemm2_go(int nc, int M, int d, int parts, const double *W, const double *Xs, double *out,
-                     hipStream_t s) {
-    const int kchunk = (cdiv(M, parts) + BK - 1) / BK * BK;
-    dim3 grid(cdiv(nc, 32 * WM), cdiv(d, 32 * WN), parts);
-    hipLaunchKernelGGL((k_gemm_f64<false, false, WM, WN, BK>), grid, dim3(256), 0, s, nc, d, M, kchunk, W, Xs, out,
-                       (const double *)nullptr, 0.0, 0, (double *)nullptr);
-}
-
 void launch_gemm2_f64(int cfg, int parts, int nc, int M, int d, const double *W, const double *Xs, double *G,
                       double *Gparts, hipStream_t s) {
     if (nc <= 0) return;
     double *out = parts > 1 ? Gparts : G;
-    switch (cfg) {
-        case 0: gemm2_go<4, 2, 16>(nc, M, d, parts, W, Xs, out, s); break;
-        case 1: gemm2_go<2, 2, 16>(nc, M, d, parts, W, Xs, out, s); break;
-        case 2: gemm2_go<2, 4, 16>(nc, M, d, parts, W, Xs, out, s); break;
-        case 3: gemm2_go<4, 2, 32>(nc, M, d, parts, W, Xs, out, s); break;
-        case 4: gemm2_go<2, 2, 32>(nc, M, d, parts, W, Xs, out, s); break;
-        default: gemm2_go<2, 4, 32>(nc, M, d, parts, W, Xs, out, s); break;
+    if (gemm_stream_ok(M, d)) {
+        launch_gemm2_f64_stream(cfg, parts, nc, M, d, W, Xs, out, s);
+    } else {
+        const int kchunk = (cdiv(M, parts) + 15) / 16 * 16;
+        hipLaunchKernelGGL((k_gemm_f64<false, false>), dim3(cdiv(nc, 64), cdiv(d, 64), parts), dim3(256), 0, s, nc, d, M,
+                           kchunk, W, Xs, out, (const double *)nullptr, 0.0, 0, (double *)nullptr);
     }
     if (parts > 1) launch_sum_parts_f64(nc, d, parts, Gparts, G, s);
 }
@@ -1931,14 +1907,15 @@ void launch_sum_fixed(size_t n, const double *v, double *out, hipStream_t s) {
 //   var(x) = k(x,x) - k_x^T (K_MM + reg I)^-1 k_x,  k_x[s] = delta^2 kernel(x, X_s)
 // Cinv = (K_MM + reg I)^-1 is formed on the host when the model is asked for it.
 // ----------------------------------------------------------------------------
-template <int WM, int WN, int BK>
-static void gemm_nt_go(int rows, int cols, int kd, const double *A, const double *B, double *C, hipStream_t s) {
-    dim3 grid(cdiv(rows, 32 * WM), cdiv(cols, 32 * WN), 1);
-    hipLaunchKernelGGL((k_gemm_f64<true, false, WM, WN, BK>), grid, dim3(256), 0, s, rows, cols, kd, kd, A, B, C,
-                       (const double *)nullptr, 0.0, 0, (double *)nullptr);
-}
 void launch_gemm_nt_f64(int rows, int cols, int kd, const double *A, const double *B, double *C, hipStream_t s) {
-    if (rows > 0 && cols > 0) gemm_nt_go<2, 2, 16>(rows, cols, kd, A, B, C, s);
+    if (rows > 0 && cols > 0)
+        hipLaunchKernelGGL((k_gemm_f64<true, false>), dim3(cdiv(rows, 64), cdiv(cols, 64)), dim3(256), 0, s, rows, cols, kd,
+                           kd, A, B, C, (const double *)nullptr, 0.0, 0, (double *)nullptr);
+}
+void launch_gemm_nn_f64(int rows, int kd, int cols, const double *A, const double *B, double *C, hipStream_t s) {
+    if (rows > 0 && cols > 0)
+        hipLaunchKernelGGL((k_gemm_f64<false, false>), dim3(cdiv(rows, 64), cdiv(cols, 64)), dim3(256), 0, s, rows, cols,
+                           kd, kd, A, B, C, (const double *)nullptr, 0.0, 0, (double *)nullptr);
 }
 
 __device__ __forceinline__ double powz(double x, double zeta, int iz) {
