@@ -594,7 +594,7 @@ void gapx::reset_arena_views(Engine &eg) {
                     &w.nb_r, &w.nb_d, &w.pairF, &w.pairE, &w.esite, &w.X, &w.norm, &w.cbuf, &w.W, &w.Wf, &w.e_part,
                     &w.G, &w.Gparts, &w.split_ws, &w.f, &w.le, &w.lv, &w.e, &w.vir, &w.minmax, &w.last_pos,
                     &w.skin_flags, &w.cmask, &w.t1_j, &w.t1_shift, &w.t1_r, &w.t2_i, &w.t2_k, &w.nl_flags, &w.eatom,
-                    &w.vK, &w.vk, &w.vV, &w.Gv, &w.pairFv, &w.pairVE, &w.varsite, &w.o_epc, &w.o_lgv, &w.o_gvg,
+                    &w.vK, &w.vk, &w.vV, &w.Gv, &w.pairFv, &w.pairVE, &w.varsite, &w.hout,
                     &w.spart})
         b->drop_view();
     for (auto *v : {&w.centres, &w.var_inst, &w.cut2_inst})
@@ -886,10 +886,13 @@ static int stage_inputs(gapx_model *m, Engine &eg, int S, const int *atom_off, c
 //    call's extents; the cell counts are the host's (from the previous call's extents),
 //    and a structure whose counts would change flags the call for redoing as well.
 static int ensure_nl_tables(Workspace &w, int T1cap);
+static bool nl_small(int N, int NC, bool dev_geo) { return !dev_geo && N <= kNlFrontAtoms && NC <= kNlFrontCells; }
 
 struct NLPlan {
     int N = 0, S = 0, NC = 0;
     bool spec = false, one_pass = false, any_np = false, dev_geo = false;
+    bool inl = false;   // the geometry goes to the list's first kernel as an argument
+    NLGeom geo1;
     int cap1 = 0, cap2 = 0, capT1 = 0;
 };
 
@@ -906,7 +909,6 @@ static bool geo_equal_static(const NLGeom &x, const NLGeom &y) {
 // device for lat_eff).
 static int nl_prepare(gapx_model *m, Engine &eg, int S, const int *atom_off, const double *d_pos, const double *h_pos,
                       const double *lats, const int *pbcs, double cutoff, bool spec, NLPlan &pl) {
-    (void)m;
     Workspace &w = eg.ws;
     hipStream_t s = eg.stream;
     const int N = atom_off[S];
@@ -980,10 +982,15 @@ static int nl_prepare(gapx_model *m, Engine &eg, int S, const int *atom_off, con
     // an earlier speculative one of the same structures.
     const bool same = eg.have_geo && eg.h_geo.size() == geo.size() && eg.h_cell_base == cbase &&
                       std::equal(geo.begin(), geo.end(), eg.h_geo.begin(), dev_geo ? geo_equal_static : geo_equal);
-    if (!same) {
+    pl.inl = S == 1 && !m->graphs && nl_small(N, NC, dev_geo);   // a graph keeps its kernels' arguments
+    CHK(w.geo.ensure((size_t)S * sizeof(NLGeom) + 8));
+    CHK(w.cell_base.ensure((size_t)(S + 1) * 4));
+    if (pl.inl) {
+        pl.geo1 = geo[0];
+        eg.h_geo = geo;
+        eg.have_geo = false;   // the device copy is the launch's
+    } else if (!same) {
         eg.have_geo = false;
-        CHK(w.geo.ensure((size_t)S * sizeof(NLGeom) + 8));
-        CHK(w.cell_base.ensure((size_t)(S + 1) * 4));
         const size_t gb = (size_t)S * sizeof(NLGeom), cb = (size_t)(S + 1) * 4;
         CHK(staging_ready(eg));
         CHK(eg.stage_geo.ensure(gb + cb + 64));
@@ -1034,7 +1041,10 @@ static int nl_prepare(gapx_model *m, Engine &eg, int S, const int *atom_off, con
         CHK(w.t2_k.ensure((size_t)N * pl.cap2 * 4 + 4));
     }
     if (spec) {
-        pl.capT1 = eg.nl_capT1;
+        // up to 2^18 entries the tables take all that the slots can hold, so that a call with
+        // more atoms than the last is not redone for the total alone
+        const long all = (long)N * pl.cap1;
+        pl.capT1 = all <= (1 << 18) ? std::max(eg.nl_capT1, (int)all) : eg.nl_capT1;
         CHK(ensure_nl_tables(w, pl.capT1));
     }
     return GAPX_OK;
@@ -1063,7 +1073,7 @@ static int ensure_nl_tables(Workspace &w, int T1cap) {
 // candidates through the cells' atom lists; larger problems also write cell-ordered
 // copies of positions and shifts, which their search reads without a dependent load
 // (the copies cost the one-block front more than its search gains).
-static bool nl_small(const NLPlan &pl) { return !pl.dev_geo && pl.N <= kNlFrontAtoms && pl.NC <= kNlFrontCells; }
+static bool nl_small(const NLPlan &pl) { return nl_small(pl.N, pl.NC, pl.dev_geo); }
 
 // Binning, the candidate search and the count scans (flags: [0] overflow, [1] largest
 // neighbour1 count, [2] largest neighbour2 count, [3] neighbour1 total).
@@ -1078,9 +1088,13 @@ static void nl_launch_front(Engine &eg, const NLPlan &pl, const double *d_pos) {
     CellAtom *cpos = small ? nullptr : w.cpos.as<CellAtom>();
     CellShift *cms = small ? nullptr : w.cms.as<CellShift>();
     if (small) {
-        launch_nl_front_small(N, NC, d_pos, dgeo, dsid, dcb, w.cell_of.as<int>(), w.map_shift.as<int>(),
-                              w.cell_cnt.as<int>(), w.cell_start.as<int>(), w.cell_atoms.as<int>(), nullptr,
-                              nullptr, w.n2_cnt.as<int>(), w.n2_fill.as<int>(), flags, s);
+        // d_pos is the engine's own buffer where positions come from the staging
+        launch_nl_front_small(N, NC, const_cast<double *>(d_pos), w.geo.as<NLGeom>(), dsid, w.cell_base.as<int>(),
+                              w.cell_of.as<int>(), w.map_shift.as<int>(), w.cell_cnt.as<int>(),
+                              w.cell_start.as<int>(), w.cell_atoms.as<int>(), nullptr, nullptr, w.n2_cnt.as<int>(),
+                              w.n2_fill.as<int>(), flags, pl.inl ? &pl.geo1 : nullptr, pl.inl ? eg.pos_src : nullptr,
+                              s);
+        if (pl.inl) eg.pos_src = nullptr;
     } else {
         {
             int *zp[5] = {w.cell_cnt.as<int>(), w.cell_fill.as<int>(), w.n2_cnt.as<int>(), w.n2_fill.as<int>(),
@@ -1167,10 +1181,13 @@ static void nl_launch_back(Engine &eg, const NLPlan &pl, const double *d_pos, bo
 }
 
 // next builds' capacities from a build's flags: per-atom slots of the largest counts plus a
-// quarter and 8, the neighbour1 tables of the total plus an eighth and 1024 (grow-only)
+// quarter and 8, shrinking by an eighth a build at most (calls for two structures in turn, a
+// dense and a sparse one, keep the slots of the dense one), the neighbour1 tables of the
+// total plus an eighth and 1024 (grow-only)
 static void update_nl_caps(Engine &eg, const int *flags) {
-    eg.nl_cap1 = (flags[1] + flags[1] / 4 + 8 + 3) & ~3;
-    eg.nl_cap2 = (flags[2] + flags[2] / 4 + 8 + 3) & ~3;
+    auto cap = [](int old, int n) { return std::max((n + n / 4 + 8 + 3) & ~3, (old - old / 8) & ~3); };
+    eg.nl_cap1 = cap(eg.nl_cap1, flags[1]);
+    eg.nl_cap2 = cap(eg.nl_cap2, flags[2]);
     const long t = (long)flags[3] + flags[3] / 8 + 1024;
     if (t < INT32_MAX / 4) eg.nl_capT1 = std::max(eg.nl_capT1, (int)t);
 }
@@ -1670,7 +1687,14 @@ static int connect_external(Engine &eg, const ExtNL &x, int N, const double *d_p
     return GAPX_OK;
 }
 
-static int resolve_pending_list(gapx_model *m, Engine &eg, std::vector<Engine::Pending> *);
+// positions still in the staging go to the device (a list that does not read them itself)
+static int flush_positions(Engine &eg, const double *d_pos, int N) {
+    if (!eg.pos_src) return GAPX_OK;
+    const double *src = eg.pos_src;
+    eg.pos_src = nullptr;
+    HIPCHK(hipMemcpyAsync(const_cast<double *>(d_pos), src, (size_t)N * 24, hipMemcpyHostToDevice, eg.stream));
+    return GAPX_OK;
+}
 
 int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, const double *d_pos, const double *h_pos,
                      const int *Z, const double *lats, const int *pbcs, double nl_cutoff, unsigned want, double *d_e,
@@ -1693,15 +1717,17 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
     const bool want_vgrad = want_var && opt->d_gvg;
     // The speculative neighbour list: no read-back inside the call, so the whole call is
     // one launch sequence (and graph).  Not for the first build, a skin (whose reuse test
-    // reads back), a supplied connection, calc options or the allocation-free entry.
-    const bool spec_ok = !ext && !opt && !noalloc && !eg.force_exact && !(rc > m->cutoff && m->nl_reuse);
+    // reads back), a supplied connection, the allocation-free entry, a mask or the options of
+    // a device call (a host call resolves before it returns).
+    const bool spec_ok = !ext && (!opt || (h_pos && !opt->mask)) && !noalloc && !eg.force_exact &&
+                         !(rc > m->cutoff && m->nl_reuse);
     // Calls queued speculatively are read (and redone if they overflowed) before anything
     // of this call is staged or queued: before a call that is not speculative, and when
     // the read-back area is full.
     if (!eg.force_exact) {
         const size_t need_max = (16 + 48 * (size_t)S + 15) & ~(size_t)15;
         if (!spec_ok || eg.pending.size() >= 64 || eg.checks_used + need_max > eg.checks.cap) {
-            CHK(resolve_pending_list(m, eg, nullptr));
+            CHK(resolve_pending(m, eg));
             eg.checks.coherent = true;   // written by the step's last kernel in eager calls
             if (spec_ok) CHK(eg.checks.ensure(std::max<size_t>(need_max * 64, 4096)));
         }
@@ -1716,6 +1742,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
     NLPlan pl;
     if (spec_ok) CHK(nl_prepare(m, eg, S, atom_off, d_pos, h_pos, lats, pbcs, rc, true, pl));
     const bool spec = spec_ok && pl.spec;
+    if (!(spec_ok && pl.inl)) CHK(flush_positions(eg, d_pos, N));
     const int t_nl0 = tm.on ? tm.mark(s) : -1;
     int P = 0;
     if (spec) {
@@ -1985,12 +2012,14 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         launch_gather(N, w.Z.as<int>(), m->d_e0.as<double>(), m->E_scale, w.nb_off.as<int>(), w.nb_rev.as<int>(),
                       w.nb_d.as<double>(), w.pairF.as<double>(), pairE, w.esite.as<double>(), o_f, o_le,
                       o_lv, cmask, S == 1 ? w.spart.as<double>() : nullptr, s);
-        if (S == 1) launch_struct_finish(N, w.spart.as<double>(), o_e, o_v, s, w.nl_flags.as<int>(), flag_slot);
-        else launch_struct_reduce(S, w.atom_off.as<int>(), o_le, o_lv, o_e, o_v, s, w.nl_flags.as<int>(), flag_slot);
         if (want_var)
             launch_gather_var(N, w.nb_off.as<int>(), w.nb_rev.as<int>(), w.pairFv.as<double>(),
                               has_d2b_var ? w.pairVE.as<double>() : nullptr, w.varsite.as<double>(), opt->d_gvg,
                               opt->d_lgv, s);
+        if (S == 1)
+            launch_struct_finish(N, w.spart.as<double>(), o_e, o_v, s, w.nl_flags.as<int>(), flag_slot, eg.out_src,
+                                 eg.out_dst, eg.out_n);
+        else launch_struct_reduce(S, w.atom_off.as<int>(), o_le, o_lv, o_e, o_v, s, w.nl_flags.as<int>(), flag_slot);
         if (marks) tm.stage(5, tg, tm.mark(s));
     };
     eg.var_valid = want_var;
@@ -2047,6 +2076,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         pc.d_e = d_e; pc.d_le = d_le; pc.d_f = d_f; pc.d_v = d_v; pc.d_lv = d_lv;
         pc.slot = eg.checks_used;
         pc.extents = pl.dev_geo;
+        if (opt) { pc.has_opt = true; pc.opt = *opt; }
         char *slot = eg.checks.as<char>() + pc.slot;
         if (!flag_slot) HIPCHK(hipMemcpyAsync(slot, w.nl_flags.p, 16, hipMemcpyDeviceToHost, s));
         if (pl.dev_geo) HIPCHK(hipMemcpyAsync(slot + 16, w.minmax.p, 48 * (size_t)S, hipMemcpyDeviceToHost, s));
@@ -2059,7 +2089,8 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
 
 // Read the pending calls' flags (after one synchronisation), refresh the capacities and
 // extents from them, and redo in order every call from the first that overflowed.
-static int resolve_pending_list(gapx_model *m, Engine &eg, std::vector<Engine::Pending> *) {
+int gapx::resolve_pending(gapx_model *m, Engine &eg, bool *redone) {
+    if (redone) *redone = false;
     if (eg.pending.empty()) return GAPX_OK;
     HIPCHK(hipStreamSynchronize(eg.stream));
     eg.staging_dirty = false;
@@ -2080,19 +2111,19 @@ static int resolve_pending_list(gapx_model *m, Engine &eg, std::vector<Engine::P
     eg.checks_used = 0;
     if (first_bad < 0) return GAPX_OK;
     eg.force_exact = true;
+    if (redone) *redone = true;
     int st = GAPX_OK;
     for (size_t k = first_bad; k < todo.size() && st == GAPX_OK; k++) {
         const Engine::Pending &p = todo[k];
         st = eval_batch(m, eg, p.S, p.off.data(), p.d_pos, nullptr, p.Z.data(), p.lats.data(), p.pbcs.data(),
-                        p.nl_cutoff, p.want, p.d_e, p.d_le, p.d_f, p.d_v, p.d_lv);
+                        p.nl_cutoff, p.want, p.d_e, p.d_le, p.d_f, p.d_v, p.d_lv, nullptr,
+                        p.has_opt ? &p.opt : nullptr);
     }
     eg.force_exact = false;
     CHK(st);
     HIPCHK(hipStreamSynchronize(eg.stream));
     return GAPX_OK;
 }
-
-int gapx::resolve_pending(gapx_model *m, Engine &eg) { return resolve_pending_list(m, eg, nullptr); }
 
 extern "C" int gapx_calc_device(gapx_model *m, int N, const double *d_pos, const int *Z, const double *lat,
                                 const int *pbc, double nl_cutoff, unsigned want, double *d_e, double *d_le,
@@ -2135,65 +2166,65 @@ int gapx::calc_host(gapx_model *m, Engine &eg, int S, const int *atom_off, const
     const int N = atom_off[S];
     if (N > 0 && !pos) return fail(GAPX_E_ARG, "positions are NULL");
     HIPCHK(hipSetDevice(m->device));
+    CHK(resolve_pending(m, eg));   // device calls queued earlier know nothing of this call's staging
     Workspace &w = eg.ws;
     hipStream_t s = eg.stream;
     CHK(w.pos.ensure((size_t)N * 24 + 24));
     CHK(ensure_outputs(w, S, N));   // before taking the output pointers below
-    // one pinned block: positions in, then results out
-    const size_t bpos = (size_t)N * 24, be = (size_t)S * 8, bv = (size_t)S * 72, bf = (size_t)N * 24,
-                 ble = (size_t)N * 8, blv = (size_t)N * 72;
-    // option outputs: device scratch read back with the rest (sized before any copy is queued)
+    // The results asked for lie one after the other on the device and in pinned memory: one copy
+    struct Out { bool on; double *dst; size_t n, off; };
+    Out o[8] = {{(want & GAPX_WANT_E) != 0, e, (size_t)S, 0},
+                {(want & GAPX_WANT_V) != 0, v, (size_t)S * 9, 0},
+                {(want & GAPX_WANT_F) != 0, f, (size_t)N * 3, 0},
+                {(want & GAPX_WANT_LOCAL_E) != 0, le, (size_t)N, 0},
+                {(want & GAPX_WANT_LOCAL_V) != 0, lv, (size_t)N * 9, 0},
+                {opt && h_epc, h_epc, m->coords.size(), 0},
+                {opt && opt->variance && h_lgv, h_lgv, (size_t)N, 0},
+                {opt && opt->variance && h_gvg, h_gvg, (size_t)N * 3, 0}};
+    size_t total = 0;
+    for (Out &q : o)
+        if (q.on) { q.off = total; total += q.n; }
+    CHK(w.hout.ensure(total * 8 + 8));
+    auto dev = [&](int k) { return o[k].on ? w.hout.as<double>() + o[k].off : nullptr; };
     CalcOpts o2;
-    const size_t bepc = m->coords.size() * 8, blgv = (size_t)N * 8, bgvg = (size_t)N * 24;
-    size_t bopt = 0;
     if (opt) {
         o2 = *opt;
-        o2.d_epc = o2.d_lgv = o2.d_gvg = nullptr;
-        if (h_epc) { CHK(w.o_epc.ensure(bepc + 8)); o2.d_epc = w.o_epc.as<double>(); bopt += bepc; }
-        if (opt->variance && h_lgv) { CHK(w.o_lgv.ensure(blgv + 8)); o2.d_lgv = w.o_lgv.as<double>(); bopt += blgv; }
-        if (opt->variance && h_gvg) { CHK(w.o_gvg.ensure(bgvg + 8)); o2.d_gvg = w.o_gvg.as<double>(); bopt += bgvg; }
+        o2.d_epc = dev(5); o2.d_lgv = dev(6); o2.d_gvg = dev(7);
     }
-    CHK(eg.stage_io.ensure(std::max(bpos, be + bv + bf + ble + blv + bopt) + 64));
+    const size_t bpos = (size_t)N * 24;
+    eg.stage_io.coherent = true;   // kernels of small calls read and write it
+    CHK(eg.stage_io.ensure(bpos + total * 8 + 64));
     char *h = eg.stage_io.as<char>();
-    if (N) {
-        memcpy(h, pos, bpos);
-        HIPCHK(hipMemcpyAsync(w.pos.p, h, bpos, hipMemcpyHostToDevice, s));
-    }
-    CHK(eval_batch(m, eg, S, atom_off, w.pos.as<double>(), pos, Z, lats, pbcs, nl_cutoff,
-                   want | GAPX_WANT_E | GAPX_WANT_LOCAL_E,   // no gradient unless one of its outputs is asked for
-                   w.e.as<double>(), w.le.as<double>(), w.f.as<double>(), w.vir.as<double>(), w.lv.as<double>(),
-                   ext, opt ? &o2 : nullptr));
-    CHK(resolve_pending(m, eg));   // a speculative call that overflowed is redone before its results are read
-    char *o = h;
-    auto get = [&](bool on, const DBuf &src, size_t bytes, char **dst) -> int {
-        *dst = nullptr;
-        if (!on || !bytes) return GAPX_OK;
-        HIPCHK(hipMemcpyAsync(o, src.p, bytes, hipMemcpyDeviceToHost, s));
-        *dst = o;
-        o += bytes;
+    double *ho = (double *)(h + bpos);
+    if (N) memcpy(h, pos, bpos);
+    // Up to 64 KB a way no copy is queued (997 atoms: 24 KB; a block moves that in 3 us, a copy
+    // launch takes as long and the gaps around it 6 to 10 us); larger ones are copied.
+    constexpr size_t kDirect = 64 << 10;
+    const bool direct = S == 1 && N > 0 && total * 8 <= kDirect && !m->graphs;
+    eg.pos_src = N ? (const double *)h : nullptr;
+    if (bpos > kDirect) CHK(flush_positions(eg, w.pos.as<double>(), N));
+    eg.out_src = w.hout.as<double>();
+    eg.out_dst = direct ? ho : nullptr;
+    eg.out_n = (int)total;
+    auto fetch = [&]() -> int {
+        if (total && !direct) HIPCHK(hipMemcpyAsync(ho, w.hout.p, total * 8, hipMemcpyDeviceToHost, s));
         return GAPX_OK;
     };
-    char *pe, *pv, *pf, *ple, *plv;
-    CHK(get(want & GAPX_WANT_E, w.e, be, &pe));
-    CHK(get(want & GAPX_WANT_V, w.vir, bv, &pv));
-    CHK(get(want & GAPX_WANT_F, w.f, bf, &pf));
-    CHK(get(want & GAPX_WANT_LOCAL_E, w.le, ble, &ple));
-    CHK(get(want & GAPX_WANT_LOCAL_V, w.lv, blv, &plv));
-    char *pepc = nullptr, *plgv = nullptr, *pgvg = nullptr;
-    if (opt) {
-        CHK(get(o2.d_epc != nullptr, w.o_epc, bepc, &pepc));
-        CHK(get(o2.d_lgv != nullptr, w.o_lgv, blgv, &plgv));
-        CHK(get(o2.d_gvg != nullptr, w.o_gvg, bgvg, &pgvg));
-    }
+    auto work = [&]() -> int {
+        CHK(eval_batch(m, eg, S, atom_off, w.pos.as<double>(), pos, Z, lats, pbcs, nl_cutoff, want, dev(0), dev(3),
+                       dev(2), dev(1), dev(4), ext, opt ? &o2 : nullptr));
+        CHK(fetch());
+        bool redone = false;   // a speculative call that overflowed: its results are copied again
+        CHK(resolve_pending(m, eg, &redone));
+        return redone ? fetch() : GAPX_OK;
+    };
+    const int st = work();
+    eg.pos_src = nullptr;
+    eg.out_dst = nullptr;
+    CHK(st);
     HIPCHK(hipStreamSynchronize(s));
-    if (pepc) memcpy(h_epc, pepc, bepc);
-    if (plgv) memcpy(h_lgv, plgv, blgv);
-    if (pgvg) memcpy(h_gvg, pgvg, bgvg);
-    if (pe) memcpy(e, pe, be);
-    if (pv) memcpy(v, pv, bv);
-    if (pf) memcpy(f, pf, bf);
-    if (ple) memcpy(le, ple, ble);
-    if (plv) memcpy(lv, plv, blv);
+    for (const Out &q : o)
+        if (q.on && q.n) memcpy(q.dst, ho + q.off, q.n * 8);
     return GAPX_OK;
 }
 

@@ -172,7 +172,7 @@ struct Workspace {
     // variance, pair sums, per-atom variances; per coordinate the instance variances
     DBuf vK, vk, vV, Gv, pairFv, pairVE, varsite;
     std::vector<DBuf> var_inst, cut2_inst;
-    DBuf o_epc, o_lgv, o_gvg;    // device outputs of the host-buffer entry points' options
+    DBuf hout;                   // the results a host-buffer call asked for, one after the other
 };
 
 // IPModel_GAP_Calc's args_str options that change what is computed (IPModel_GAP.f95:324-335)
@@ -299,6 +299,11 @@ struct Engine {
     HBuf stage_in;    // Z, structure map, centre lists
     HBuf stage_geo;   // lattice inverses, fractional extents, geometry table
     HBuf stage_io;    // positions in, results out (host-buffer entry points)
+    // Small host calls of one structure: the list's first kernel reads the positions from the
+    // staging (pos_src, until one has) and the step's last kernel writes the results there
+    const double *pos_src = nullptr, *out_src = nullptr;
+    double *out_dst = nullptr;
+    int out_n = 0;
     HBuf ctl;         // the neighbour-count read-back
     StageTimer timer;
     std::vector<int> h_Z, h_off, h_sid, h_cell_base;
@@ -335,6 +340,8 @@ struct Engine {
         double *d_e = nullptr, *d_le = nullptr, *d_f = nullptr, *d_v = nullptr, *d_lv = nullptr;
         size_t slot = 0;             // byte offset of its flags (+ extents) in `checks`
         bool extents = false;
+        bool has_opt = false;        // a host call's options (without a mask), its outputs on the device
+        CalcOpts opt;
     };
     std::vector<Pending> pending;
     HBuf checks;                     // pinned (fine-grained) read-back slots of the pending calls
@@ -379,8 +386,8 @@ int eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, const doub
 // Forget every arena view of a workspace and the state that refers to its buffers.
 void reset_arena_views(Engine &eg);
 // Read the overflow flags of the engine's speculative calls (one synchronisation) and
-// redo, exactly and in order, every call from the first that overflowed.
-int resolve_pending(gapx_model *m, Engine &eg);
+// redo, exactly and in order, every call from the first that overflowed (*redone: one was).
+int resolve_pending(gapx_model *m, Engine &eg, bool *redone = nullptr);
 // Host-buffer evaluation of S structures on engine eg (pinned staging both ways).
 // ext: a caller-supplied connection (one structure), else calc_connect.
 // opt (nullable): per-call options; their host outputs h_epc[n_coord], h_lgv[N], h_gvg[3N]

@@ -58,12 +58,14 @@ void launch_nl_cell_rank(int N, const int *cell_of, const int *start, const int 
                          int *atoms, const double *pos, const int *map_shift, CellAtom *cpos, CellShift *cms,
                          hipStream_t s);
 // bin, scan, fill and rank in one block for N <= kNlFrontAtoms atoms in NC <= kNlFrontCells
-// cells (also zeroes n2_cnt, n2_fill and the four flags)
+// cells (also zeroes n2_cnt, n2_fill and the four flags); one (nullable): the geometry of the
+// only structure, which is then written to geo and cell_base, and src (nullable): its positions
+// in pinned host memory, written to pos
 constexpr int kNlFrontAtoms = 8192, kNlFrontCells = 8192;
-void launch_nl_front_small(int N, int NC, const double *pos, const NLGeom *geo, const int *sid,
-                           const int *cell_base, int *cell_of, int *map_shift, int *cell_cnt, int *cell_start,
-                           int *cell_atoms, CellAtom *cpos, CellShift *cms, int *n2_cnt, int *n2_fill, int *flags,
-                           hipStream_t s);
+void launch_nl_front_small(int N, int NC, double *pos, NLGeom *geo, const int *sid, int *cell_base, int *cell_of,
+                           int *map_shift, int *cell_cnt, int *cell_start, int *cell_atoms, CellAtom *cpos,
+                           CellShift *cms, int *n2_cnt, int *n2_fill, int *flags, const NLGeom *one,
+                           const double *src, hipStream_t s);
 // mode 0: count; 1: fill the CSR tables; 2: one pass into per-atom slots of cap1 / cap2
 // (counts in n1_cnt / n2_cnt, *ovf = 1 when a slot range overflows)
 void launch_nl_pairs(int mode, int N, const double *pos, const int *map_shift, const int *cell_of,
@@ -245,9 +247,11 @@ void launch_gather(int N, const int *Z, const double *e0, double E_scale, const 
                    hipStream_t s);
 // the energy and virial of one structure of N atoms from the gather's block partials;
 // with flag_dst (pinned host memory, written by the device without a copy launch) the
-// four neighbour-list build flags at flag_src are copied there as well
+// four neighbour-list build flags at flag_src are copied there as well, and with out_dst
+// (pinned too) the out_n results at out_src
 void launch_struct_finish(int N, const double *part, double *e_out, double *virial_out, hipStream_t s,
-                          const int *flag_src = nullptr, int *flag_dst = nullptr);
+                          const int *flag_src = nullptr, int *flag_dst = nullptr, const double *out_src = nullptr,
+                          double *out_dst = nullptr, int out_n = 0);
 void launch_struct_reduce(int S, const int *atom_off, const double *local_e, const double *local_virial,
                           double *e_out, double *virial_out, hipStream_t s, const int *flag_src = nullptr,
                           int *flag_dst = nullptr);

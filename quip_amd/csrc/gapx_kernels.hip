@@ -396,12 +396,8 @@ __device__ __forceinline__ void mult3_exact(const double *g, double p0, double p
 
 // Cell of atom n and its map shift (Connection.f95 cell_of_pos with the lattice shift
 // that folds the position into the cell): writes map_shift[3n..3n+2], returns the cell.
-__device__ __forceinline__ int nl_bin_atom(int n, const double *__restrict__ pos, const NLGeom *__restrict__ geo,
-                                           const int *__restrict__ sid, const int *__restrict__ cell_base,
-                                           int *map_shift) {
+__device__ __forceinline__ int nl_bin_atom(int n, const double *pos, const NLGeom &g, int base, int *map_shift) {
 #pragma clang fp contract(off)
-    const int st = sid[n];
-    const NLGeom &g = geo[st];
     double lp[3];
     mult3_exact(g.inv_eff, pos[3 * n], pos[3 * n + 1], pos[3 * n + 2], lp);
     int ci[3];
@@ -414,14 +410,14 @@ __device__ __forceinline__ int nl_bin_atom(int n, const double *__restrict__ pos
         c = c < 1 ? 1 : (c > g.cells[a] ? g.cells[a] : c);
         ci[a] = c - 1;
     }
-    return cell_base[st] + (ci[2] * g.cells[1] + ci[1]) * g.cells[0] + ci[0];
+    return base + (ci[2] * g.cells[1] + ci[1]) * g.cells[0] + ci[0];
 }
 __global__ void k_nl_bin(int N, const double *__restrict__ pos, const NLGeom *__restrict__ geo,
                          const int *__restrict__ sid, const int *__restrict__ cell_base, int *cell_of,
                          int *map_shift, int *cell_cnt) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
-    const int cell = nl_bin_atom(n, pos, geo, sid, cell_base, map_shift);
+    const int st = sid[n], cell = nl_bin_atom(n, pos, geo[st], cell_base[st], map_shift);
     cell_of[n] = cell;
     atomicAdd(&cell_cnt[cell], 1);
 }
@@ -473,14 +469,20 @@ void launch_nl_cell_rank(int N, const int *cell_of, const int *start, const int 
 // arrival order and rank each cell's atoms by descending index, with the cells and
 // their unsorted lists in LDS.  The same tables as the separate kernels: the order
 // within a cell is fixed by the ranking, not by the atomics.
+// ONE: a single structure whose geometry comes as a kernel argument, written to geo[0] and
+// cell_base for the kernels after it, and whose positions may come from pinned host memory
+// (src, copied to pos first): no copy launches before the list.  8 Si atoms, host call: the
+// position copy took 3 us and the gaps around it 9 us; for a slab, whose geometry changes
+// with every call, two more copies went.
 constexpr int kFrontThreads = 1024;
-__global__ __launch_bounds__(kFrontThreads) void k_nl_front_small(int N, int NC, const double *__restrict__ pos,
-                                                                  const NLGeom *__restrict__ geo,
-                                                                  const int *__restrict__ sid,
-                                                                  const int *__restrict__ cell_base, int *cell_of,
-                                                                  int *map_shift, int *cell_cnt, int *cell_start,
-                                                                  int *cell_atoms, CellAtom *cpos, CellShift *cms,
-                                                                  int *n2_cnt, int *n2_fill, int *flags) {
+template <bool ONE>
+__global__ __launch_bounds__(kFrontThreads) void k_nl_front_small(int N, int NC, double *pos, NLGeom *geo,
+                                                                  const int *__restrict__ sid, int *cell_base,
+                                                                  int *cell_of, int *map_shift, int *cell_cnt,
+                                                                  int *cell_start, int *cell_atoms, CellAtom *cpos,
+                                                                  CellShift *cms, int *n2_cnt, int *n2_fill,
+                                                                  int *flags, NLGeom one, const double *src) {
+    __shared__ NLGeom sgeo;
     __shared__ int scnt[kNlFrontCells], sfill[kNlFrontCells];
     __shared__ int scell[kNlFrontAtoms], suns[kNlFrontAtoms];
     __shared__ int wsum[kFrontThreads / 64];
@@ -488,13 +490,26 @@ __global__ __launch_bounds__(kFrontThreads) void k_nl_front_small(int N, int NC,
     for (int c = t; c < NC; c += kFrontThreads) scnt[c] = 0;
     for (int i = t; i < N; i += kFrontThreads) { n2_cnt[i] = 0; n2_fill[i] = 0; }
     if (t < 4) flags[t] = 0;
+    if (ONE) {
+        if (t == 0) {
+            sgeo = one;
+            geo[0] = one;
+            cell_base[0] = 0;
+            cell_base[1] = NC;
+        }
+        if (src)
+            for (int i = t; i < 3 * N; i += kFrontThreads) pos[i] = src[i];
+    }
     __syncthreads();
     for (int n0 = t; n0 < N; n0 += 4 * kFrontThreads) {   // four atoms' loads in flight per thread
         int cl[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const int n = n0 + u * kFrontThreads;
-            cl[u] = n < N ? nl_bin_atom(n, pos, geo, sid, cell_base, map_shift) : -1;
+            cl[u] = -1;
+            if (n >= N) continue;
+            if (ONE) cl[u] = nl_bin_atom(n, pos, sgeo, 0, map_shift);
+            else cl[u] = nl_bin_atom(n, pos, geo[sid[n]], cell_base[sid[n]], map_shift);
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -544,12 +559,18 @@ __global__ __launch_bounds__(kFrontThreads) void k_nl_front_small(int N, int NC,
         if (cpos) put_cell_atom(st + rank, n, pos, map_shift, cpos, cms);
     }
 }
-void launch_nl_front_small(int N, int NC, const double *pos, const NLGeom *geo, const int *sid,
-                           const int *cell_base, int *cell_of, int *map_shift, int *cell_cnt, int *cell_start,
-                           int *cell_atoms, CellAtom *cpos, CellShift *cms, int *n2_cnt, int *n2_fill, int *flags,
-                           hipStream_t s) {
-    hipLaunchKernelGGL(k_nl_front_small, dim3(1), dim3(kFrontThreads), 0, s, N, NC, pos, geo, sid, cell_base, cell_of,
-                       map_shift, cell_cnt, cell_start, cell_atoms, cpos, cms, n2_cnt, n2_fill, flags);
+void launch_nl_front_small(int N, int NC, double *pos, NLGeom *geo, const int *sid, int *cell_base, int *cell_of,
+                           int *map_shift, int *cell_cnt, int *cell_start, int *cell_atoms, CellAtom *cpos,
+                           CellShift *cms, int *n2_cnt, int *n2_fill, int *flags, const NLGeom *one,
+                           const double *src, hipStream_t s) {
+    if (one)
+        hipLaunchKernelGGL(k_nl_front_small<true>, dim3(1), dim3(kFrontThreads), 0, s, N, NC, pos, geo, sid, cell_base,
+                           cell_of, map_shift, cell_cnt, cell_start, cell_atoms, cpos, cms, n2_cnt, n2_fill, flags,
+                           *one, src);
+    else
+        hipLaunchKernelGGL(k_nl_front_small<false>, dim3(1), dim3(kFrontThreads), 0, s, N, NC, pos, geo, sid, cell_base,
+                           cell_of, map_shift, cell_cnt, cell_start, cell_atoms, cpos, cms, n2_cnt, n2_fill, flags,
+                           NLGeom(), nullptr);
 }
 
 // Wave-parallel form of the same search: a group of lanes per atom1, lanes over the
@@ -2193,9 +2214,12 @@ __global__ __launch_bounds__(kReduceThreads) void k_struct_reduce(const int *ato
 }
 // One structure: the totals from the gather's block partials (10 per block, blocks of 8
 // atoms in order): thread t sums partials t, t+512, ... in turn, then the fixed tree.
+// With out_dst (pinned host memory) the block then hands out_n results, the totals among
+// them, to the host: each copy launch after the step cost 2 us and a gap of 6 to 10 us.
 __global__ __launch_bounds__(kReduceThreads) void k_struct_finish(int nb, const double *part, double *e_out,
                                                                   double *virial_out, const int *flag_src,
-                                                                  int *flag_dst) {
+                                                                  int *flag_dst, const double *out_src,
+                                                                  double *out_dst, int out_n) {
     __shared__ double sred[10][kReduceThreads / 64];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     if (flag_dst && t < 4) flag_dst[t] = flag_src[t];
@@ -2228,12 +2252,16 @@ __global__ __launch_bounds__(kReduceThreads) void k_struct_finish(int nb, const 
         if (t == 0) e_out[0] = x;
         else virial_out[t - 1] = x;
     }
+    if (!out_dst) return;
+    __threadfence_block();
+    __syncthreads();
+    for (int i = t; i < out_n; i += kReduceThreads) out_dst[i] = out_src[i];
 }
 void launch_struct_finish(int N, const double *part, double *e_out, double *virial_out, hipStream_t s,
-                          const int *flag_src, int *flag_dst) {
+                          const int *flag_src, int *flag_dst, const double *out_src, double *out_dst, int out_n) {
     if (N > 0)
         hipLaunchKernelGGL(k_struct_finish, dim3(1), dim3(kReduceThreads), 0, s, cdiv(N, 8), part, e_out, virial_out,
-                           flag_src, flag_dst);
+                           flag_src, flag_dst, out_src, out_dst, out_n);
 }
 void launch_struct_reduce(int S, const int *atom_off, const double *local_e, const double *local_virial,
                           double *e_out, double *virial_out, hipStream_t s, const int *flag_src, int *flag_dst) {
