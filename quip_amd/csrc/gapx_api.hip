@@ -1320,7 +1320,11 @@ static int gemm_tune(gapx_model *m, Engine &eg, Coord &c, int nc, GemmTune &out,
     out = GemmTune();
     out.parts = gemm2_parts(nc, c.dim);
     const bool fusable = gp_f64_fused_supported(c.dim) && c.d_XsP.p;
-    if (fusable) out.f64parts = gp_f64_parts_default(nc, c.M);   // the default: the fused kernel
+    const bool tile = gp_f64_tile_serves(nc);
+    if (fusable) {   // the default: the fused kernel
+        out.f64tile = tile;
+        out.f64parts = tile ? gp_f64_tile_parts_default(nc, c.M) : gp_f64_parts_default(nc, c.M);
+    }
     if (!m->autotune || nc <= 0) return GAPX_OK;
     int bucket = 0;
     while ((1 << bucket) < nc) bucket++;
@@ -1376,14 +1380,14 @@ static int gemm_tune(gapx_model *m, Engine &eg, Coord &c, int nc, GemmTune &out,
     if (fusable) {   // the fused kernel (with its partial-G sum) against the two GEMMs
         float fbest = 1e30f;
         int fparts = 0;
-        for (int p = 1, prev = 0; p <= 8 && st == GAPX_OK; p *= 2) {
-            const int v = gp_f64_parts_valid(p, c.M);
+        for (int p = 1, prev = 0; p <= (tile ? 32 : 8) && st == GAPX_OK; p *= 2) {
+            const int v = tile ? gp_f64_tile_parts_valid(p, c.M) : gp_f64_parts_valid(p, c.M);
             if (v == prev) continue;
             prev = v;
             float t = 0;
             int nt = 0;
             st = timed([&] {
-                launch_gp_fused_f64(nc, c.M, c.dim, v, w.X.as<double>(), c.d_XsP.as<double>(), c.d_w.as<double>(),
+                launch_gp_fused_f64(tile, nc, c.M, c.dim, v, w.X.as<double>(), c.d_XsP.as<double>(), c.d_w.as<double>(),
                                     c.zeta, w.G.as<double>(), w.Gparts.as<double>(), w.e_part.as<double>(), &nt, s);
                 launch_gp_finish_f64(nc, c.dim, nt, w.Gparts.as<double>(), w.G.as<double>(), nt, nullptr, nullptr,
                                      nullptr, s);
@@ -1391,6 +1395,7 @@ static int gemm_tune(gapx_model *m, Engine &eg, Coord &c, int nc, GemmTune &out,
             if (st == GAPX_OK && t < fbest) { fbest = t; fparts = v; }
         }
         best.f64_ms = fbest;
+        best.f64tile = tile;
         best.f64parts = (st == GAPX_OK && fbest < best.g1_ms + best.g2_ms) ? fparts : 0;
     }
     hipEventDestroy(ea);
@@ -1801,10 +1806,11 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         mX = std::max(mX, (size_t)nc * c.dim * 8);
         mN = std::max(mN, (size_t)nc * 8);
         mC = std::max(mC, (size_t)nc * KLM * 8);
-        mE = std::max(mE, (size_t)nc * ((c.M + 31) / 32 + 1) * 8);
+        mE = std::max(mE, (size_t)nc * ((c.M + 31) / 32 + 32) * 8);   // a column per tile, chunk or part
         if (m->precision == GAPX_PREC_FP64) {
             mW = std::max(mW, (size_t)nc * c.M * 8);
-            mGp = std::max(mGp, (size_t)8 * nc * c.dim * 8);
+            const bool tile = gp_f64_fused_supported(c.dim) && gp_f64_tile_serves(nc);
+            mGp = std::max(mGp, (size_t)(tile ? 32 : 8) * nc * c.dim * 8);
         } else if (fused[k]) {
             size_t b = fused_scratch_bytes(m->precision, c, nc, 0);
             if (m->autotune && !noalloc) {   // the tuner's candidates
@@ -1940,7 +1946,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
             int ntile = 0;
             const bool f64fused = m->precision == GAPX_PREC_FP64 && grad && tu.f64parts > 0;
             if (f64fused) {   // K -> W -> G in one kernel
-                launch_gp_fused_f64(nc, c.M, c.dim, tu.f64parts, w.X.as<double>(), c.d_XsP.as<double>(),
+                launch_gp_fused_f64(tu.f64tile, nc, c.M, c.dim, tu.f64parts, w.X.as<double>(), c.d_XsP.as<double>(),
                                     c.d_w.as<double>(), c.zeta, w.G.as<double>(), w.Gparts.as<double>(),
                                     w.e_part.as<double>(), &ntile, s);
             } else if (m->precision == GAPX_PREC_FP64) {
@@ -2037,7 +2043,8 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         key.push_back(es);
         for (size_t k = 0; k < NCOORD; k++)
             key.insert(key.end(), {(long long)eg.h_centres[k].size(), tunes[k].g1, tunes[k].g2, tunes[k].parts,
-                                   tunes[k].fparts, tunes[k].g1lds, tunes[k].g2lds, tunes[k].f64parts});
+                                   tunes[k].fparts, tunes[k].g1lds, tunes[k].g2lds, tunes[k].f64parts,
+                                   tunes[k].f64tile});
         if (!eg.gexec || key != eg.gkey) {
             if (eg.gexec) {
                 hipGraphExecDestroy(eg.gexec);

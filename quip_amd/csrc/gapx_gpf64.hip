@@ -162,7 +162,147 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
 }
 
+// The same contraction for calls of few centres.  A chunk of 32 points costs a wavefront of
+// the kernel above 256 products of 64 cycles in a row (6.8 us), however few of its 16 centres
+// exist.  Here the four wavefronts of a block share 16 points x 16 centres: each forms K
+// over a quarter of the components, the quarters meet in LDS (always summed in the same
+// order), every wave turns them into W and adds W Xs for a quarter of G's columns: 32
+// products a wave and step (0.9 us; a step takes 2.1 us alone on its CU).  A block walks its
+// part of the points in steps of 16, the next points fetched into registers meanwhile; two
+// blocks on a CU fill each other's waits.  32 centres a block were slower at every size.
+template <int DK, int ZI>
+__global__ __launch_bounds__(256, 2) void k_gp_tile_f64(int nc, int M, int d, int ntiles, int tiles_per_part,
+                                                        const double *__restrict__ X, const double *__restrict__ XsP,
+                                                        const double *__restrict__ wvec, double zeta, int izeta,
+                                                        double *__restrict__ G, double *__restrict__ Gpart,
+                                                        double *__restrict__ e_part) {
+    constexpr int DP = 32 * DK;
+    constexpr int KW = 2 * DK;             // k-steps of K^T per wave
+    constexpr int QW = (2 * DK + 3) / 4;   // 16-column tiles of G per wave (the last wave's may not exist)
+    constexpr int LD = DP + 1;
+    __shared__ double xs[16 * LD];
+    __shared__ double xw[16];
+    __shared__ double red[4][4][64];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int c16 = lane & 15, g4 = lane >> 4;
+    const int row0 = blockIdx.x * 16;
+    const int part = blockIdx.y, nparts = gridDim.y;
+    const int t_beg = part * tiles_per_part, t_end = min(ntiles, t_beg + tiles_per_part);
+
+    double2_t pf[DK];
+    double pw = 0.0;
+    auto fetch = [&](int tile) {   // 16 rows of the padded sparse matrix
+        const double2_t *src = (const double2_t *)(XsP + (size_t)tile * 16 * DP);
+#pragma unroll
+        for (int u = 0; u < DK; u++) pf[u] = src[t + 256 * u];
+        const int sp = 16 * tile + t;
+        if (t < 16) pw = sp < M ? wvec[sp] : 0.0;
+    };
+    auto put = [&]() {
+#pragma unroll
+        for (int u = 0; u < DK; u++) {
+            const int idx = t + 256 * u;
+            const int r = idx / (DP / 2), c = (idx % (DP / 2)) * 2;
+            xs[r * LD + c] = pf[u][0];
+            xs[r * LD + c + 1] = pf[u][1];
+        }
+        if (t < 16) xw[t] = pw;
+    };
+    if (t_beg < t_end) fetch(t_beg);
+    double xf[KW];   // B operand of K^T: X[row][k] of the wave's quarter of the components
+#pragma unroll
+    for (int i = 0; i < KW; i++) {
+        const int row = row0 + c16, k = 4 * (wv * KW + i) + g4;
+        xf[i] = (row < nc && k < d) ? X[(size_t)row * d + k] : 0.0;
+    }
+    double4_t gacc[QW];
+#pragma unroll
+    for (int q = 0; q < QW; q++) gacc[q] = (double4_t){0.0, 0.0, 0.0, 0.0};
+    double esum = 0.0;
+    if (t_beg < t_end) put();
+    __syncthreads();
+    for (int tile = t_beg; tile < t_end; tile++) {
+        if (tile + 1 < t_end) fetch(tile + 1);
+        double4_t ka = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < KW; i++)
+            ka = __builtin_amdgcn_mfma_f64_16x16x4f64(xs[c16 * LD + 4 * (wv * KW + i) + g4], xf[i], ka, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; v++) red[wv][v][lane] = ka[v];
+        __syncthreads();
+        // element v: K[centre c16][sparse point 16 tile + g4 + 4 v]
+        double wf[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const double ws = xw[g4 + 4 * v];
+            const double kv = (red[0][v][lane] + red[1][v][lane]) + (red[2][v][lane] + red[3][v][lane]);
+            double kz1, kz;
+            if constexpr (ZI > 0) {
+                kz1 = 1.0;
+#pragma unroll
+                for (int q = 1; q < ZI; q++) kz1 *= kv;
+                kz = kz1 * kv;
+            } else if (izeta > 0) {
+                kz1 = 1.0;
+                for (int q = 1; q < izeta; q++) kz1 *= kv;
+                kz = kz1 * kv;
+            } else {
+                kz1 = pow(kv, zeta - 1.0);
+                kz = pow(kv, zeta);
+            }
+            esum += ws * kz;
+            wf[v] = ws * zeta * kz1;
+        }
+#pragma unroll
+        for (int q = 0; q < QW; q++) {
+            const int col = 16 * (wv * QW + q) + c16;   // past DP in a wave's missing tiles: not read
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const double b = col < DP ? xs[(4 * v + g4) * LD + col] : 0.0;
+                gacc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(wf[v], b, gacc[q], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+        if (tile + 1 < t_end) {
+            put();
+            __syncthreads();
+        }
+    }
+    // energy of centre c16 over this part: the four lane groups hold different sparse points
+    esum += __shfl_xor(esum, 16, 64);
+    esum += __shfl_xor(esum, 32, 64);
+    if (wv == 0 && g4 == 0 && row0 + c16 < nc) e_part[(size_t)(row0 + c16) * nparts + part] = esum;
+#pragma unroll
+    for (int q = 0; q < QW; q++) {
+        const int col = 16 * (wv * QW + q) + c16;
+        if (col >= d) continue;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int row = row0 + g4 + 4 * v;
+            if (row >= nc) continue;
+            if (nparts == 1) G[(size_t)row * d + col] = gacc[q][v];
+            else Gpart[((size_t)part * nc + row) * d + col] = gacc[q][v];
+        }
+    }
+}
+
 bool gp_f64_fused_supported(int d) { return d >= 1 && d <= 256; }
+
+// The 16-centre form serves up to 512 centres: on 253 components and 500 points it took 13 us
+// against 27 for 8 centres, 17 against 30 for 216 and 22 against 35 for 500; on 2000 points 21
+// against 76 (two GEMMs and their sums: 45) for 8, 36 against 81 (46) for 288, but at 997 62
+// against the GEMMs' 58.  Its parts are sums of 16 points, at most 32 of them (the partial G
+// rows are written and read once: 64 parts took longer at every size).
+bool gp_f64_tile_serves(int nc) { return nc <= 512; }
+int gp_f64_tile_parts_valid(int parts, int M) {
+    const int tiles = cdivf(M, 16);
+    parts = std::max(1, std::min({parts, tiles, 32}));
+    return cdivf(tiles, cdivf(tiles, parts));
+}
+// default: two blocks per CU
+int gp_f64_tile_parts_default(int nc, int M) {
+    return gp_f64_tile_parts_valid(512 / std::max(1, cdivf(nc, 16)), M);
+}
 
 int gp_f64_parts_valid(int parts, int M) {
     const int chunks = cdivf(M, F64_CH);
@@ -184,31 +324,32 @@ static int int_zeta_f(double z) {
     return (fabs(z - r) == 0.0 && r >= 1.0 && r <= 16.0) ? (int)r : 0;
 }
 
-void launch_gp_fused_f64(int nc, int M, int d, int parts_req, const double *X, const double *XsP,
+void launch_gp_fused_f64(bool tile, int nc, int M, int d, int parts_req, const double *X, const double *XsP,
                          const double *wvec, double zeta, double *G, double *Gparts, double *e_part, int *ntile_out,
                          hipStream_t s) {
-    const int chunks = cdivf(M, F64_CH);
-    const int parts = gp_f64_parts_valid(parts_req, M);
-    const int per = cdivf(chunks, parts);
+    const int steps = cdivf(M, tile ? 16 : F64_CH);
+    const int parts = tile ? gp_f64_tile_parts_valid(parts_req, M) : gp_f64_parts_valid(parts_req, M);
+    const int per = cdivf(steps, parts);
     *ntile_out = parts;
     if (nc <= 0) return;
     const int DK = (d + 31) / 32;
-    dim3 grid(cdivf(nc, 64), parts);
+    const dim3 grid(cdivf(nc, tile ? 16 : 64), parts);
     const int iz = int_zeta_f(zeta);
-#define GPF(K)                                                                                                  \
-    case K:                                                                                                     \
-        if (iz == 4)                                                                                            \
-            hipLaunchKernelGGL((k_gp_fused_f64<K, 4>), grid, dim3(256), 0, s, nc, M, d, chunks, per, X, XsP, wvec, \
-                               zeta, iz, G, Gparts, e_part);                                                    \
-        else                                                                                                    \
-            hipLaunchKernelGGL((k_gp_fused_f64<K, 0>), grid, dim3(256), 0, s, nc, M, d, chunks, per, X, XsP, wvec, \
-                               zeta, iz, G, Gparts, e_part);                                                    \
+#define GPF1(F, K, Z)                                                                                              \
+    hipLaunchKernelGGL((F<K, Z>), grid, dim3(256), 0, s, nc, M, d, steps, per, X, XsP, wvec, zeta, iz, G, Gparts, e_part)
+#define GPF(K)                                                        \
+    case K:                                                           \
+        if (tile && iz == 4) GPF1(k_gp_tile_f64, K, 4);               \
+        else if (tile) GPF1(k_gp_tile_f64, K, 0);                     \
+        else if (iz == 4) GPF1(k_gp_fused_f64, K, 4);                 \
+        else GPF1(k_gp_fused_f64, K, 0);                              \
         break;
     switch (DK) {
         GPF(1) GPF(2) GPF(3) GPF(4) GPF(5) GPF(6) GPF(7) GPF(8)
         default: return;
     }
 #undef GPF
+#undef GPF1
 }
 
 }  // namespace gapx

@@ -114,6 +114,7 @@ struct GemmTune {
     // split GEMMs' tiles (-1 = the default rule, 0 = 64 x 64, 1 = 128 x 128 LDS tiles)
     int fparts = 0, g1lds = -1, g2lds = -1;
     // FP64: sparse-point parts of the fused GP kernel (0 = the two GEMMs) and its time
+    bool f64tile = false;   // ... in its form for few centres
     int f64parts = 0;
     float f64_ms = 0;
 };

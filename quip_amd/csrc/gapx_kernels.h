@@ -160,7 +160,11 @@ void launch_gemm2_f64(int cfg, int parts, int nc, int M, int d, const double *W,
 bool gp_f64_fused_supported(int d);
 int gp_f64_parts_default(int nc, int M);
 int gp_f64_parts_valid(int parts, int M);
-void launch_gp_fused_f64(int nc, int M, int d, int parts_req, const double *X, const double *XsP,
+// tile: the form for few centres, whose parts follow rules of their own
+bool gp_f64_tile_serves(int nc);
+int gp_f64_tile_parts_default(int nc, int M);
+int gp_f64_tile_parts_valid(int parts, int M);
+void launch_gp_fused_f64(bool tile, int nc, int M, int d, int parts_req, const double *X, const double *XsP,
                          const double *wvec, double zeta, double *G, double *Gparts, double *e_part, int *ntile_out,
                          hipStream_t s);
 void launch_sum_parts_f64(int nc, int d, int parts, const double *Gparts, double *G, hipStream_t s);
