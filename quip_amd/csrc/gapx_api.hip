@@ -594,7 +594,7 @@ void gapx::reset_arena_views(Engine &eg) {
                     &w.nb_r, &w.nb_d, &w.pairF, &w.pairE, &w.esite, &w.X, &w.norm, &w.cbuf, &w.W, &w.Wf, &w.e_part,
                     &w.G, &w.Gparts, &w.split_ws, &w.f, &w.le, &w.lv, &w.e, &w.vir, &w.minmax, &w.last_pos,
                     &w.skin_flags, &w.cmask, &w.t1_j, &w.t1_shift, &w.t1_r, &w.t2_i, &w.t2_k, &w.nl_flags, &w.eatom,
-                    &w.vK, &w.vk, &w.vV, &w.Gv, &w.pairFv, &w.pairVE, &w.varsite, &w.hout,
+                    &w.vK, &w.vk, &w.vV, &w.vrow, &w.Gv, &w.pairFv, &w.pairVE, &w.varsite, &w.hout,
                     &w.spart})
         b->drop_view();
     for (auto *v : {&w.centres, &w.var_inst, &w.cut2_inst})
@@ -1839,7 +1839,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
     CHK(w.esite.ensure((size_t)(N + 1) * 8));
     if (opt && opt->d_epc) CHK(w.eatom.ensure((size_t)(N + 1) * 8));
     if (want_var) {
-        CHK(w.vK.ensure(mV)); CHK(w.vk.ensure(mV)); CHK(w.vV.ensure(mV));
+        CHK(w.vK.ensure(mV)); CHK(w.vk.ensure(mV)); CHK(w.vV.ensure(mV)); CHK(w.vrow.ensure(mN));
         CHK(w.Gv.ensure(mX));
         CHK(w.pairFv.ensure((size_t)(P + 1) * 24));
         CHK(w.pairVE.ensure((size_t)(P + 1) * 8));
@@ -1980,15 +1980,15 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
             if (d_epc) launch_sum_fixed((size_t)nc * ntile, w.e_part.as<double>(), d_epc + k, s);
             if (marks) { tm.stage(1, t0, t1); tm.stage(2, t1, t2); }
             if (want_var) {   // FP64 whatever the GEMM precision
-                launch_gemm_nt_f64(nc, c.M, c.dim, w.X.as<double>(), c.d_Xs.as<double>(), w.vK.as<double>(), s);
-                launch_var_cov(nc, c.M, w.vK.as<double>(), d2, c.zeta, w.vk.as<double>(), s);
-                launch_gemm_nn_f64(nc, c.M, c.M, w.vk.as<double>(), c.d_Cinv.as<double>(), w.vV.as<double>(), s);
+                launch_var_k(nc, c.M, c.dim, w.X.as<double>(), c.d_Xs.as<double>(), d2, c.zeta, w.vK.as<double>(),
+                             w.vk.as<double>(), s);
+                launch_var_v(nc, c.M, w.vk.as<double>(), c.d_Cinv.as<double>(), w.vV.as<double>(), s);
                 launch_var_rows(nc, c.M, c.dim, w.X.as<double>(), w.vK.as<double>(), w.vk.as<double>(),
                                 w.vV.as<double>(), d2, c.zeta, centres, w.var_inst[k].as<double>(),
-                                w.varsite.as<double>(), s);
+                                w.varsite.as<double>(), w.vrow.as<double>(), s);
                 if (want_vgrad) {
-                    launch_gemm_nn_f64(nc, c.M, c.dim, w.vV.as<double>(), c.d_Xs.as<double>(), w.Gv.as<double>(), s);
-                    launch_var_self_grad(nc, c.dim, w.X.as<double>(), d2, c.zeta, w.Gv.as<double>(), s);
+                    launch_var_grad(nc, c.M, c.dim, w.vV.as<double>(), c.d_Xs.as<double>(), w.vrow.as<double>(),
+                                    w.X.as<double>(), w.Gv.as<double>(), s);
                     launch_soap_bwd(sp, nc, centres, w.Z.as<int>(), w.nb_off.as<int>(), w.nb_j.as<int>(),
                                     w.nb_r.as<double>(), w.nb_d.as<double>(), w.X.as<double>(), w.Gv.as<double>(),
                                     w.norm.as<double>(), w.cbuf.as<double>(), w.pairFv.as<double>(), shared_pairs(k), s);

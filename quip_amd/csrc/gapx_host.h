@@ -171,7 +171,7 @@ struct Workspace {
     DBuf eatom;                  // per-atom distance_2b energies of one coordinate (energy_per_coordinate)
     // GAP variance: K, k = delta^2 K^zeta, V = k Cinv (each nc x M), per-centre G of the
     // variance, pair sums, per-atom variances; per coordinate the instance variances
-    DBuf vK, vk, vV, Gv, pairFv, pairVE, varsite;
+    DBuf vK, vk, vV, vrow, Gv, pairFv, pairVE, varsite;
     std::vector<DBuf> var_inst, cut2_inst;
     DBuf hout;                   // the results a host-buffer call asked for, one after the other
 };

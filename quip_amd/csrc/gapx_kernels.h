@@ -218,18 +218,20 @@ void launch_sum_fixed(size_t n, const double *v, double *out, hipStream_t s);
 
 // GAP variance (projected-process estimate), FP64.
 // C = A (rows x kd) . B^T (cols x kd), and C = A (rows x kd) . B (kd x cols), no epilogue
-void launch_gemm_nn_f64(int rows, int kd, int cols, const double *A, const double *B, double *C, hipStream_t s);
-void launch_gemm_nt_f64(int rows, int cols, int kd, const double *A, const double *B, double *C, hipStream_t s);
-// kv[i][s] = delta2 K[i][s]^zeta
-void launch_var_cov(int nc, int M, const double *K, double delta2, double zeta, double *kv, hipStream_t s);
+// The variance's products: K = X Xs^T with kv = delta2 K^zeta, V = kv Cinv, and the gradient
+// rows Gv_i = V_i Xs + srow_i x_i
+void launch_var_k(int nc, int M, int d, const double *X, const double *Xs, double delta2, double zeta, double *K,
+                  double *kv, hipStream_t s);
+void launch_var_v(int nc, int M, const double *kv, const double *Cinv, double *V, hipStream_t s);
+void launch_var_grad(int nc, int M, int d, const double *V, const double *Xs, const double *srow, const double *X,
+                     double *Gv, hipStream_t s);
 // Per centre row i (V = kv . Cinv): var_i = delta2 (x_i.x_i)^zeta - sum_s kv_is V_is, then
 // V_is <- -2 zeta delta2 K_is^(zeta-1) V_is (the variance's weight on X_s);
-// var_inst[i] = var_i and varsite[centres[i]] += var_i.
+// var_inst[i] = var_i, varsite[centres[i]] += var_i and srow[i] = 2 zeta delta2
+// (x_i.x_i)^(zeta-1), the factor of x_i in the gradient of k(x, x).
 void launch_var_rows(int nc, int M, int d, const double *X, const double *K, const double *kv, double *V,
                      double delta2, double zeta, const int *centres, double *var_inst, double *varsite,
-                     hipStream_t s);
-// Gv_i += 2 zeta delta2 (x_i.x_i)^(zeta-1) x_i  (the gradient of k(x, x))
-void launch_var_self_grad(int nc, int d, const double *X, double delta2, double zeta, double *Gv, hipStream_t s);
+                     double *srow, hipStream_t s);
 // distance_2b variance with the ard_se kernel (M <= kMaxVarSparse): per directed pair p of a
 // descriptor instance, var = delta2 - k^T Cinv k; pairVE[p] += var fc^2, pairFv[p] += d(var fc^2)/dr u;
 // var_inst[p] = var and cut2_inst[p] = fc^2 (NaN-filled by the caller for non-instances).

@@ -1597,7 +1597,17 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 
 constexpr int GPAD = 1;   // odd: the 16 k-rows one stash write touches fall on distinct bank pairs
 
-// C = A . B (+ fused GP epilogue).  A is row-major (rows x K, k contiguous);
+__device__ __forceinline__ double powz(double x, double zeta, int iz) {
+    if (iz > 0) {
+        double r = 1.0;
+        for (int q = 0; q < iz; q++) r *= x;
+        return r;
+    }
+    if (iz == 0 && zeta == 0.0) return 1.0;
+    return pow(x, zeta);
+}
+
+// C = A . B; EPI 0: no epilogue, 1: the GP's, 2 and 3: the variance's (see k_gemm_f64_wave).  A is row-major (rows x K, k contiguous);
 // B is row-major (cols x K) when BT, else (K x cols).  4 wavefronts in a 2x2
 // grid, each owning 32 x 32 outputs, block tile 64 x 64, k tiles of 16.
 // The next k tile is fetched into registers while the current one feeds the
@@ -1607,10 +1617,11 @@ constexpr int GPAD = 1;   // odd: the 16 k-rows one stash write touches fall on 
 // The occupancy hint keeps the accumulators in ordinary VGPRs for the whole kernel:
 // without it the compiler places them in AGPRs and copies all of them out and back
 // around every k tile.
-template <bool BT, bool EPI>
+template <bool BT, int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_gemm_f64(
     int Mr, int Nc, int Kd, int kchunk, const double *__restrict__ A, const double *__restrict__ B,
-    double *__restrict__ C, const double *__restrict__ wvec, double zeta, int izeta, double *__restrict__ e_part) {
+    double *__restrict__ C, const double *__restrict__ wvec, double zeta, int izeta, double *__restrict__ e_part,
+    double delta2, double *__restrict__ kv2, const double *__restrict__ srow, const double *__restrict__ X) {
     constexpr int WM = 2, WN = 2, GBK = 16;
     constexpr int BM = 32 * WM, BN = 32 * WN;
     constexpr int AL = BM * GBK / 256;   // A elements per thread per k tile
@@ -1696,12 +1707,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         for (int j = 0; j < WN; j++) {
             const int col = n0 + wn * 16 * WN + j * 16 + (lane & 15);
             double wv = 0.0;
-            if (EPI) wv = (col < Nc) ? wvec[col] : 0.0;
+            if (EPI == 1) wv = (col < Nc) ? wvec[col] : 0.0;
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = m0 + wm * 16 * WM + i * 16 + (lane >> 4) + 4 * v;
                 double kv = acc[i][j][v];
-                if (EPI) {
+                if (EPI == 1) {
                     double kz1, kz;
                     if (izeta > 0) {
                         kz1 = 1.0;
@@ -1714,10 +1725,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                     rowsum[i][v] += wv * kz;
                     kv = wv * zeta * kz1;
                 }
-                if ((!EPI || store) && row < Mr && col < Nc) C[(size_t)row * Nc + col] = kv;
+                if ((EPI != 1 || store) && row < Mr && col < Nc) {
+                    const size_t q = (size_t)row * Nc + col;
+                    if (EPI == 3) kv += srow[row] * X[q];
+                    C[q] = kv;
+                    if (EPI == 2) kv2[q] = delta2 * powz(kv, zeta, izeta);
+                }
             }
         }
-    if (EPI) {
+    if (EPI == 1) {
 #pragma unroll
         for (int i = 0; i < WM; i++)
 #pragma unroll
@@ -1753,8 +1769,9 @@ void launch_gemm1_f64(int cfg, int nc, int M, int d, const double *X, const doub
         launch_gemm1_f64_stream(cfg, nc, M, d, X, Xs, wvec, zeta, W, e_part, s);
         return;
     }
-    hipLaunchKernelGGL((k_gemm_f64<true, true>), dim3(cdiv(nc, 64), cdiv(M, 64)), dim3(256), 0, s, nc, M, d, d, X, Xs, W,
-                       wvec, zeta, int_zeta(zeta), e_part);
+    hipLaunchKernelGGL((k_gemm_f64<true, 1>), dim3(cdiv(nc, 64), cdiv(M, 64)), dim3(256), 0, s, nc, M, d, d, X, Xs, W,
+                       wvec, zeta, int_zeta(zeta), e_part, 0.0, (double *)nullptr, (const double *)nullptr,
+                       (const double *)nullptr);
 }
 
 // split-K partial sums, reduced in a fixed order
@@ -1782,8 +1799,9 @@ void launch_gemm2_f64(int cfg, int parts, int nc, int M, int d, const double *W,
         launch_gemm2_f64_stream(cfg, parts, nc, M, d, W, Xs, out, s);
     } else {
         const int kchunk = (cdiv(M, parts) + 15) / 16 * 16;
-        hipLaunchKernelGGL((k_gemm_f64<false, false>), dim3(cdiv(nc, 64), cdiv(d, 64), parts), dim3(256), 0, s, nc, d, M,
-                           kchunk, W, Xs, out, (const double *)nullptr, 0.0, 0, (double *)nullptr);
+        hipLaunchKernelGGL((k_gemm_f64<false, 0>), dim3(cdiv(nc, 64), cdiv(d, 64), parts), dim3(256), 0, s, nc, d, M,
+                           kchunk, W, Xs, out, (const double *)nullptr, 0.0, 0, (double *)nullptr, 0.0, (double *)nullptr,
+                           (const double *)nullptr, (const double *)nullptr);
     }
     if (parts > 1) launch_sum_parts_f64(nc, d, parts, Gparts, G, s);
 }
@@ -1928,35 +1946,79 @@ void launch_sum_fixed(size_t n, const double *v, double *out, hipStream_t s) {
 //   var(x) = k(x,x) - k_x^T (K_MM + reg I)^-1 k_x,  k_x[s] = delta^2 kernel(x, X_s)
 // Cinv = (K_MM + reg I)^-1 is formed on the host when the model is asked for it.
 // ----------------------------------------------------------------------------
-void launch_gemm_nt_f64(int rows, int cols, int kd, const double *A, const double *B, double *C, hipStream_t s) {
-    if (rows > 0 && cols > 0)
-        hipLaunchKernelGGL((k_gemm_f64<true, false>), dim3(cdiv(rows, 64), cdiv(cols, 64)), dim3(256), 0, s, rows, cols, kd,
-                           kd, A, B, C, (const double *)nullptr, 0.0, 0, (double *)nullptr);
-}
-void launch_gemm_nn_f64(int rows, int kd, int cols, const double *A, const double *B, double *C, hipStream_t s) {
-    if (rows > 0 && cols > 0)
-        hipLaunchKernelGGL((k_gemm_f64<false, false>), dim3(cdiv(rows, 64), cdiv(cols, 64)), dim3(256), 0, s, rows, cols,
-                           kd, kd, A, B, C, (const double *)nullptr, 0.0, 0, (double *)nullptr);
-}
-
-__device__ __forceinline__ double powz(double x, double zeta, int iz) {
-    if (iz > 0) {
-        double r = 1.0;
-        for (int q = 0; q < iz; q++) r *= x;
-        return r;
+constexpr long kVarWaveTiles = 1024;   // 16 x 16 tiles: the limit of k_gemm_f64_wave
+// The products of the variance: C = A B' (NT) or A B (NN) with the epilogues EPI 0: none,
+// 2: also kv = delta2 C^zeta, 3: C + srow[row] X[row][col].  Few tiles: a wavefront holds 16 x 16
+// of C and loads its operands from memory in their MFMA layouts, 32 k-steps at a time, each
+// reloaded after its product; no LDS, no barriers.  The k-steps follow one another as in
+// k_gemm_f64, so results are bitwise its own: the variance magnifies their last bits.
+// 216 x 500 x 500 (k_gemm_f64 on 32 blocks, a microsecond per staged k tile): 32 -> 18 us,
+// 216 x 500 x 253: 17 -> 10.  Up to 1024 tiles, one per SIMD (500 x 500 x 500: 32 -> 19); past
+// that the operands' path is full: 2016 tiles, k 500, 34 to 42 us against k_gemm_f64's 32.
+template <bool BT, int EPI>
+__global__ __launch_bounds__(256) void k_gemm_f64_wave(int Mr, int Nc, int Kd, const double *__restrict__ A,
+                                                       const double *__restrict__ B, double *__restrict__ C,
+                                                       double delta2, double zeta, int iz, double *__restrict__ kv,
+                                                       const double *__restrict__ srow,
+                                                       const double *__restrict__ X) {
+    constexpr int U = 32;   // k-steps in flight
+    const int lane = threadIdx.x & 63, c16 = lane & 15, g4 = lane >> 4;
+    const int m0 = blockIdx.x * 16, n0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * 16;
+    if (n0 >= Nc) return;
+    // rows and columns past the edge read those of the edge; what they give is not stored
+    const double *pa = A + (size_t)min(m0 + c16, Mr - 1) * Kd;
+    const double *pb = BT ? B + (size_t)min(n0 + c16, Nc - 1) * Kd : B + min(n0 + c16, Nc - 1);
+    double fa[U], fb[U];
+    auto load = [&](int u, int k) {   // past Kd: its last element, replaced by zero where it is used
+        k = min(k, Kd - 1);
+        fa[u] = pa[k];
+        fb[u] = BT ? pb[k] : pb[(size_t)k * Nc];
+    };
+#pragma unroll
+    for (int u = 0; u < U; u++) load(u, 4 * u + g4);
+    double4_t acc = {0.0, 0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < Kd; k0 += 4 * U) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = k0 + 4 * u + g4;
+            const double a = k < Kd ? fa[u] : 0.0, b = k < Kd ? fb[u] : 0.0;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+            load(u, k + 4 * U);
+        }
     }
-    if (iz == 0 && zeta == 0.0) return 1.0;
-    return pow(x, zeta);
+    const int col = n0 + c16;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int row = m0 + g4 + 4 * v;
+        if (row >= Mr || col >= Nc) continue;
+        const size_t q = (size_t)row * Nc + col;
+        double x = acc[v];
+        if (EPI == 3) x += srow[row] * X[q];
+        C[q] = x;
+        if (EPI == 2) kv[q] = delta2 * powz(x, zeta, iz);
+    }
 }
-
-__global__ void k_var_cov(size_t n, const double *K, double delta2, double zeta, int iz, double *kv) {
-    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < n) kv[q] = delta2 * powz(K[q], zeta, iz);
+template <bool BT, int EPI>
+static void gemm_var_go(int Mr, int Nc, int Kd, const double *A, const double *B, double *C, double delta2,
+                        double zeta, int iz, double *kv, const double *srow, const double *X, hipStream_t s) {
+    if (Mr <= 0 || Nc <= 0) return;
+    if ((long)cdiv(Mr, 16) * cdiv(Nc, 16) <= kVarWaveTiles)
+        hipLaunchKernelGGL((k_gemm_f64_wave<BT, EPI>), dim3(cdiv(Mr, 16), cdiv(Nc, 64)), dim3(256), 0, s, Mr, Nc, Kd,
+                           A, B, C, delta2, zeta, iz, kv, srow, X);
+    else
+        hipLaunchKernelGGL((k_gemm_f64<BT, EPI>), dim3(cdiv(Mr, 64), cdiv(Nc, 64)), dim3(256), 0, s, Mr, Nc, Kd, Kd, A,
+                           B, C, (const double *)nullptr, zeta, iz, (double *)nullptr, delta2, kv, srow, X);
 }
-void launch_var_cov(int nc, int M, const double *K, double delta2, double zeta, double *kv, hipStream_t s) {
-    const size_t n = (size_t)nc * M;
-    if (n) hipLaunchKernelGGL(k_var_cov, dim3(cdiv((long)n, 256)), dim3(256), 0, s, n, K, delta2, zeta,
-                              int_zeta(zeta), kv);
+void launch_var_k(int nc, int M, int d, const double *X, const double *Xs, double delta2, double zeta, double *K,
+                  double *kv, hipStream_t s) {
+    gemm_var_go<true, 2>(nc, M, d, X, Xs, K, delta2, zeta, int_zeta(zeta), kv, nullptr, nullptr, s);
+}
+void launch_var_v(int nc, int M, const double *kv, const double *Cinv, double *V, hipStream_t s) {
+    gemm_var_go<false, 0>(nc, M, M, kv, Cinv, V, 0.0, 0.0, 0, nullptr, nullptr, nullptr, s);
+}
+void launch_var_grad(int nc, int M, int d, const double *V, const double *Xs, const double *srow, const double *X,
+                     double *Gv, hipStream_t s) {
+    gemm_var_go<false, 3>(nc, d, M, V, Xs, Gv, 0.0, 0.0, 0, nullptr, srow, X, s);
 }
 
 __device__ __forceinline__ double wave_sum_v(double v) {   // fixed butterfly over the 64 lanes
@@ -1967,7 +2029,8 @@ __device__ __forceinline__ double wave_sum_v(double v) {   // fixed butterfly ov
 // one wavefront per centre row
 __global__ __launch_bounds__(256) void k_var_rows(int nc, int M, int d, const double *X, const double *K,
                                                   const double *kv, double *V, double delta2, double zeta, int iz,
-                                                  int iz1, const int *centres, double *var_inst, double *varsite) {
+                                                  int iz1, const int *centres, double *var_inst, double *varsite,
+                                                  double *srow) {
     const int lane = threadIdx.x & 63;
     const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (i >= nc) return;
@@ -1989,32 +2052,15 @@ __global__ __launch_bounds__(256) void k_var_rows(int nc, int M, int d, const do
         const double var = delta2 * powz(xx, zeta, iz) - kck;
         var_inst[i] = var;
         varsite[centres[i]] += var;
+        srow[i] = 2.0 * zeta * delta2 * powz(xx, zeta - 1.0, iz1);   // the gradient's own-term factor
     }
 }
 void launch_var_rows(int nc, int M, int d, const double *X, const double *K, const double *kv, double *V,
                      double delta2, double zeta, const int *centres, double *var_inst, double *varsite,
-                     hipStream_t s) {
+                     double *srow, hipStream_t s) {
     if (nc > 0)
         hipLaunchKernelGGL(k_var_rows, dim3(cdiv(nc, 4)), dim3(256), 0, s, nc, M, d, X, K, kv, V, delta2, zeta,
-                           int_zeta(zeta), int_zeta(zeta - 1.0), centres, var_inst, varsite);
-}
-
-__global__ __launch_bounds__(256) void k_var_self_grad(int nc, int d, const double *X, double delta2, double zeta,
-                                                       int iz1, double *Gv) {
-    const int lane = threadIdx.x & 63;
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= nc) return;
-    const double *x = X + (size_t)i * d;
-    double xx = 0.0;
-    for (int q = lane; q < d; q += 64) xx += x[q] * x[q];
-    xx = wave_sum_v(xx);
-    const double g = 2.0 * zeta * delta2 * powz(xx, zeta - 1.0, iz1);
-    for (int q = lane; q < d; q += 64) Gv[(size_t)i * d + q] += g * x[q];
-}
-void launch_var_self_grad(int nc, int d, const double *X, double delta2, double zeta, double *Gv, hipStream_t s) {
-    if (nc > 0)
-        hipLaunchKernelGGL(k_var_self_grad, dim3(cdiv(nc, 4)), dim3(256), 0, s, nc, d, X, delta2, zeta,
-                           int_zeta(zeta - 1.0), Gv);
+                           int_zeta(zeta), int_zeta(zeta - 1.0), centres, var_inst, varsite, srow);
 }
 
 // one thread per first atom over its pairs; the covariance vector sits in a per-lane array
@@ -2065,29 +2111,33 @@ void launch_d2b_var(int N, const int *Z, int Z1, int Z2, double rc, double ctw, 
                            theta, Cinv, nb_off, nb_j, nb_r, nb_d, pairFv, pairVE, var_inst, cut2_inst, mask);
 }
 
-__global__ void k_gather_var(int N, const int *nb_off, const int *nb_rev, const double *pairFv,
-                             const double *pairVE, const double *varsite, double *gvg, double *lgv) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ double half_sum_g(double v) {   // sum over the 32 lanes of a half-wave
+    for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+// a half-wave per atom, lanes over its pairs (216 atoms, a thread each: 17.6 us)
+__global__ __launch_bounds__(256) void k_gather_var(int N, const int *nb_off, const int *nb_rev, const double *pairFv,
+                                                    const double *pairVE, const double *varsite, double *gvg,
+                                                    double *lgv) {
+    const int hl = threadIdx.x & 31, j = blockIdx.x * 8 + (threadIdx.x >> 5);
     if (j >= N) return;
-    double g0 = 0.0, g1 = 0.0, g2 = 0.0, ve = 0.0;
-    for (int q = nb_off[j]; q < nb_off[j + 1]; q++) {
+    double g[3] = {0.0, 0.0, 0.0}, ve = 0.0;
+    for (int q = nb_off[j] + hl; q < nb_off[j + 1]; q += 32) {
         const int r = nb_rev[q];
-        g0 += pairFv[3 * q] - pairFv[3 * r];
-        g1 += pairFv[3 * q + 1] - pairFv[3 * r + 1];
-        g2 += pairFv[3 * q + 2] - pairFv[3 * r + 2];
+#pragma unroll
+        for (int k = 0; k < 3; k++) g[k] += pairFv[3 * q + k] - pairFv[3 * r + k];
         if (pairVE) ve += pairVE[q] + pairVE[r];
     }
-    if (gvg) {
-        gvg[3 * (size_t)j] = -g0;
-        gvg[3 * (size_t)j + 1] = -g1;
-        gvg[3 * (size_t)j + 2] = -g2;
-    }
-    if (lgv) lgv[j] = varsite[j] + 0.5 * ve;
+#pragma unroll
+    for (int k = 0; k < 3; k++) g[k] = half_sum_g(g[k]);
+    ve = half_sum_g(ve);
+    if (gvg && hl < 3) gvg[3 * (size_t)j + hl] = -(hl == 0 ? g[0] : (hl == 1 ? g[1] : g[2]));
+    if (lgv && hl == 0) lgv[j] = varsite[j] + 0.5 * ve;
 }
 void launch_gather_var(int N, const int *nb_off, const int *nb_rev, const double *pairFv, const double *pairVE,
                        const double *varsite, double *gvg, double *lgv, hipStream_t s) {
     if (N > 0)
-        hipLaunchKernelGGL(k_gather_var, dim3(cdiv(N, 128)), dim3(128), 0, s, N, nb_off, nb_rev, pairFv, pairVE,
+        hipLaunchKernelGGL(k_gather_var, dim3(cdiv(N, 8)), dim3(256), 0, s, N, nb_off, nb_rev, pairFv, pairVE,
                            varsite, gvg, lgv);
 }
 
@@ -2097,10 +2147,6 @@ void launch_gather_var(int N, const int *nb_off, const int *nb_rev, const double
 // local_e_j = e_site + (pairE[q] + pairE[rev q])/2 + e0(Z_j); block partial sums.
 // ----------------------------------------------------------------------------
 constexpr int GATHER_BS = 256;   // 4 wavefronts, two atoms each (a half-wave per atom)
-__device__ __forceinline__ double half_sum_g(double v) {   // sum over the 32 lanes of a half-wave
-    for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
 __global__ __launch_bounds__(GATHER_BS) void k_gather(int N, const int *Z, const double *e0, double E_scale,
                                                       const int *nb_off, const int *nb_rev, const double *nb_d,
                                                       const double *pairF, const double *pairE, const double *esite,
