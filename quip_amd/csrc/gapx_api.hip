@@ -536,6 +536,7 @@ int gapx::new_engine(gapx_model *m, std::unique_ptr<Engine> &out) {
     std::unique_ptr<Engine> e(new Engine());
     hipError_t he = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
     if (he != hipSuccess) return fail(GAPX_E_DEVICE, "hipStreamCreate: %s", hipGetErrorString(he));
+    e->ctl.coherent = true;   // the overlap flag of a reused list is stored there by its kernel
     e->ws.centres.resize(m->coords.size());
     e->ws.var_inst.resize(m->coords.size());
     e->ws.cut2_inst.resize(m->coords.size());
@@ -1196,6 +1197,7 @@ static void update_nl_caps(Engine &eg, const int *flags) {
 static int build_nl(gapx_model *m, Engine &eg, int S, const int *atom_off, const double *d_pos, const double *h_pos,
                     const double *lats, const int *pbcs, double cutoff, int *P_out) {
     NLPlan pl;
+    eg.nl_valid = false;   // the tables of a list kept for reuse go
     CHK(nl_prepare(m, eg, S, atom_off, d_pos, h_pos, lats, pbcs, cutoff, false, pl));
     Workspace &w = eg.ws;
     hipStream_t s = eg.stream;
@@ -1218,52 +1220,90 @@ static int build_nl(gapx_model *m, Engine &eg, int S, const int *atom_off, const
     return GAPX_OK;
 }
 
+static int overlap_error() { return fail(GAPX_E_GEOMETRY, "calc_dists: two atoms overlap exactly"); }
+constexpr int kHostMoveAtoms = 32768;   // their host pass stays below the read-back it replaces
+
+// Whether host positions alone tell that no atom of one structure has moved by half the skin
+// since the positions `last`: the plain displacements are below it, and too short for any
+// fractional component to round to another image.  A pass over 997 atoms takes 1 us; the
+// device's test, its read-back and the empty stream behind it took 50.  False leaves the
+// decision to the device.
+static bool moved_little(const double *pos, const double *last, int N, const double *lat, double half_skin) {
+    double gi[9];
+    inv3(lat, gi);
+    for (int a = 0; a < 3; a++)
+        if (half_skin * std::sqrt(gi[a] * gi[a] + gi[3 + a] * gi[3 + a] + gi[6 + a] * gi[6 + a]) >= 0.49) return false;
+    double mx = 0.0;
+    for (int i = 0; i < N; i++) {
+        const double x = pos[3 * i] - last[3 * i], y = pos[3 * i + 1] - last[3 * i + 1], z = pos[3 * i + 2] - last[3 * i + 2];
+        const double r2 = x * x + y * y + z * z;
+        if (!(r2 < 1e300)) return false;   // not finite
+        mx = std::max(mx, r2);
+    }
+    return mx < half_skin * half_skin * (1.0 - 1e-9);
+}
+
 // calc_connect with skin reuse (Connection.f95:1085-1127): with a cutoff above the
 // model's (a skin), a list built for the same structures, cutoff and lattices is
 // kept while no atom has moved by half the skin since that build; its distances
-// are then recomputed as calc_dists does (Connection.f95:1321-1445) and the full
-// per-atom view re-formed.  The displacement test and the distances run in one
-// pass and are read back with one synchronisation, as the rebuild's count is.
+// are then recomputed as calc_dists does (Connection.f95:1321-1445) with the full
+// per-atom view, whose kernel also clears the step's accumulators (*cleared).
+// Host calls of one structure decide on their own positions where those suffice and
+// read nothing back; eg.overlap is then looked at with the results.  Otherwise the
+// displacement test and the view run in one pass, read back with one synchronisation.
 static int connect(gapx_model *m, Engine &eg, int S, const int *atom_off, const double *d_pos, const double *h_pos,
-                   const double *lats, const int *pbcs, double cutoff, int *P_out) {
+                   const double *lats, const int *pbcs, double cutoff, bool has_d2b, int *P_out, bool *cleared) {
     Workspace &w = eg.ws;
     hipStream_t s = eg.stream;
     const int N = atom_off[S];
     const double skin = cutoff - m->cutoff;
     eg.last_rebuilt = true;
+    *cleared = false;
     if (skin > 0 && m->nl_reuse && eg.nl_valid && eg.nl_cut == cutoff && (int)eg.nl_pbcs.size() == 3 * S &&
         std::equal(lats, lats + 9 * S, eg.nl_lats.begin()) && std::equal(pbcs, pbcs + 3 * S, eg.nl_pbcs.begin())) {
-        CHK(w.skin_flags.ensure(64));
-        launch_fill_i32(w.skin_flags.as<int>(), 4, 0, s);
-        unsigned long long *md = (unsigned long long *)w.skin_flags.p;
-        int *ov = w.skin_flags.as<int>() + 2;
-        launch_nl_skin_check(N, d_pos, w.last_pos.as<double>(), w.geo.as<NLGeom>(), w.sid.as<int>(),
-                             w.n1_off.as<int>(), w.n1_j.as<int>(), w.n1_shift.as<int>(), w.n1_r.as<double>(), md, ov,
-                             s);
+        const size_t P = 2 * (size_t)eg.n1_total_last;
+        CHK(w.pairF.ensure((P + 1) * 24));
+        CHK(w.pairE.ensure((P + 1) * 8));
+        CHK(w.esite.ensure((size_t)(N + 1) * 8));
         CHK(eg.ctl.ensure(64));
-        HIPCHK(hipMemcpyAsync(eg.ctl.p, w.skin_flags.p, 16, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        eg.staging_dirty = false;
-        if (eg.timer.on) eg.timer.resolve(eg.timer.cur ^ 1);   // the previous call has finished
-        double maxd;
-        memcpy(&maxd, eg.ctl.p, 8);
-        const int overlap = eg.ctl.as<int>()[2];
+        volatile int *ov = eg.ctl.as<int>() + 2;
+        *ov = 0;
+        const bool little = h_pos && S == 1 && eg.nl_last.size() == 3 * (size_t)N &&
+                            moved_little(h_pos, eg.nl_last.data(), N, lats, 0.5 * skin);
+        if (!little) {
+            CHK(w.skin_flags.ensure(64));
+            launch_fill_i32(w.skin_flags.as<int>(), 2, 0, s);
+            launch_nl_max_disp(N, d_pos, w.last_pos.as<double>(), w.geo.as<NLGeom>(), w.sid.as<int>(),
+                               (unsigned long long *)w.skin_flags.p, s);
+            HIPCHK(hipMemcpyAsync(eg.ctl.p, w.skin_flags.p, 8, hipMemcpyDeviceToHost, s));
+        }
+        launch_nl_full(N, d_pos, w.geo.as<NLGeom>(), w.sid.as<int>(), w.n1_off.as<int>(), w.n1_j.as<int>(),
+                       w.n1_shift.as<int>(), w.n1_r.as<double>(), w.n2_off.as<int>(), w.n2_is.as<int>(),
+                       w.n2_ks.as<int>(), w.n1_rev.as<int>(), w.nb_off.as<int>(), w.nb_j.as<int>(),
+                       w.nb_rev.as<int>(), w.nb_r.as<double>(), w.nb_d.as<double>(), 0, s, w.pairF.as<double>(),
+                       has_d2b ? w.pairE.as<double>() : nullptr, w.esite.as<double>(), (int *)ov);
+        double maxd = 0.0;
+        if (!little) {
+            HIPCHK(hipStreamSynchronize(s));
+            eg.staging_dirty = false;
+            if (eg.timer.on) eg.timer.resolve(eg.timer.cur ^ 1);   // the previous call has finished
+            memcpy(&maxd, eg.ctl.p, 8);
+        }
         if (maxd < 0.5 * skin) {
-            if (overlap) return fail(GAPX_E_GEOMETRY, "calc_dists: two atoms overlap exactly");
-            launch_nl_full(N, d_pos, w.geo.as<NLGeom>(), w.sid.as<int>(), w.n1_off.as<int>(), w.n1_j.as<int>(),
-                           w.n1_shift.as<int>(), w.n1_r.as<double>(), w.n2_off.as<int>(), w.n2_is.as<int>(),
-                           w.n2_ks.as<int>(), w.n1_rev.as<int>(), w.nb_off.as<int>(), w.nb_j.as<int>(),
-                           w.nb_rev.as<int>(), w.nb_r.as<double>(), w.nb_d.as<double>(), 0, s);
+            if (!little && *ov) return overlap_error();
+            eg.overlap = little;
             eg.last_rebuilt = false;
-            *P_out = 2 * eg.n1_total_last;
+            *P_out = (int)P;
+            *cleared = true;
             return GAPX_OK;
         }
     }
-    eg.nl_valid = false;
     CHK(build_nl(m, eg, S, atom_off, d_pos, h_pos, lats, pbcs, cutoff, P_out));
     if (skin > 0 && m->nl_reuse) {   // remember this build for the next call
         CHK(w.last_pos.ensure((size_t)N * 24 + 24));
         if (N) HIPCHK(hipMemcpyAsync(w.last_pos.p, d_pos, (size_t)N * 24, hipMemcpyDeviceToDevice, s));
+        eg.nl_last.clear();
+        if (h_pos && S == 1 && N <= kHostMoveAtoms) eg.nl_last.assign(h_pos, h_pos + 3 * (size_t)N);
         eg.nl_cut = cutoff;
         eg.nl_lats.assign(lats, lats + 9 * S);
         eg.nl_pbcs.assign(pbcs, pbcs + 3 * S);
@@ -1749,6 +1789,10 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
     const bool spec = spec_ok && pl.spec;
     if (!(spec_ok && pl.inl)) CHK(flush_positions(eg, d_pos, N));
     const int t_nl0 = tm.on ? tm.mark(s) : -1;
+    // pair energies exist only with a distance_2b term; without one the gather skips them
+    bool has_d2b = false, cleared = false;
+    for (auto &c : m->coords) has_d2b = has_d2b || c->kind == 2;
+    eg.overlap = false;
     int P = 0;
     if (spec) {
         P = 2 * pl.capT1;   // a capacity: kernels that loop over pairs read their counts on the device
@@ -1772,7 +1816,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         eg.last_rebuilt = true;
         P = 2 * n1_total;
     } else if (ext) CHK(connect_external(eg, *ext, N, d_pos, lats, &P));
-    else CHK(connect(m, eg, S, atom_off, d_pos, h_pos, lats, pbcs, rc, &P));
+    else CHK(connect(m, eg, S, atom_off, d_pos, h_pos, lats, pbcs, rc, has_d2b, &P, &cleared));
     if (tm.on && !spec) tm.stage(0, t_nl0, tm.mark(s));
 
     // Prepare: every buffer the launches use is sized here (to the largest
@@ -1872,9 +1916,6 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
     double *o_lv = (want & GAPX_WANT_LOCAL_V) && d_lv ? d_lv : w.lv.as<double>();
 
     // The launch sequence (stage events only when timing, never inside a graph).
-    // pair energies exist only with a distance_2b term; without one the gather skips them
-    bool has_d2b = false;
-    for (size_t k = 0; k < NCOORD; k++) has_d2b = has_d2b || m->coords[k]->kind == 2;
     double *pairE = has_d2b ? w.pairE.as<double>() : nullptr;
     double *d_epc = opt ? opt->d_epc : nullptr;
     if (S == 1) CHK(w.spart.ensure((size_t)(N / 8 + 2) * 80));   // the gather's block partials
@@ -1888,7 +1929,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
             nl_launch_front(eg, pl, d_pos);
             nl_launch_back(eg, pl, d_pos, true, true, w.pairF.as<double>(), pairE, w.esite.as<double>());
             if (marks) tm.stage(0, t_nl0, tm.mark(s));
-        } else {
+        } else if (!cleared) {
             launch_zero_step(w.pairF.as<double>(), pairE, w.esite.as<double>(), N, nullptr, P, (size_t)P, s);
         }
         if (d_epc) launch_fill_f64(d_epc, NCOORD, 0.0, s);
@@ -2035,7 +2076,7 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         // replay the captured sequence when nothing it depends on has changed
         std::vector<long long> key = {S, N, P, m->precision, (long long)want, (long long)(uintptr_t)o_e,
                                       (long long)(uintptr_t)o_v, (long long)(uintptr_t)o_f, (long long)(uintptr_t)o_le,
-                                      (long long)(uintptr_t)o_lv, alloc_generation(), spec ? 1 : 0};
+                                      (long long)(uintptr_t)o_lv, alloc_generation(), (spec ? 1 : 0) + (cleared ? 2 : 0)};
         if (spec)
             key.insert(key.end(), {(long long)(uintptr_t)d_pos, pl.NC, pl.cap1, pl.cap2, pl.capT1, pl.dev_geo ? 1 : 0});
         long long es;
@@ -2230,6 +2271,10 @@ int gapx::calc_host(gapx_model *m, Engine &eg, int S, const int *atom_off, const
     eg.out_dst = nullptr;
     CHK(st);
     HIPCHK(hipStreamSynchronize(s));
+    if (eg.overlap && eg.ctl.as<int>()[2]) {
+        eg.last_rebuilt = true;
+        return overlap_error();
+    }
     for (const Out &q : o)
         if (q.on && q.n) memcpy(q.dst, ho + q.off, q.n * 8);
     return GAPX_OK;

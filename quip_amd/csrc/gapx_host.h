@@ -314,7 +314,8 @@ struct Engine {
     // skin reuse: the last build's cutoff and lattices; valid while the atoms are the same
     bool nl_valid = false, last_rebuilt = true;
     double nl_cut = 0;
-    std::vector<double> nl_lats;
+    std::vector<double> nl_lats, nl_last;   // nl_last: its positions, for host calls of one structure
+    bool overlap = false;   // a reused list whose overlap flag (ctl) is read with the results
     std::vector<int> nl_pbcs;
     hipGraphExec_t gexec = nullptr;   // the captured launch sequence after the neighbour count
     std::vector<long long> gkey;

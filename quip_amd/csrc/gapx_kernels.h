@@ -79,17 +79,17 @@ void launch_nl_compact(int N, int cap1, int cap2, const int *n1_off, const int *
 // cap2 > 0: the unsorted entries are read from the one-pass slots (atom j's at j * cap2)
 void launch_nl_n2_sort(int N, const int *n2_off, const int *n2_i, const int *n2_k, const int *cell_of,
                        const int *n1_off, int *n2_is, int *n2_ks, int *n1_rev, int cap2, hipStream_t s);
-// cap1 > 0: neighbour1 data from the one-pass slots (atom a's entry k at a * cap1 + k)
+// cap1 > 0: neighbour1 data from the one-pass slots (atom a's entry k at a * cap1 + k);
+// overlap (pinned): a reused list, its distances recomputed as calc_dists does
 void launch_nl_full(int N, const double *pos, const NLGeom *geo, const int *sid, const int *n1_off, const int *n1_j,
                     const int *n1_shift, const double *n1_r, const int *n2_off, const int *n2_i, const int *n2_k,
                     const int *n1_rev, int *nb_off, int *nb_j, int *nb_rev, double *nb_r, double *nb_d, int cap1,
                     hipStream_t s, double *pairF = nullptr,
-                    double *pairE = nullptr, double *esite = nullptr);
+                    double *pairE = nullptr, double *esite = nullptr, int *overlap = nullptr);
 // skin reuse: max displacement since the last build (bits of a double, atomicMax into a
-// zeroed word) and the stored neighbour1 distances recomputed as calc_dists does
-void launch_nl_skin_check(int N, const double *pos, const double *last, const NLGeom *geo, const int *sid,
-                          const int *n1_off, const int *n1_j, const int *n1_shift, double *n1_r,
-                          unsigned long long *max_disp, int *overlap, hipStream_t s);
+// zeroed word)
+void launch_nl_max_disp(int N, const double *pos, const double *last, const NLGeom *geo, const int *sid,
+                        unsigned long long *max_disp, hipStream_t s);
 void launch_minmax_frac(int S, const int *atom_off, const double *pos, const double *g, double *out, hipStream_t s);
 // lat_eff of structures with a non-periodic axis from this call's extents mm (6 per
 // structure) into geo; flags[0] |= 4 when a structure's cell counts differ from geo's

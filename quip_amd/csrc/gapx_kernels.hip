@@ -920,6 +920,28 @@ void launch_nl_n2_sort(int N, const int *n2_off, const int *n2_i, const int *n2_
 #undef N2S
 }
 
+// connection_calc_dists (Connection.f95:1321-1445) for a neighbour1 entry of atom i:
+// r_ij = norm(pos_j + lattice.shift - pos_i) with j_pos formed as
+// pos_j + ((L1 s1 + L2 s2) + L3 s3).  The reference visits every pair from both
+// ends and the later visit wins, so for i < j the stored value is computed from
+// j's side (shift negated); self images from i's side.
+__device__ __forceinline__ double pair_dist(const double *pos, const NLGeom &g, int i, int j, int s0, int s1, int s2) {
+#pragma clang fp contract(off)
+    int from = i, to = j;          // r = norm(pos(to) + L.s - pos(from))
+    if (j != i) { from = j; to = i; s0 = -s0; s1 = -s1; s2 = -s2; }
+    double v[3];
+    for (int k = 0; k < 3; k++) {
+        double t = g.lat[k] * (double)s0;
+        t = t + g.lat[3 + k] * (double)s1;
+        t = t + g.lat[6 + k] * (double)s2;
+        v[k] = (pos[3 * to + k] + t) - pos[3 * from + k];
+    }
+    double dsq = v[0] * v[0];
+    dsq = dsq + v[1] * v[1];
+    dsq = dsq + v[2] * v[2];
+    return sqrt(dsq);
+}
+
 // Full per-atom neighbour view in connection_neighbour order (neighbour2 first,
 // Connection.f95:2038-2051), with diff = pos_j - pos_i + lattice.shift summed
 // m = 1..3 (:2120-2125) and the index of the mirror pair.  A group of 32 lanes
@@ -929,14 +951,17 @@ void launch_nl_n2_sort(int N, const int *n2_off, const int *n2_i, const int *n2_
 // neighbour2 and the mirror slots n1_rev keep the compacted numbering.
 // With pairF non-null the step's accumulators are cleared on the way: pairF (and pairE,
 // if given) over every pair written, esite over every atom.
-template <bool SLOT>
+// DIST: a reused list (calc_connect's skin): the distances come from the positions as
+// calc_dists has them (see pair_dist) instead of n1_r; *overlap = 1 (pinned host memory, by
+// a plain store) for atoms that overlap.
+template <bool SLOT, bool DIST>
 __global__ __launch_bounds__(256) void k_nl_full(int N, const double *__restrict__ pos,
                                                  const NLGeom *__restrict__ geo, const int *__restrict__ sid,
                                                  const int *n1_off, const int *n1_j, const int *n1_shift,
                                                  const double *n1_r, const int *n2_off, const int *n2_i,
                                                  const int *n2_k, const int *n1_rev, int *nb_off, int *nb_j,
                                                  int *nb_rev, double *nb_r, double *nb_d, int cap1, double *pairF,
-                                                 double *pairE, double *esite) {
+                                                 double *pairE, double *esite, int *overlap) {
 #pragma clang fp contract(off)
     auto at1 = [&](int a, int k) -> size_t { return SLOT ? (size_t)a * cap1 + k : (size_t)n1_off[a] + k; };
     const int lane = threadIdx.x & 31;
@@ -980,7 +1005,12 @@ __global__ __launch_bounds__(256) void k_nl_full(int N, const double *__restrict
         const int p = base + q;
         nb_j[p] = j;
         nb_rev[p] = rev;
-        nb_r[p] = n1_r[e1];
+        if (DIST) {
+            // the neighbour1 entry is its owner's (i, or j for an entry of neighbour2)
+            const double r = sgn > 0 ? pair_dist(pos, g, i, j, s0, s1, s2) : pair_dist(pos, g, j, i, -s0, -s1, -s2);
+            if (r < 1e-10) *overlap = 1;
+            nb_r[p] = r;
+        } else nb_r[p] = n1_r[e1];
         nb_d[3 * p] = d0; nb_d[3 * p + 1] = d1; nb_d[3 * p + 2] = d2;
         if (pairF) {
             pairF[3 * p] = 0.0; pairF[3 * p + 1] = 0.0; pairF[3 * p + 2] = 0.0;
@@ -991,15 +1021,19 @@ __global__ __launch_bounds__(256) void k_nl_full(int N, const double *__restrict
 void launch_nl_full(int N, const double *pos, const NLGeom *geo, const int *sid, const int *n1_off, const int *n1_j,
                     const int *n1_shift, const double *n1_r, const int *n2_off, const int *n2_i, const int *n2_k,
                     const int *n1_rev, int *nb_off, int *nb_j, int *nb_rev, double *nb_r, double *nb_d, int cap1,
-                    hipStream_t s, double *pairF, double *pairE, double *esite) {
-    if (cap1 > 0)
-        hipLaunchKernelGGL(k_nl_full<true>, dim3(cdiv(N + 1, 8)), dim3(256), 0, s, N, pos, geo, sid, n1_off, n1_j,
-                           n1_shift, n1_r, n2_off, n2_i, n2_k, n1_rev, nb_off, nb_j, nb_rev, nb_r, nb_d, cap1, pairF,
-                           pairE, esite);
-    else
-        hipLaunchKernelGGL(k_nl_full<false>, dim3(cdiv(N + 1, 8)), dim3(256), 0, s, N, pos, geo, sid, n1_off, n1_j,
+                    hipStream_t s, double *pairF, double *pairE, double *esite, int *overlap) {
+    if (overlap)
+        hipLaunchKernelGGL((k_nl_full<false, true>), dim3(cdiv(N + 1, 8)), dim3(256), 0, s, N, pos, geo, sid, n1_off, n1_j,
                            n1_shift, n1_r, n2_off, n2_i, n2_k, n1_rev, nb_off, nb_j, nb_rev, nb_r, nb_d, 0, pairF,
-                           pairE, esite);
+                           pairE, esite, overlap);
+    else if (cap1 > 0)
+        hipLaunchKernelGGL((k_nl_full<true, false>), dim3(cdiv(N + 1, 8)), dim3(256), 0, s, N, pos, geo, sid, n1_off, n1_j,
+                           n1_shift, n1_r, n2_off, n2_i, n2_k, n1_rev, nb_off, nb_j, nb_rev, nb_r, nb_d, cap1, pairF,
+                           pairE, esite, nullptr);
+    else
+        hipLaunchKernelGGL((k_nl_full<false, false>), dim3(cdiv(N + 1, 8)), dim3(256), 0, s, N, pos, geo, sid, n1_off, n1_j,
+                           n1_shift, n1_r, n2_off, n2_i, n2_k, n1_rev, nb_off, nb_j, nb_rev, nb_r, nb_d, 0, pairF,
+                           pairE, esite, nullptr);
 }
 
 // Skin reuse (calc_connect with cutoff_skin, Connection.f95:1085-1127).
@@ -1033,47 +1067,11 @@ __global__ void k_nl_max_disp(int N, const double *__restrict__ pos, const doubl
     if (threadIdx.x == 0) atomicMax(out, (unsigned long long)__double_as_longlong(red[0]));
 }
 
-// connection_calc_dists (Connection.f95:1321-1445) on the stored neighbour1
-// entries: r_ij = norm(pos_j + lattice.shift - pos_i) with j_pos formed as
-// pos_j + ((L1 s1 + L2 s2) + L3 s3).  The reference visits every pair from both
-// ends and the later visit wins, so for i < j the stored value is computed from
-// j's side (shift negated); self images from i's side.  r < 1e-10 sets *overlap.
-__global__ void k_nl_dists(int N, const double *__restrict__ pos, const NLGeom *__restrict__ geo,
-                           const int *__restrict__ sid, const int *__restrict__ n1_off, const int *__restrict__ n1_j,
-                           const int *__restrict__ n1_shift, double *n1_r, int *overlap) {
-#pragma clang fp contract(off)
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const NLGeom &g = geo[sid[i]];
-    for (int e = n1_off[i]; e < n1_off[i + 1]; e++) {
-        const int j = n1_j[e];
-        int s0 = n1_shift[3 * e], s1 = n1_shift[3 * e + 1], s2 = n1_shift[3 * e + 2];
-        int from = i, to = j;          // r = norm(pos(to) + L.s - pos(from))
-        if (j != i) { from = j; to = i; s0 = -s0; s1 = -s1; s2 = -s2; }
-        double v[3];
-        for (int k = 0; k < 3; k++) {
-            double t = g.lat[k] * (double)s0;
-            t = t + g.lat[3 + k] * (double)s1;
-            t = t + g.lat[6 + k] * (double)s2;
-            v[k] = (pos[3 * to + k] + t) - pos[3 * from + k];
-        }
-        double dsq = v[0] * v[0];
-        dsq = dsq + v[1] * v[1];
-        dsq = dsq + v[2] * v[2];
-        const double r = sqrt(dsq);
-        if (r < 1e-10) atomicOr(overlap, 1);
-        n1_r[e] = r;
-    }
-}
-
-void launch_nl_skin_check(int N, const double *pos, const double *last, const NLGeom *geo, const int *sid,
-                          const int *n1_off, const int *n1_j, const int *n1_shift, double *n1_r,
-                          unsigned long long *max_disp, int *overlap, hipStream_t s) {
-    if (N <= 0) return;
-    hipLaunchKernelGGL(k_nl_max_disp, dim3(std::min(cdiv(N, 256), 1024)), dim3(256), 0, s, N, pos, last, geo, sid,
-                       max_disp);
-    hipLaunchKernelGGL(k_nl_dists, dim3(cdiv(N, 256)), dim3(256), 0, s, N, pos, geo, sid, n1_off, n1_j, n1_shift,
-                       n1_r, overlap);
+void launch_nl_max_disp(int N, const double *pos, const double *last, const NLGeom *geo, const int *sid,
+                        unsigned long long *max_disp, hipStream_t s) {
+    if (N > 0)
+        hipLaunchKernelGGL(k_nl_max_disp, dim3(std::min(cdiv(N, 256), 1024)), dim3(256), 0, s, N, pos, last, geo, sid,
+                           max_disp);
 }
 
 // min / max of fractional coordinates (g .mult. pos) per axis, for calc_lat_eff;
