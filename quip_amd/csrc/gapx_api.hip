@@ -1224,15 +1224,9 @@ static int overlap_error() { return fail(GAPX_E_GEOMETRY, "calc_dists: two atoms
 constexpr int kHostMoveAtoms = 32768;   // their host pass stays below the read-back it replaces
 
 // Whether host positions alone tell that no atom of one structure has moved by half the skin
-// since the positions `last`: the plain displacements are below it, and too short for any
-// fractional component to round to another image.  A pass over 997 atoms takes 1 us; the
-// device's test, its read-back and the empty stream behind it took 50.  False leaves the
-// decision to the device.
-static bool moved_little(const double *pos, const double *last, int N, const double *lat, double half_skin) {
-    double gi[9];
-    inv3(lat, gi);
-    for (int a = 0; a < 3; a++)
-        if (half_skin * std::sqrt(gi[a] * gi[a] + gi[3 + a] * gi[3 + a] + gi[6 + a] * gi[6 + a]) >= 0.49) return false;
+// since the positions `last`.  A pass over 997 atoms takes 1 us; the device's test, its
+// read-back and the empty stream behind it took 50.  False leaves the decision to the device.
+static bool moved_little(const double *pos, const double *last, int N, double half_skin) {
     double mx = 0.0;
     for (int i = 0; i < N; i++) {
         const double x = pos[3 * i] - last[3 * i], y = pos[3 * i + 1] - last[3 * i + 1], z = pos[3 * i + 2] - last[3 * i + 2];
@@ -1269,12 +1263,11 @@ static int connect(gapx_model *m, Engine &eg, int S, const int *atom_off, const 
         volatile int *ov = eg.ctl.as<int>() + 2;
         *ov = 0;
         const bool little = h_pos && S == 1 && eg.nl_last.size() == 3 * (size_t)N &&
-                            moved_little(h_pos, eg.nl_last.data(), N, lats, 0.5 * skin);
+                            moved_little(h_pos, eg.nl_last.data(), N, 0.5 * skin);
         if (!little) {
             CHK(w.skin_flags.ensure(64));
             launch_fill_i32(w.skin_flags.as<int>(), 2, 0, s);
-            launch_nl_max_disp(N, d_pos, w.last_pos.as<double>(), w.geo.as<NLGeom>(), w.sid.as<int>(),
-                               (unsigned long long *)w.skin_flags.p, s);
+            launch_nl_max_disp(N, d_pos, w.last_pos.as<double>(), (unsigned long long *)w.skin_flags.p, s);
             HIPCHK(hipMemcpyAsync(eg.ctl.p, w.skin_flags.p, 8, hipMemcpyDeviceToHost, s));
         }
         launch_nl_full(N, d_pos, w.geo.as<NLGeom>(), w.sid.as<int>(), w.n1_off.as<int>(), w.n1_j.as<int>(),

@@ -88,8 +88,7 @@ void launch_nl_full(int N, const double *pos, const NLGeom *geo, const int *sid,
                     double *pairE = nullptr, double *esite = nullptr, int *overlap = nullptr);
 // skin reuse: max displacement since the last build (bits of a double, atomicMax into a
 // zeroed word)
-void launch_nl_max_disp(int N, const double *pos, const double *last, const NLGeom *geo, const int *sid,
-                        unsigned long long *max_disp, hipStream_t s);
+void launch_nl_max_disp(int N, const double *pos, const double *last, unsigned long long *max_disp, hipStream_t s);
 void launch_minmax_frac(int S, const int *atom_off, const double *pos, const double *g, double *out, hipStream_t s);
 // lat_eff of structures with a non-periodic axis from this call's extents mm (6 per
 // structure) into geo; flags[0] |= 4 when a structure's cell counts differ from geo's

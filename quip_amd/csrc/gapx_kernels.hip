@@ -1037,26 +1037,17 @@ void launch_nl_full(int N, const double *pos, const NLGeom *geo, const int *sid,
 }
 
 // Skin reuse (calc_connect with cutoff_skin, Connection.f95:1085-1127).
-// Largest displacement of any atom since the positions `last` of the last build,
-// minimum image over periodic axes (fractional displacement wrapped to the
-// nearest lattice vector), as the bits of a non-negative double in *out (atomicMax).
+// Largest displacement of any atom since the positions `last` of the last build, as the
+// bits of a non-negative double in *out (atomicMax).  The plain displacement: the list's
+// shifts belong to the images the atoms had, so one that crossed the cell rebuilds it.
 __global__ void k_nl_max_disp(int N, const double *__restrict__ pos, const double *__restrict__ last,
-                              const NLGeom *__restrict__ geo, const int *__restrict__ sid,
                               unsigned long long *out) {
     __shared__ double red[256];
     double mx = 0.0;
     for (int n = blockIdx.x * blockDim.x + threadIdx.x; n < N; n += gridDim.x * blockDim.x) {
-        const NLGeom &g = geo[sid[n]];
         const double dx = pos[3 * n] - last[3 * n], dy = pos[3 * n + 1] - last[3 * n + 1],
                      dz = pos[3 * n + 2] - last[3 * n + 2];
-        // fractional displacement through the inverse of the true lattice (kept in lat_inv order)
-        double f[3];
-        for (int a = 0; a < 3; a++) f[a] = g.ginv[a] * dx + g.ginv[3 + a] * dy + g.ginv[6 + a] * dz;
-        for (int a = 0; a < 3; a++)
-            if (g.pbc[a]) f[a] -= rint(f[a]);
-        double c[3];
-        for (int k = 0; k < 3; k++) c[k] = g.lat[k] * f[0] + g.lat[3 + k] * f[1] + g.lat[6 + k] * f[2];
-        mx = fmax(mx, sqrt(c[0] * c[0] + c[1] * c[1] + c[2] * c[2]));
+        mx = fmax(mx, sqrt(dx * dx + dy * dy + dz * dz));
     }
     red[threadIdx.x] = mx;
     __syncthreads();
@@ -1067,10 +1058,9 @@ __global__ void k_nl_max_disp(int N, const double *__restrict__ pos, const doubl
     if (threadIdx.x == 0) atomicMax(out, (unsigned long long)__double_as_longlong(red[0]));
 }
 
-void launch_nl_max_disp(int N, const double *pos, const double *last, const NLGeom *geo, const int *sid,
-                        unsigned long long *max_disp, hipStream_t s) {
+void launch_nl_max_disp(int N, const double *pos, const double *last, unsigned long long *max_disp, hipStream_t s) {
     if (N > 0)
-        hipLaunchKernelGGL(k_nl_max_disp, dim3(std::min(cdiv(N, 256), 1024)), dim3(256), 0, s, N, pos, last, geo, sid,
+        hipLaunchKernelGGL(k_nl_max_disp, dim3(std::min(cdiv(N, 256), 1024)), dim3(256), 0, s, N, pos, last,
                            max_disp);
 }
 

@@ -47,6 +47,9 @@ def test_reuse_on_host_positions(reps, pair, tmp_path):
         check(False, "small moves")
     at.positions[0] = built[0] + [0.0, 0.31, 0.0]   # from the build's place, whatever the small moves were
     check(True, "past half the skin")
+    at.positions[n // 2] += at.cell[0]   # the same crystal, other images: the kept shifts are not its own
+    check(True, "across the cell")
+    check(False, "unmoved")
     pot.descriptors(at.copy(), cutoff=5.5)
     check(True, "after another use of the tables")
     check(False, "unmoved")
