@@ -853,9 +853,10 @@ __global__ __launch_bounds__(512) void k_gp_fused_split(int nc, int M, int d, in
 __device__ __forceinline__ int sk_block_of(long x, int B, long U) { return (int)(((x + 1) * B - 1) / U); }
 
 // Stream-K fix-up.  Blocks [0, gblocks): G of the row blocks that several blocks of the
-// grid share, each such row block once (by the grid boundary k that falls first inside
-// it), kSkQ blocks per boundary streaming a 1/kSkQ share of the row block's elements each
-// (16: batch512 28.9 -> 26.6 us against 4; the sums are the same).
+// grid share, kSkQ blocks for each grid boundary that falls inside, every one of them a share
+// of the row block's elements (16: batch512 28.9 -> 26.6 us against 4; the sums are the same).
+// 4055 centres put eight boundaries into a row block; with the first one's blocks doing all
+// of it, nine dependent loads in a row, twice, took 14.5 us.
 // A shared row block's slots are contiguous 128 x d FP32 tiles and its G rows are
 // contiguous, so elements go by flat index, four at a time.  Its first block b0 reached
 // it after an earlier row block (slot 1) unless its range starts at the row block
@@ -874,25 +875,33 @@ __global__ __launch_bounds__(256) void k_gp_sk_finish(int nc, int d, int C, int 
         if (x % C == 0) return;
         const int rb = (int)(x / C);
         const int b0 = sk_block_of((long)rb * C, B, U), b1 = sk_block_of((long)rb * C + C - 1, B, U);
-        if (b0 != k - 1) return;   // an earlier boundary of this row block does it
+        const int share = k - 1 - b0, shares = b1 - b0;   // of the row block's boundaries
         const int b0_slot = 2 * b0 + ((long)b0 * U / B < (long)rb * C ? 1 : 0);
         const size_t n = (size_t)min(128, nc - rb * 128) * d;   // elements of the row block's G rows
         const size_t tile = (size_t)128 * d;                    // floats per slot
         double *g = G + (size_t)rb * tile;
-        for (size_t i4 = (size_t)q * 256 + threadIdx.x; i4 < n / 4; i4 += 256 * kSkQ) {
+        for (size_t i4 = (size_t)(share * kSkQ + q) * 256 + threadIdx.x; i4 < n / 4; i4 += (size_t)256 * kSkQ * shares) {
             double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-            for (int b = b0; b <= b1; b++) {
-                const size_t sl = b == b0 ? b0_slot : 2 * (size_t)b;
-                const float4 v = ((const float4 *)(Gslot + sl * tile))[i4];
-                a0 += (double)v.x;
-                a1 += (double)v.y;
-                a2 += (double)v.z;
-                a3 += (double)v.w;
+            for (int b = b0; b <= b1; b += 4) {   // four slots' loads in flight
+                float4 v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int be = min(b + e, b1);
+                    v[e] = ((const float4 *)(Gslot + (be == b0 ? (size_t)b0_slot : 2 * (size_t)be) * tile))[i4];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (b + e <= b1) {
+                        a0 += (double)v[e].x;
+                        a1 += (double)v[e].y;
+                        a2 += (double)v[e].z;
+                        a3 += (double)v[e].w;
+                    }
             }
             ((double2 *)g)[2 * i4] = make_double2(a0 * inv_wscale, a1 * inv_wscale);
             ((double2 *)g)[2 * i4 + 1] = make_double2(a2 * inv_wscale, a3 * inv_wscale);
         }
-        if (q == 0 && threadIdx.x < n % 4) {   // the last row block's tail
+        if (share == 0 && q == 0 && threadIdx.x < n % 4) {   // the last row block's tail
             const size_t e = n / 4 * 4 + threadIdx.x;
             double a = 0.0;
             for (int b = b0; b <= b1; b++) a += (double)Gslot[(b == b0 ? b0_slot : 2 * (size_t)b) * tile + e];
