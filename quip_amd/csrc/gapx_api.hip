@@ -1366,6 +1366,7 @@ static int gemm_tune(gapx_model *m, Engine &eg, Coord &c, int nc, GemmTune &out,
         auto it = c.tune.find(bucket);
         if (it != c.tune.end()) {
             out = it->second;
+            if (out.f64tile && out.f64parts > 0) out.f64parts = gp_f64_tile_parts_default(nc, c.M);
             return GAPX_OK;
         }
     }
@@ -1413,8 +1414,9 @@ static int gemm_tune(gapx_model *m, Engine &eg, Coord &c, int nc, GemmTune &out,
     if (fusable) {   // the fused kernel (with its partial-G sum) against the two GEMMs
         float fbest = 1e30f;
         int fparts = 0;
-        for (int p = 1, prev = 0; p <= (tile ? 32 : 8) && st == GAPX_OK; p *= 2) {
-            const int v = tile ? gp_f64_tile_parts_valid(p, c.M) : gp_f64_parts_valid(p, c.M);
+        // the form for few centres has one count per size, by rule
+        for (int p = tile ? 8 : 1, prev = 0; p <= 8 && st == GAPX_OK; p *= 2) {
+            const int v = tile ? gp_f64_tile_parts_default(nc, c.M) : gp_f64_parts_valid(p, c.M);
             if (v == prev) continue;
             prev = v;
             float t = 0;
@@ -1845,9 +1847,15 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         mC = std::max(mC, (size_t)nc * KLM * 8);
         mE = std::max(mE, (size_t)nc * ((c.M + 31) / 32 + 32) * 8);   // a column per tile, chunk or part
         if (m->precision == GAPX_PREC_FP64) {
-            mW = std::max(mW, (size_t)nc * c.M * 8);
             const bool tile = gp_f64_fused_supported(c.dim) && gp_f64_tile_serves(nc);
-            mGp = std::max(mGp, (size_t)(tile ? 32 : 8) * nc * c.dim * 8);
+            GemmTune cached;
+            if (tile && noalloc) CHK(gemm_tune(m, eg, c, nc, cached, true));
+            if (cached.f64tile && cached.f64parts > 0) {   // the space of the form that will run, and no W
+                mGp = std::max(mGp, (size_t)cached.f64parts * nc * c.dim * 8);
+            } else {
+                mW = std::max(mW, (size_t)nc * c.M * 8);
+                mGp = std::max(mGp, (size_t)(tile && !noalloc ? 32 : 8) * nc * c.dim * 8);
+            }
         } else if (fused[k]) {
             size_t b = fused_scratch_bytes(m->precision, c, nc, 0);
             if (m->autotune && !noalloc) {   // the tuner's candidates

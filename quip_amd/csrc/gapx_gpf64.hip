@@ -299,9 +299,10 @@ int gp_f64_tile_parts_valid(int parts, int M) {
     parts = std::max(1, std::min({parts, tiles, 32}));
     return cdivf(tiles, cdivf(tiles, parts));
 }
-// default: two blocks per CU
+// A block per CU, two steps a part at least: within 10% of the fastest count at all of these
+// sizes.  A rule and not a timing: the counts lie too close for two models to choose alike.
 int gp_f64_tile_parts_default(int nc, int M) {
-    return gp_f64_tile_parts_valid(512 / std::max(1, cdivf(nc, 16)), M);
+    return gp_f64_tile_parts_valid(std::min(256 / std::max(1, cdivf(nc, 16)), cdivf(M, 32)), M);
 }
 
 int gp_f64_parts_valid(int parts, int M) {
