@@ -1448,6 +1448,18 @@ static int gemm_tune(gapx_model *m, Engine &eg, Coord &c, int nc, GemmTune &out,
     return GAPX_OK;
 }
 
+// Bytes of W and of the partial G that the FP64 GP of nc centres takes: of the chosen form
+// (known: f64parts parts of the fused kernel, or with 0 the two GEMMs with a split-K factor
+// of gemm2_split), else of whatever gemm_tune may choose and times on the way.
+GpF64Space gapx::gp_f64_space(bool known, int f64parts, int gemm2_split, int nc, int M, int d) {
+    GpF64Space sp = {8, 8};
+    int parts = known ? (f64parts > 0 ? f64parts : gemm2_split) : 8;
+    if (!known && gp_f64_fused_supported(d) && gp_f64_tile_serves(nc)) parts = 32;
+    if (!known || f64parts <= 0) sp.W = std::max(sp.W, (size_t)nc * M * 8);
+    if (parts > 1) sp.Gparts = std::max(sp.Gparts, (size_t)parts * nc * d * 8);
+    return sp;
+}
+
 // Split-form autotuner, as gemm_tune for the FP64 tiles: per coordinate, precision and
 // centre-count bucket the first evaluation times the fused kernel (with its partial-G sum)
 // for 1, 2, 4 and 8 sparse-point parts and the stream-K schedule (-1), or the split GEMMs
@@ -1850,15 +1862,13 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         mC = std::max(mC, (size_t)nc * KLM * 8);
         mE = std::max(mE, (size_t)nc * ((c.M + 31) / 32 + 32) * 8);   // a column per tile, chunk or part
         if (m->precision == GAPX_PREC_FP64) {
-            const bool tile = gp_f64_fused_supported(c.dim) && gp_f64_tile_serves(nc);
-            GemmTune cached;
-            if (tile && noalloc) CHK(gemm_tune(m, eg, c, nc, cached, true));
-            if (cached.f64tile && cached.f64parts > 0) {   // the space of the form that will run, and no W
-                mGp = std::max(mGp, (size_t)cached.f64parts * nc * c.dim * 8);
-            } else {
-                mW = std::max(mW, (size_t)nc * c.M * 8);
-                mGp = std::max(mGp, (size_t)(tile && !noalloc ? 32 : 8) * nc * c.dim * 8);
-            }
+            // An allocation-free call looks at the tuning table here and nowhere else: other
+            // threads tune the same buckets, and a second look could choose a form whose
+            // space this one did not size.  An allocating call sizes for every choice.
+            if (noalloc) CHK(gemm_tune(m, eg, c, nc, tunes[k], true));
+            const GpF64Space sp = gp_f64_space(noalloc, tunes[k].f64parts, tunes[k].parts, nc, c.M, c.dim);
+            mW = std::max(mW, sp.W);
+            mGp = std::max(mGp, sp.Gparts);
         } else if (fused[k]) {
             size_t b = fused_scratch_bytes(m->precision, c, nc, 0);
             if (m->autotune && !noalloc) {   // the tuner's candidates
@@ -1898,8 +1908,9 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         Coord &c = *m->coords[k];
         const int nc = (int)eg.h_centres[k].size();
         if (c.kind != 1 || nc == 0 || skipped(k)) continue;
-        if (m->precision == GAPX_PREC_FP64) CHK(gemm_tune(m, eg, c, nc, tunes[k], noalloc));
-        else {
+        if (m->precision == GAPX_PREC_FP64) {
+            if (!noalloc) CHK(gemm_tune(m, eg, c, nc, tunes[k]));
+        } else {
             if (c.split_prec != m->precision) {
                 if (noalloc)
                     return fail(GAPX_E_ARG, "split copies of the sparse points are missing (set the precision first)");

@@ -118,6 +118,8 @@ struct GemmTune {
     int f64parts = 0;
     float f64_ms = 0;
 };
+struct GpF64Space { size_t W, Gparts; };   // bytes
+GpF64Space gp_f64_space(bool known, int f64parts, int gemm2_split, int nc, int M, int d);
 constexpr size_t kTuneScratchCap = (size_t)256 << 20;   // largest partial-G buffer a tuning candidate may use
 constexpr size_t kNoallocTuneCap = (size_t)32 << 20;    // largest one an allocation-free call sizes for a cached tuning
 
