@@ -1768,6 +1768,10 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
     if (ext && S != 1) return fail(GAPX_E_ARG, "a supplied connection covers one structure");
     if (ext && opt) return fail(GAPX_E_ARG, "calc options with a supplied connection");
     if (opt && opt->only_coord < 0) return fail(GAPX_E_ARG, "only_descriptor must be >= 0");
+    if (S == 0) {   // no structure, no result: nothing is launched or left pending
+        eg.var_valid = false;
+        return GAPX_OK;
+    }
     const bool want_var = opt && opt->variance;
     const bool want_vgrad = want_var && opt->d_gvg;
     // The speculative neighbour list: no read-back inside the call, so the whole call is

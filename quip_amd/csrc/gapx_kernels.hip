@@ -2293,9 +2293,9 @@ __global__ __launch_bounds__(kReduceThreads) void k_struct_finish(int nb, const 
 }
 void launch_struct_finish(int N, const double *part, double *e_out, double *virial_out, hipStream_t s,
                           const int *flag_src, int *flag_dst, const double *out_src, double *out_dst, int out_n) {
-    if (N > 0)
-        hipLaunchKernelGGL(k_struct_finish, dim3(1), dim3(kReduceThreads), 0, s, cdiv(N, 8), part, e_out, virial_out,
-                           flag_src, flag_dst, out_src, out_dst, out_n);
+    // no atoms: no partials, so the totals are zero and the flags are still handed on
+    hipLaunchKernelGGL(k_struct_finish, dim3(1), dim3(kReduceThreads), 0, s, cdiv(N, 8), part, e_out, virial_out,
+                       flag_src, flag_dst, out_src, out_dst, out_n);
 }
 void launch_struct_reduce(int S, const int *atom_off, const double *local_e, const double *local_virial,
                           double *e_out, double *virial_out, hipStream_t s, const int *flag_src, int *flag_dst) {
