@@ -125,9 +125,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                     kz1 = 1.0;
                     for (int q = 1; q < izeta; q++) kz1 *= kv;
                     kz = kz1 * kv;
-                } else {
+                } else if (ws != 0.0) {
                     kz1 = pow(kv, zeta - 1.0);
                     kz = pow(kv, zeta);
+                } else {   // the padding: K is zero, and its power infinite for zeta < 1
+                    kz1 = kz = 0.0;
                 }
                 esum += ws * kz;
                 wf[j][v] = ws * zeta * kz1;
@@ -246,9 +248,11 @@ __global__ __launch_bounds__(256, 2) void k_gp_tile_f64(int nc, int M, int d, in
                 kz1 = 1.0;
                 for (int q = 1; q < izeta; q++) kz1 *= kv;
                 kz = kz1 * kv;
-            } else {
+            } else if (ws != 0.0) {
                 kz1 = pow(kv, zeta - 1.0);
                 kz = pow(kv, zeta);
+            } else {   // the padding, as above
+                kz1 = kz = 0.0;
             }
             esum += ws * kz;
             wf[v] = ws * zeta * kz1;

@@ -637,9 +637,11 @@ __device__ __forceinline__ void fused_sub(int h, const typename Half<PREC>::T *_
                     kz1 = 1.0;
                     for (int q = 1; q < izeta; q++) kz1 *= kv;
                     kz = kz1 * kv;
-                } else {
+                } else if (wsv != 0.0) {
                     kz1 = pow(kv, zeta - 1.0);
                     kz = pow(kv, zeta);
+                } else {   // the padding: K is zero, and its power infinite for zeta < 1
+                    kz1 = kz = 0.0;
                 }
                 rs += wsv * kz;
                 const double wk = wsv * zeta * kz1 * wscale;
