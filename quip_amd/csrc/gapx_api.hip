@@ -1953,9 +1953,8 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         }
         if (d_epc) launch_fill_f64(d_epc, NCOORD, 0.0, s);
         if (want_var) {
-            double *zp[3] = {w.pairFv.as<double>(), w.varsite.as<double>(), w.pairVE.as<double>()};
-            const size_t zn[3] = {(size_t)P * 3, (size_t)N, (size_t)P};
-            launch_zero_f64_multi(has_d2b_var ? 3 : 2, zp, zn, s);
+            launch_var_clear(N, w.nb_off.as<int>() + N, P, w.pairFv.as<double>(),
+                             has_d2b_var ? w.pairVE.as<double>() : nullptr, w.varsite.as<double>(), s);
         }
         // whether an earlier coordinate writes forces on coordinate k's pairs too: a pair
         // descriptor, or one with a centre species in common (0 is every species).  Otherwise the
@@ -1982,9 +1981,8 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
                            d_epc ? w.eatom.as<double>() : nullptr, s);
                 if (d_epc) launch_sum_fixed(N, w.eatom.as<double>(), d_epc + k, s);
                 if (want_var) {
-                    const double nan = std::nan("");
-                    launch_fill_f64(w.var_inst[k].as<double>(), P, nan, s);
-                    launch_fill_f64(w.cut2_inst[k].as<double>(), P, nan, s);
+                    launch_fill_pairs(w.nb_off.as<int>() + N, P, w.var_inst[k].as<double>(),
+                                      w.cut2_inst[k].as<double>(), std::nan(""), s);
                     launch_d2b_var(N, w.Z.as<int>(), c.Z1, c.Z2, c.rc, c.ctw, c.M, c.d_Xs.as<double>(), d2,
                                    c.d_theta.as<double>(), c.d_Cinv.as<double>(), w.nb_off.as<int>(), w.nb_j.as<int>(),
                                    w.nb_r.as<double>(), w.nb_d.as<double>(), w.pairFv.as<double>(),
@@ -2089,7 +2087,6 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         if (marks) tm.stage(5, tg, tm.mark(s));
     };
     eg.var_valid = want_var;
-    eg.var_P = P;
 
     if (use_graph) {
         // replay the captured sequence when nothing it depends on has changed
@@ -2385,10 +2382,12 @@ extern "C" int gapx_descriptor_variances(gapx_model *m, int coord, int max_entri
         if (!cen.empty()) HIPCHK(hipMemcpy(v.data(), w.var_inst[coord].p, cen.size() * 8, hipMemcpyDeviceToHost));
         for (size_t q = 0; q < cen.size(); q++) put(v[q], 1.0, cen[q], -1);
     } else {
-        const int N = (int)eg.h_Z.size(), P = eg.var_P;
-        std::vector<int> off(N + 1), nj(P + 1);
-        std::vector<double> v(P + 1), c2(P + 1);
+        const int N = (int)eg.h_Z.size();
+        std::vector<int> off(N + 1);
         HIPCHK(hipMemcpy(off.data(), w.nb_off.p, (size_t)(N + 1) * 4, hipMemcpyDeviceToHost));
+        const int P = off[N];   // the list's pairs, not the room it was given
+        std::vector<int> nj(P + 1);
+        std::vector<double> v(P + 1), c2(P + 1);
         if (P) {
             HIPCHK(hipMemcpy(nj.data(), w.nb_j.p, (size_t)P * 4, hipMemcpyDeviceToHost));
             HIPCHK(hipMemcpy(v.data(), w.var_inst[coord].p, (size_t)P * 8, hipMemcpyDeviceToHost));

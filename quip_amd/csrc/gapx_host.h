@@ -324,9 +324,8 @@ struct Engine {
     int n1_total_last = 0;
     int nl_cap1 = 0, nl_cap2 = 0;   // slot sizes of the one-pass neighbour search (0: count first)
     int ncell_last = 0;
-    // the last calc that formed GAP variances: its pair count (instance buffers are per coordinate)
+    // whether the last calc formed GAP variances (instance buffers are per coordinate)
     bool var_valid = false;
-    int var_P = 0;
     // Speculative neighbour lists (no read-back inside a call): the capacity of the
     // neighbour1 tables, the inverse lattices and the last read extents of non-periodic
     // axes, and the calls whose overflow flags are not read yet, with what redoes them.

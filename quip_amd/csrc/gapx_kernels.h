@@ -38,7 +38,6 @@ void launch_fill_i32(int *p, int n, int v, hipStream_t s);
 void launch_fill_f64(double *p, size_t n, double v, hipStream_t s);
 constexpr int kMultiFill = 6;   // arrays one zero-fill launch covers
 void launch_zero_i32_multi(int k, int *const *p, const int *n, hipStream_t s);
-void launch_zero_f64_multi(int k, double *const *p, const size_t *n, hipStream_t s);
 void launch_scan2_max(const int *in1, const int *in2, int n, int *out1, int *out2, int *mx, int *tot1, int *part1,
                       int *part2, hipStream_t s);
 // n <= 65536: both scans (maxima to flags[1], flags[2], the in1 total to flags[3]) and the
@@ -95,8 +94,11 @@ void launch_minmax_frac(int S, const int *atom_off, const double *pos, const dou
 void launch_geom_np(int S, const int *atom_off, const double *mm, NLGeom *geo, int *flags, hipStream_t s);
 // empty every list (offsets zeroed) after a slot or capacity overflow; flags[0] |= 2 for capacity
 void launch_nl_guard(int N, int *flags, int cap, int *n1_off, int *n2_off, hipStream_t s);
-// p[0 .. mult * (*cnt)) = 0 with *cnt read on the device; cap bounds the grid
-void launch_zero_counted(double *p, const int *cnt, int mult, size_t cap, hipStream_t s);
+// the variance's clears in one launch: pairFv (3 per pair) and pairVE (nullable) of *pairs pairs
+// (read on the device; cap bounds the grid), varsite of N atoms; a and b of *pairs pairs = v
+void launch_var_clear(int N, const int *pairs, size_t cap, double *pairFv, double *pairVE, double *varsite,
+                      hipStream_t s);
+void launch_fill_pairs(const int *pairs, size_t cap, double *a, double *b, double v, hipStream_t s);
 // the per-step clears in one launch: pairF (3 per pair) and pairE (nullable) of *cnt pairs
 // (cnt on the device) or n_pairs (cnt null), and esite (N)
 void launch_zero_step(double *pairF, double *pairE, double *esite, int N, const int *cnt, int n_pairs,

@@ -79,15 +79,9 @@ void launch_fill_f64(double *p, size_t n, double v, hipStream_t s) {
 
 // Zero up to kMultiFill arrays in one launch (blockIdx.y picks the array).
 struct ZeroI32Set { int *p[kMultiFill]; int n[kMultiFill]; };
-struct ZeroF64Set { double *p[kMultiFill]; size_t n[kMultiFill]; };
 __global__ void k_zero_i32_multi(ZeroI32Set z) {
     const int a = blockIdx.y;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < z.n[a]; i += gridDim.x * blockDim.x) z.p[a][i] = 0;
-}
-__global__ void k_zero_f64_multi(ZeroF64Set z) {
-    const int a = blockIdx.y;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < z.n[a]; i += (size_t)gridDim.x * blockDim.x)
-        z.p[a][i] = 0.0;
 }
 void launch_zero_i32_multi(int k, int *const *p, const int *n, hipStream_t s) {
     ZeroI32Set z = {};
@@ -97,15 +91,6 @@ void launch_zero_i32_multi(int k, int *const *p, const int *n, hipStream_t s) {
         hipLaunchKernelGGL(k_zero_i32_multi, dim3(std::min(cdiv(mx, 256), 4096), std::min(k, kMultiFill)), dim3(256), 0,
                            s, z);
 }
-void launch_zero_f64_multi(int k, double *const *p, const size_t *n, hipStream_t s) {
-    ZeroF64Set z = {};
-    size_t mx = 0;
-    for (int a = 0; a < k && a < kMultiFill; a++) { z.p[a] = p[a]; z.n[a] = p[a] ? n[a] : 0; mx = std::max(mx, z.n[a]); }
-    if (mx > 0)
-        hipLaunchKernelGGL(k_zero_f64_multi, dim3((int)std::min<size_t>((mx + 255) / 256, 8192), std::min(k, kMultiFill)),
-                           dim3(256), 0, s, z);
-}
-
 
 // ----------------------------------------------------------------------------
 // exclusive prefix sum of n ints into out[0..n] (out[n] = total), three passes:
@@ -1172,15 +1157,30 @@ void launch_nl_guard(int N, int *flags, int cap, int *n1_off, int *n2_off, hipSt
     hipLaunchKernelGGL(k_nl_guard, dim3(cdiv(N + 1, 256)), dim3(256), 0, s, N, flags, cap, n1_off, n2_off);
 }
 
-// zero the first mult * count doubles of p, count = *cnt read on the device
-__global__ void k_zero_counted(double *p, const int *cnt, int mult) {
-    const size_t n = (size_t)(*cnt) * mult;
-    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x)
-        p[q] = 0.0;
+// The variance's arrays over the pairs of the present list (*pairs, on the device) and its
+// atoms.  A list that is not read back has room for the largest one the engine has met: a call
+// of 64 atoms after one of 110592 would clear and fill 5 million pairs.
+__global__ void k_var_clear(int N, const int *pairs, double *pairFv, double *pairVE, double *varsite) {
+    const size_t np = (size_t)*pairs, stride = (size_t)gridDim.x * blockDim.x;
+    const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (size_t q = i0; q < 3 * np; q += stride) pairFv[q] = 0.0;
+    if (pairVE)
+        for (size_t q = i0; q < np; q += stride) pairVE[q] = 0.0;
+    for (size_t q = i0; q < (size_t)N; q += stride) varsite[q] = 0.0;
 }
-void launch_zero_counted(double *p, const int *cnt, int mult, size_t cap, hipStream_t s) {
-    const int blocks = std::max(1, std::min(cdiv((long)cap, 256), 2048));
-    hipLaunchKernelGGL(k_zero_counted, dim3(blocks), dim3(256), 0, s, p, cnt, mult);
+void launch_var_clear(int N, const int *pairs, size_t cap, double *pairFv, double *pairVE, double *varsite,
+                      hipStream_t s) {
+    const size_t mx = std::max<size_t>(3 * cap, (size_t)N);
+    hipLaunchKernelGGL(k_var_clear, dim3(std::max(1, std::min(cdiv((long)mx, 256), 2048))), dim3(256), 0, s, N, pairs,
+                       pairFv, pairVE, varsite);
+}
+__global__ void k_fill_pairs(const int *pairs, double *a, double *b, double v) {
+    const size_t np = (size_t)*pairs, stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < np; q += stride) a[q] = b[q] = v;
+}
+void launch_fill_pairs(const int *pairs, size_t cap, double *a, double *b, double v, hipStream_t s) {
+    hipLaunchKernelGGL(k_fill_pairs, dim3(std::max(1, std::min(cdiv((long)cap, 256), 2048))), dim3(256), 0, s, pairs, a,
+                       b, v);
 }
 
 // The per-step clears in one launch: pair forces (3 per pair) and pair energies
