@@ -1768,10 +1768,8 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
     if (ext && S != 1) return fail(GAPX_E_ARG, "a supplied connection covers one structure");
     if (ext && opt) return fail(GAPX_E_ARG, "calc options with a supplied connection");
     if (opt && opt->only_coord < 0) return fail(GAPX_E_ARG, "only_descriptor must be >= 0");
-    if (S == 0) {   // no structure, no result: nothing is launched or left pending
-        eg.var_valid = false;
-        return GAPX_OK;
-    }
+    eg.var_valid = false;   // a call that fails leaves no instances of another structure's lists
+    if (S == 0) return GAPX_OK;   // no structure, no result: nothing is launched or left pending
     const bool want_var = opt && opt->variance;
     const bool want_vgrad = want_var && opt->d_gvg;
     // The speculative neighbour list: no read-back inside the call, so the whole call is
@@ -2087,6 +2085,9 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         if (marks) tm.stage(5, tg, tm.mark(s));
     };
     eg.var_valid = want_var;
+    eg.var_kept.clear();
+    eg.var_has.assign(NCOORD, 0);
+    for (size_t k = 0; want_var && k < NCOORD; k++) eg.var_has[k] = !skipped(k);
 
     if (use_graph) {
         // replay the captured sequence when nothing it depends on has changed
@@ -2352,31 +2353,20 @@ extern "C" int gapx_calc_device_ex(gapx_model *m, int N, const double *d_pos, co
 // in the reference's instance order (print_gap_variance, IPModel_GAP.f95:506-516):
 // soap, one per centre atom (atoms[2k] = centre, atoms[2k+1] = -1, cutoff_sq = 1);
 // distance_2b, one per directed pair (i, j) with i ascending and j in i's neighbour order.
-extern "C" int gapx_descriptor_variances(gapx_model *m, int coord, int max_entries, double *variance,
-                                         double *cutoff_sq, int *atoms, int *n_entries) {
-    if (!m || !n_entries) return fail(GAPX_E_ARG, "NULL argument");
-    if (coord < 0 || coord >= (int)m->coords.size()) return fail(GAPX_E_ARG, "coordinate %d out of range", coord);
-    Engine &eg = *m->eng;
-    if (!eg.var_valid) return fail(GAPX_E_ARG, "no variance formed by the last calc (ask for GAPX_WANT_VARIANCE)");
+// Read from the device, whose lists are still that calc's.
+static int read_instances(gapx_model *m, Engine &eg, int coord, VarInstances &out) {
     HIPCHK(hipSetDevice(m->device));
-    hipStream_t s = eg.stream;
-    HIPCHK(hipStreamSynchronize(s));
-    const Coord &c = *m->coords[coord];
+    HIPCHK(hipStreamSynchronize(eg.stream));
     Workspace &w = eg.ws;
-    int k = 0;
+    out = VarInstances();
+    if (!eg.var_has[coord]) return GAPX_OK;   // a coordinate the last calc skipped (only_descriptor)
     auto put = [&](double var, double c2, int a, int b) {
-        if (k < max_entries) {
-            if (variance) variance[k] = var;
-            if (cutoff_sq) cutoff_sq[k] = c2;
-            if (atoms) { atoms[2 * k] = a; atoms[2 * k + 1] = b; }
-        }
-        k++;
+        out.var.push_back(var);
+        out.cut2.push_back(c2);
+        out.atoms.push_back(a);
+        out.atoms.push_back(b);
     };
-    if (!w.var_inst[coord].p) {   // a coordinate the last calc skipped (only_descriptor)
-        *n_entries = 0;
-        return GAPX_OK;
-    }
-    if (c.kind == 1) {
+    if (m->coords[coord]->kind == 1) {
         const auto &cen = eg.h_centres[coord];
         std::vector<double> v(cen.size());
         if (!cen.empty()) HIPCHK(hipMemcpy(v.data(), w.var_inst[coord].p, cen.size() * 8, hipMemcpyDeviceToHost));
@@ -2397,7 +2387,25 @@ extern "C" int gapx_descriptor_variances(gapx_model *m, int coord, int max_entri
             for (int p = off[i]; p < off[i + 1]; p++)
                 if (!std::isnan(v[p])) put(v[p], c2[p], i, nj[p]);
     }
-    *n_entries = k;
+    return GAPX_OK;
+}
+
+extern "C" int gapx_descriptor_variances(gapx_model *m, int coord, int max_entries, double *variance,
+                                         double *cutoff_sq, int *atoms, int *n_entries) {
+    if (!m || !n_entries) return fail(GAPX_E_ARG, "NULL argument");
+    if (coord < 0 || coord >= (int)m->coords.size()) return fail(GAPX_E_ARG, "coordinate %d out of range", coord);
+    Engine &eg = *m->eng;
+    if (!eg.var_valid) return fail(GAPX_E_ARG, "no variance formed by the last calc (ask for GAPX_WANT_VARIANCE)");
+    VarInstances read;
+    if (eg.var_kept.empty()) CHK(read_instances(m, eg, coord, read));
+    const VarInstances &vi = eg.var_kept.empty() ? read : eg.var_kept[coord];
+    const int n = (int)vi.var.size();
+    for (int k = 0; k < std::min(n, max_entries); k++) {
+        if (variance) variance[k] = vi.var[k];
+        if (cutoff_sq) cutoff_sq[k] = vi.cut2[k];
+        if (atoms) { atoms[2 * k] = vi.atoms[2 * k]; atoms[2 * k + 1] = vi.atoms[2 * k + 1]; }
+    }
+    *n_entries = n;
     return GAPX_OK;
 }
 
@@ -2587,6 +2595,11 @@ extern "C" int gapx_descriptors(gapx_model *m, int coord, int N, const double *p
     const int off[2] = {0, N};
     CHK(check_batch(1, off, Z, lat, pbc));
     if (N > 0 && !pos) return fail(GAPX_E_ARG, "positions are NULL");
+    if (eg.var_valid && eg.var_kept.empty()) {   // the lists and centres of the last calc's variances go
+        std::vector<VarInstances> kept(m->coords.size());
+        for (size_t k = 0; k < kept.size(); k++) CHK(read_instances(m, eg, (int)k, kept[k]));
+        eg.var_kept.swap(kept);
+    }
     CHK(w.pos.ensure((size_t)N * 24 + 24));
     CHK(eg.stage_io.ensure((size_t)N * 24 + 64));
     if (N) {

@@ -178,6 +178,12 @@ struct Workspace {
     DBuf hout;                   // the results a host-buffer call asked for, one after the other
 };
 
+// Per-instance GAP variances of one coordinate: value, covariance_cutoff^2, two atoms each
+struct VarInstances {
+    std::vector<double> var, cut2;
+    std::vector<int> atoms;
+};
+
 // IPModel_GAP_Calc's args_str options that change what is computed (IPModel_GAP.f95:324-335)
 struct CalcOpts {
     const unsigned char *mask = nullptr;   // atom_mask_name: host, N bytes
@@ -324,8 +330,11 @@ struct Engine {
     int n1_total_last = 0;
     int nl_cap1 = 0, nl_cap2 = 0;   // slot sizes of the one-pass neighbour search (0: count first)
     int ncell_last = 0;
-    // whether the last calc formed GAP variances (instance buffers are per coordinate)
+    // whether the last calc formed GAP variances, and for which coordinates; their instances
+    // once the lists that they belong to have gone (empty before)
     bool var_valid = false;
+    std::vector<char> var_has;
+    std::vector<VarInstances> var_kept;
     // Speculative neighbour lists (no read-back inside a call): the capacity of the
     // neighbour1 tables, the inverse lattices and the last read extents of non-periodic
     // axes, and the calls whose overflow flags are not read yet, with what redoes them.
