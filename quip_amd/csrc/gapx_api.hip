@@ -536,7 +536,10 @@ int gapx::new_engine(gapx_model *m, std::unique_ptr<Engine> &out) {
     std::unique_ptr<Engine> e(new Engine());
     hipError_t he = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
     if (he != hipSuccess) return fail(GAPX_E_DEVICE, "hipStreamCreate: %s", hipGetErrorString(he));
-    e->ctl.coherent = true;   // the overlap flag of a reused list is stored there by its kernel
+    // pinned memory that kernels are handed a pointer into, whichever call allocates it first:
+    e->ctl.coherent = true;        // the overlap flag of a reused list
+    e->stage_io.coherent = true;   // positions and results of small host calls
+    e->checks.coherent = true;     // the list's flags, written by an eager step's last kernel
     e->ws.centres.resize(m->coords.size());
     e->ws.var_inst.resize(m->coords.size());
     e->ws.cut2_inst.resize(m->coords.size());
@@ -1785,7 +1788,6 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         const size_t need_max = (16 + 48 * (size_t)S + 15) & ~(size_t)15;
         if (!spec_ok || eg.pending.size() >= 64 || eg.checks_used + need_max > eg.checks.cap) {
             CHK(resolve_pending(m, eg));
-            eg.checks.coherent = true;   // written by the step's last kernel in eager calls
             if (spec_ok) CHK(eg.checks.ensure(std::max<size_t>(need_max * 64, 4096)));
         }
     }
@@ -2257,7 +2259,6 @@ int gapx::calc_host(gapx_model *m, Engine &eg, int S, const int *atom_off, const
         o2.d_epc = dev(5); o2.d_lgv = dev(6); o2.d_gvg = dev(7);
     }
     const size_t bpos = (size_t)N * 24;
-    eg.stage_io.coherent = true;   // kernels of small calls read and write it
     CHK(eg.stage_io.ensure(bpos + total * 8 + 64));
     char *h = eg.stage_io.as<char>();
     double *ho = (double *)(h + bpos);
