@@ -43,18 +43,22 @@ struct StreamTile {
     static constexpr int AS = BM * kGK, BS = BN * kGK, BUF = AS + BS;
     __amdgpu_buffer_rsrc_t ra, rb;
     unsigned ao[AI], bo[BI], bstep;   // this lane's byte offsets; bytes per k row of the plain B
-    int wv, fa, fb;
+    int wv, fa, fb, kb;               // kb: the row of the plain B where its resource starts
 
     __device__ __forceinline__ static __amdgpu_buffer_rsrc_t rsrc(const double *p, size_t bytes) {
         return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, (int)(unsigned)bytes, 0x00020000);
     }
-    __device__ __forceinline__ void init(const double *A, const double *B, int Mr, int Nc, int Kd, int m0, int n0) {
+    __device__ __forceinline__ void init(const double *A, const double *B, int Mr, int Nc, int Kd, int m0, int n0,
+                                         int kbeg, int kend) {
         const int t = threadIdx.x, lane = t & 63, g = lane >> 4, l16 = lane & 15;
         wv = __builtin_amdgcn_readfirstlane(t >> 6);
         const int ar = min(BM, Mr - m0), br = min(BN, Nc - n0);
         ra = rsrc(A + (size_t)m0 * Kd, (size_t)ar * Kd * 8);
-        // the plain B's last pair of an odd row length ends 8 bytes past the last row
-        rb = BT ? rsrc(B + (size_t)n0 * Kd, (size_t)br * Kd * 8) : rsrc(B, (size_t)Kd * Nc * 8 + 8);
+        // of the plain B the rows of this block's k range; the last pair of an odd row length
+        // ends 8 bytes past the last row
+        kb = kbeg;
+        rb = BT ? rsrc(B + (size_t)n0 * Kd, (size_t)br * Kd * 8)
+                : rsrc(B + (size_t)kbeg * Nc, (size_t)(kend - kbeg) * Nc * 8 + 8);
         bstep = (unsigned)Nc * 8;
 #pragma unroll
         for (int i = 0; i < AI; i++) {
@@ -82,7 +86,7 @@ struct StreamTile {
 #pragma unroll
         for (int i = 0; i < BI; i++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void *)(buf + AS + 128 * (wv + 8 * i)),
-                                                     16, (int)bo[i], BT ? k0 * 8 : (int)((unsigned)k0 * bstep), 0, 0);
+                                                     16, (int)bo[i], BT ? k0 * 8 : (int)((unsigned)(k0 - kb) * bstep), 0, 0);
     }
     // a last k tile of kt < 16, zeros beyond it
     __device__ __forceinline__ void stage_tail(const double *A, const double *B, int Mr, int Nc, int Kd, int m0, int n0,
@@ -170,13 +174,13 @@ __global__ __launch_bounds__(512) void k_gemm_f64_stream(int Mr, int Nc, int Kd,
     const int nb = gridDim.x, bx = blockIdx.x, ntn = cdivg(Nc, ST::BN);
     const int tile = nb % 8 == 0 ? (bx % 8) * (nb / 8) + bx / 8 : bx, tm = tile / ntn, tn = tile - tm * ntn;
     const int m0 = tm * ST::BM, n0 = tn * ST::BN;
-    const int kbeg = blockIdx.z * kchunk, kend = min(Kd, kbeg + kchunk);
+    const int kbeg = blockIdx.z * kchunk, kend = max(kbeg, min(Kd, kbeg + kchunk));
     const bool store = C != nullptr;   // energies alone need no W
     C += (size_t)blockIdx.z * Mr * Nc;
     double4_t acc[TM][TN];
     ST st;
-    st.init(A, B, Mr, Nc, Kd, m0, n0);
-    st.run(A, B, Mr, Nc, Kd, m0, n0, kbeg, max(kbeg, kend), buf0, buf1, acc);
+    st.init(A, B, Mr, Nc, Kd, m0, n0, kbeg, kend);
+    st.run(A, B, Mr, Nc, Kd, m0, n0, kbeg, kend, buf0, buf1, acc);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3;
     double *red = buf1;   // [4][BM]; the tail left it free
     if constexpr (EPI) __syncthreads();
@@ -239,9 +243,14 @@ static int int_zeta_g(double z) {
 
 static const int kTile[kGemmTiles][2] = {{4, 2}, {2, 2}, {2, 1}};   // (TM, TN): 128 x 128, 64 x 128, 64 x 64
 
-// the byte offsets of a tile's rows and of the whole plain B stay within 31 bits
-bool gemm_stream_ok(int M, int d) {
-    return (size_t)192 * std::max(M, d) * 8 < (1ull << 31) && (size_t)M * d * 8 + 8 < (1ull << 31);
+// Byte offsets stay within 31 bits: those of a tile's rows of both matrices (K), those of its
+// rows of W and of a part's rows of the plain Xs (G).  64-bit addresses of the tiles staged
+// through registers reach further, at 394 us against 338 (2048 x 2701 x 2000).
+constexpr size_t kReach = (size_t)1 << 31;
+static int part_rows(int parts, int M) { return (cdivg(M, parts) + kGK - 1) / kGK * kGK; }
+bool gemm1_stream_ok(int d) { return (size_t)128 * d * 8 < kReach; }
+bool gemm2_stream_ok(int parts, int M, int d) {
+    return (size_t)128 * M * 8 < kReach && (size_t)part_rows(parts, M) * d * 8 + 8 < kReach;
 }
 int gemm_stream_ntile(int t, int M) { return cdivg(M, 64 * kTile[t][1]); }
 
@@ -267,7 +276,7 @@ void launch_gemm1_f64_stream(int t, int nc, int M, int d, const double *X, const
 }
 template <int TM, int TN>
 static void stream2_go(int nc, int M, int d, int parts, const double *W, const double *Xs, double *out, hipStream_t s) {
-    const int kchunk = (cdivg(M, parts) + kGK - 1) / kGK * kGK;
+    const int kchunk = part_rows(parts, M);
     hipLaunchKernelGGL((k_gemm_f64_stream<false, false, 0, TM, TN>), dim3(cdivg(nc, 32 * TM) * cdivg(d, 64 * TN), 1, parts),
                        dim3(512), 0, s, nc, d, M, kchunk, W, Xs, out, (const double *)nullptr, 0.0, 0, (double *)nullptr);
 }

@@ -136,10 +136,11 @@ void launch_soap_bwd(const SoapDev &sp, int nc, const int *centres, const int *Z
 
 // GEMMs
 // Tile configuration `cfg` in [0, kGemmTiles): 128 x 128, 64 x 128, 64 x 64 (gapx_gemm64.hip); a product
-// whose byte offsets pass 31 bits (gemm_stream_ok) and those of the GAP variance, whose digits
+// whose byte offsets pass 31 bits (gemm1_stream_ok, gemm2_stream_ok) and those of the GAP variance, whose digits
 // depend on the order of summation, run on 64 x 64 tiles staged through registers.
 constexpr int kGemmTiles = 3;
-bool gemm_stream_ok(int M, int d);
+bool gemm1_stream_ok(int d);
+bool gemm2_stream_ok(int parts, int M, int d);
 int gemm_stream_ntile(int cfg, int M);
 void launch_gemm1_f64_stream(int cfg, int nc, int M, int d, const double *X, const double *Xs, const double *wvec,
                              double zeta, double *W, double *e_part, hipStream_t s);

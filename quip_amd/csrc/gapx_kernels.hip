@@ -1750,7 +1750,7 @@ static int int_zeta(double z) {
 
 void launch_gemm1_f64(int cfg, int nc, int M, int d, const double *X, const double *Xs, const double *wvec,
                       double zeta, double *W, double *e_part, int *ntile_out, hipStream_t s) {
-    const bool stream = gemm_stream_ok(M, d);
+    const bool stream = gemm1_stream_ok(d);
     *ntile_out = stream ? gemm_stream_ntile(cfg, M) : cdiv(M, 64);
     if (nc <= 0) return;
     if (stream) {
@@ -1783,7 +1783,7 @@ void launch_gemm2_f64(int cfg, int parts, int nc, int M, int d, const double *W,
                       double *Gparts, hipStream_t s) {
     if (nc <= 0) return;
     double *out = parts > 1 ? Gparts : G;
-    if (gemm_stream_ok(M, d)) {
+    if (gemm2_stream_ok(parts, M, d)) {
         launch_gemm2_f64_stream(cfg, parts, nc, M, d, W, Xs, out, s);
     } else {
         const int kchunk = (cdiv(M, parts) + 15) / 16 * 16;
