@@ -1308,17 +1308,6 @@ static int connect(gapx_model *m, Engine &eg, int S, const int *atom_off, const 
     return GAPX_OK;
 }
 
-// Scratch outputs.  Growing them frees the old blocks, so callers that hand
-// these buffers in as outputs size them first.
-static int ensure_outputs(Workspace &w, int S, int N) {
-    CHK(w.f.ensure((size_t)N * 24 + 24));
-    CHK(w.le.ensure((size_t)N * 8 + 8));
-    CHK(w.lv.ensure((size_t)N * 72 + 72));
-    CHK(w.e.ensure((size_t)S * 8 + 8));
-    CHK(w.vir.ensure((size_t)S * 72 + 72));
-    return GAPX_OK;
-}
-
 static SoapDev soap_dev(const Coord &c) {
     SoapDev sp;
     sp.rc = c.rc; sp.ctw = c.ctw; sp.alpha = 0.5 / (c.sigma * c.sigma); sp.cw = c.cw; sp.u00 = c.u00;
@@ -1907,7 +1896,6 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
         CHK(w.pairVE.ensure((size_t)(P + 1) * 8));
         CHK(w.varsite.ensure((size_t)(N + 1) * 8));
     }
-    CHK(ensure_outputs(w, S, N));
     for (size_t k = 0; k < NCOORD; k++) {
         Coord &c = *m->coords[k];
         const int nc = (int)eg.h_centres[k].size();
@@ -1928,11 +1916,19 @@ int gapx::eval_batch(gapx_model *m, Engine &eg, int S, const int *atom_off, cons
                 tunes[k].fparts = 0;
         }
     }
-    double *o_e = (want & GAPX_WANT_E) && d_e ? d_e : w.e.as<double>();
-    double *o_v = (want & GAPX_WANT_V) && d_v ? d_v : w.vir.as<double>();
-    double *o_f = (want & GAPX_WANT_F) && d_f ? d_f : w.f.as<double>();
-    double *o_le = (want & GAPX_WANT_LOCAL_E) && d_le ? d_le : w.le.as<double>();
-    double *o_lv = (want & GAPX_WANT_LOCAL_V) && d_lv ? d_lv : w.lv.as<double>();
+    // results that the caller takes go to its buffers, the others to scratch
+    double *o_e, *o_v, *o_f, *o_le, *o_lv;
+    auto output = [&](unsigned bit, double *given, DBuf &scratch, size_t n, double **o) -> int {
+        const bool taken = (want & bit) && given;
+        if (!taken) CHK(scratch.ensure((n + 1) * 8));
+        *o = taken ? given : scratch.as<double>();
+        return GAPX_OK;
+    };
+    CHK(output(GAPX_WANT_E, d_e, w.e, S, &o_e));
+    CHK(output(GAPX_WANT_V, d_v, w.vir, (size_t)S * 9, &o_v));
+    CHK(output(GAPX_WANT_F, d_f, w.f, (size_t)N * 3, &o_f));
+    CHK(output(GAPX_WANT_LOCAL_E, d_le, w.le, N, &o_le));
+    CHK(output(GAPX_WANT_LOCAL_V, d_lv, w.lv, (size_t)N * 9, &o_lv));
 
     // The launch sequence (stage events only when timing, never inside a graph).
     double *pairE = has_d2b ? w.pairE.as<double>() : nullptr;
@@ -2237,7 +2233,6 @@ int gapx::calc_host(gapx_model *m, Engine &eg, int S, const int *atom_off, const
     Workspace &w = eg.ws;
     hipStream_t s = eg.stream;
     CHK(w.pos.ensure((size_t)N * 24 + 24));
-    CHK(ensure_outputs(w, S, N));   // before taking the output pointers below
     // The results asked for lie one after the other on the device and in pinned memory: one copy
     struct Out { bool on; double *dst; size_t n, off; };
     Out o[8] = {{(want & GAPX_WANT_E) != 0, e, (size_t)S, 0},

@@ -104,7 +104,7 @@ static size_t engine_bytes(const Engine &eg) {
                           &w.nb_r, &w.nb_d, &w.pairF, &w.pairE, &w.esite, &w.X, &w.norm, &w.cbuf, &w.W, &w.Wf,
                           &w.e_part, &w.G, &w.Gparts, &w.split_ws, &w.f, &w.le, &w.lv, &w.e, &w.vir, &w.minmax,
                           &w.last_pos, &w.skin_flags, &w.cmask, &w.t1_j, &w.t1_shift, &w.t1_r, &w.t2_i, &w.t2_k,
-                          &w.nl_flags, &w.spart, &w.cpos, &w.cms})
+                          &w.nl_flags, &w.spart, &w.cpos, &w.cms, &w.hout})
         b += x->cap;
     for (const DBuf &x : w.centres) b += x.cap;
     return b;
