@@ -178,8 +178,9 @@ void launch_gp_finish_f32(int nc, int d, int parts, const float *Gparts, double 
                           const int *centres, const double *e_part, double *esite, hipStream_t s);
 // mixed precision forms: Xs pre-split into hi/lo (bf16 or fp16) copies, row- and column-major
 // W is scaled by wscale (a power of two) before its hi/lo split; GEMM2 divides it out.
-// lds_mode: -1 the 128 x 128 LDS tiles once they fill the GPU, else 64 x 64; 0 / 1 force
-// the 64 x 64 / 128 x 128 tiles (an element's MFMA passes run in the same order in both)
+// lds_mode: -1 the LDS tiles once they fill the GPU, else 64 x 64; 0 / 1 force the 64 x 64 / the
+// LDS tiles, of 128 or 256 by their number (an element's MFMA passes run in the same order in all)
+int gemm_split_edge(bool second, int rows, int cols, int ldk, int lds_mode);
 void launch_gemm1_split(int prec, int nc, int M, int d, int dpad, int lds_mode, const double *X, const void *Xs_hi,
                         const void *Xs_lo, const double *wvec, double zeta, double wscale, float *Wf,
                         double *e_part, int *ntile_out, void *xsplit_ws, hipStream_t s);

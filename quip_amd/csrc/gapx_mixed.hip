@@ -419,12 +419,10 @@ __global__ __launch_bounds__(256) void k_gemm2_split_lds(int nc, int d, int Mpad
 
 // 128 x 128 tiles when they alone fill the GPU (two per CU); 64 x 64 tiles otherwise
 // (lds_mode: -1 this rule, 0 the 64 x 64 tiles, 1 the LDS tiles)
-static bool use_lds_tiles(int rows, int cols, int lds_mode = -1) {
+static bool use_lds_tiles(int rows, int cols, int lds_mode) {
     if (lds_mode >= 0) return lds_mode == 1;
     return (long)cdivm(rows, kLT) * cdivm(cols, kLT) >= 512;
 }
-static bool use_big_tiles(int rows, int cols, int ldk, int per_round);
-
 
 // LDS rows of the fused split kernel: no padding; 16-byte vectors XOR-swizzled, vector c
 // of row r at c ^ (r & XSM), so that the rows one fragment read touches fall on distinct
@@ -1189,9 +1187,12 @@ static int int_zeta_m(double z) {
 // Measured at 2720 and 2016 k: GEMM 1 256 tiles 193-210 us a full round (167 us from 64 tiles on),
 // 128 tiles 102-124 (256 of them), 152-164 (512), 228-270 (720), 298-319 us (1008); GEMM 2
 // 119-155 (132 tiles), 129-152 (253) against 156-170 (528), 220-230 us (990).
-static bool use_big_tiles(int rows, int cols, int ldk, int per_round) {
+// The tile edge of a split GEMM of rows x cols over ldk (second: GEMM 2).
+int gemm_split_edge(bool second, int rows, int cols, int ldk, int lds_mode) {
+    if (!use_lds_tiles(rows, cols, lds_mode)) return 64;
     const long big = (long)cdivm(rows, kBT) * cdivm(cols, kBT), small = (long)cdivm(rows, kLT) * cdivm(cols, kLT);
-    return small >= per_round * ((big + 255) / 256) && (size_t)kBT * ldk * 2 < kBBytes;
+    const bool use_big = small >= (second ? 430 : 600) * ((big + 255) / 256) && (size_t)kBT * ldk * 2 < kBBytes;
+    return use_big ? kBT : kLT;
 }
 
 void launch_gemm1_split(int prec, int nc, int M, int d, int dpad, int lds_mode, const double *X, const void *Xs_hi,
@@ -1199,11 +1200,10 @@ void launch_gemm1_split(int prec, int nc, int M, int d, int dpad, int lds_mode, 
                         double *e_part, int *ntile_out, void *xsplit_ws, hipStream_t s) {
     const int Mpad = (M + 31) / 32 * 32;
     dim3 grid(cdivm(nc, 64), cdivm(M, 64));
-    const bool lds = use_lds_tiles(nc, M, lds_mode);
-    const bool big = lds && use_big_tiles(nc, M, dpad, 600);
-    const int edge = big ? kBT : kLT;
+    const int edge = gemm_split_edge(false, nc, M, dpad, lds_mode);
+    const bool lds = edge > 64, big = edge == kBT;
     const int ntn = cdivm(M, edge), nblk = cdivm(nc, edge) * ntn;
-    *ntile_out = lds ? ntn : (int)grid.y;
+    *ntile_out = ntn;
     if (nc <= 0) return;
     const size_t xsz = (size_t)((nc + 63) / 64 * 64) * dpad;
     char *xs = (char *)xsplit_ws;
@@ -1365,8 +1365,8 @@ void launch_gemm2_split(int prec, int nc, int M, int d, int dpad, int Mpad, int 
     const char *wf = (const char *)Wf;
     const void *Whi = wf, *Wlo = wf + (size_t)nc * Mpad * 2;
     const double inv = 1.0 / wscale;
-    if (use_lds_tiles(nc, d, lds_mode) && use_big_tiles(nc, d, Mpad, 430)) {
-        const int ntn = cdivm(d, kBT), nblk = cdivm(nc, kBT) * ntn;
+    const int edge = gemm_split_edge(true, nc, d, Mpad, lds_mode), ntn = cdivm(d, edge), nblk = cdivm(nc, edge) * ntn;
+    if (edge == kBT) {
         if (prec == 1)
             hipLaunchKernelGGL(k_gemm2_split_big<1>, dim3(nblk), dim3(512), 0, s, nc, d, Mpad, ntn,
                                (const __bf16 *)Whi, (const __bf16 *)Wlo, (const __bf16 *)XsT_hi,
@@ -1377,8 +1377,7 @@ void launch_gemm2_split(int prec, int nc, int M, int d, int dpad, int Mpad, int 
                                (const _Float16 *)XsT_lo, inv, G);
         return;
     }
-    if (use_lds_tiles(nc, d, lds_mode)) {
-        const int ntn = cdivm(d, kLT), nblk = cdivm(nc, kLT) * ntn;
+    if (edge == kLT) {
         if (prec == 1)
             hipLaunchKernelGGL(k_gemm2_split_lds<1>, dim3(nblk), dim3(256), 0, s, nc, d, Mpad, ntn,
                                (const __bf16 *)Whi, (const __bf16 *)Wlo, (const __bf16 *)XsT_hi,
