@@ -649,9 +649,11 @@ struct BwdLds {
 // centres at 8/6: 1.09 -> 0.63 ms against a lane per neighbour reading dE/dc' from LDS (VALU issue
 // 44%, matrix pipe 26% of it); 32768 SiC centres at 12/8: 3.80 -> 0.90 ms.  A wavefront per centre and
 // 2 wavefronts per SIMD: with spills at 3 the reloads queue behind the data on their way (1.07 ms).
+// Two species up to l = 4 take 3, with 183 to 190 registers cut to 168: 55296 centres at 5/4 868 -> 798 us.
 // SP: the number of species where it is fixed at compile time, else 0.
+constexpr int bwd_waves(int L, int SP) { return L <= 4 && SP == 2 ? 3 : 2; }
 template <int N, int L, int NW, int SP>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_soap_bwd_x(
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(bwd_waves(L, SP), 8))) void k_soap_bwd_x(
     SoapDev sp, int nc, int cpb, const int *__restrict__ centres, const int *__restrict__ Z,
     const int *__restrict__ nb_off, const int *__restrict__ nb_j, const double *__restrict__ nb_r,
     const double *__restrict__ nb_d, const double *__restrict__ X, const double *__restrict__ G,
@@ -663,7 +665,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 8)))
     constexpr bool AHEAD = SP && QR <= 4;                              // X and G of the next centre in registers
     constexpr int UN = SP ? (NQ * SP + NW - 1) / NW : 1;               // quads of groups per wavefront (one species each)
     constexpr bool CAHEAD = SP && UN * SP * NA <= 12;                  // the next centre's c likewise
-    static_assert(SP <= 1 || NW == 2 * SP, "wavefronts are dealt evenly to the species");
+    static_assert(SP <= 1 || NW % SP == 0, "wavefronts are dealt evenly to the species");
     const int S = SP ? SP : sp.S, KLM = S * N * LM, d = SP ? DC + 1 : sp.dim;
     const int SB = SP ? SP : SB_;
     const bool p_lds = SP || p_lds_;
@@ -992,11 +994,13 @@ int soap_fast_supported(int n, int L) {
 }
 
 // What a block may take: within it the power spectrum, c and dE/dp are kept in LDS where
-// they fit, so that at least two blocks share a CU; many species go through memory.
-constexpr int kSoapLdsCap = 60 * 1024;   // without the constant tables (at most 4 KB)
+// they fit, so that two blocks of four wavefronts, what the registers of bases past l = 4 allow,
+// share a CU (160 KB; the constant tables take up to 3 KB more); the rest goes through memory.
+// 22400 centres of five species at 6/6: the adjoint 3326 us with dE/dp in memory.
+constexpr int kSoapLdsCap = 76 * 1024;
 
 struct FwdPlan {
-    bool split, p_lds, c_lds;
+    bool own, split, p_lds, c_lds;
     int nw;
     size_t lds;
 };
@@ -1004,32 +1008,46 @@ static size_t table_lds(const SoapDev &sp) {
     const int nq4 = (soap_groups(sp.L) + 3) / 4 * 4;
     return (size_t)(sp.n * sp.n + 24 + 4 * nq4 + sp.L + 1) * 8 + 4 * nq4 * 4;
 }
-static FwdPlan fwd_plan(const SoapDev &sp, bool split) {
+// A wavefront per species: its own neighbours with all harmonics, and its own rows of dE/dc
+// (bases up to 8/6, two to four species).  Otherwise four wavefronts share a centre, m < 4 and
+// m >= 4 apart.  A small basis leaves those little to do between their barriers, and species
+// that are not fixed at compile time have c and dE/dp read where they are needed.  Forward
+// + adjoint of 55296 centres at 5/4: two species 868 + 1237 -> 541 + 868 us, four 938 + 1528 ->
+// 626 + 875; of 8/6, four species: 1646 + 3510 -> 1196 + 1549.  Two species have half as many
+// wavefronts this way: up to 512 centres, whose four wavefronts the card holds at once, these
+// are faster (500 centres at 8/6 53 us against 61, 600 centres 67 against 63).
+static bool wave_per_species(const SoapDev &sp, int nc) {
+    return sp.n <= 8 && sp.L <= 6 && sp.S >= (nc > 512 ? 2 : 3) && sp.S <= 4;
+}
+static FwdPlan fwd_plan(const SoapDev &sp, bool own, bool split) {
     FwdPlan f;
     const int NA = (sp.n + 3) / 4;
-    f.split = split || sp.S > 1;
-    f.nw = sp.S > 1 ? 4 : split ? 2 : 1;
+    f.own = own;
+    f.split = split || (sp.S > 1 && !own);
+    f.nw = own ? sp.S : sp.S > 1 ? 4 : split ? 2 : 1;
     f.p_lds = f.c_lds = true;
     if (FwdLds(NA, sp.L, sp.S, f.nw, sp.dim, true, true).total > kSoapLdsCap) f.p_lds = false;
     if (FwdLds(NA, sp.L, sp.S, f.nw, sp.dim, f.p_lds, true).total > kSoapLdsCap) f.c_lds = false;
     f.lds = FwdLds(NA, sp.L, sp.S, f.nw, sp.dim, f.p_lds, f.c_lds).total + table_lds(sp);
-    return f;
+    // the form of fixed species keeps both in LDS
+    return own && !(f.p_lds && f.c_lds) ? fwd_plan(sp, false, split) : f;
 }
 struct BwdPlan {
-    bool p_lds;
+    bool own, p_lds;
     int nw, SB;
     size_t lds;
 };
-static BwdPlan bwd_plan(const SoapDev &sp, bool split) {
+static BwdPlan bwd_plan(const SoapDev &sp, bool own, bool split) {
     BwdPlan b;
     const int NA = (sp.n + 3) / 4;
-    b.nw = sp.S > 1 ? 4 : split ? 2 : 1;
+    b.own = own;
+    b.nw = own ? sp.S : sp.S > 1 ? 4 : split ? 2 : 1;
     b.p_lds = true;
     b.SB = sp.S;
     if (BwdLds(NA, sp.L, sp.S, sp.S, b.nw, sp.dim, true).total > kSoapLdsCap) b.p_lds = false;
     while (b.SB > 1 && BwdLds(NA, sp.L, sp.S, b.SB, b.nw, sp.dim, b.p_lds).total > kSoapLdsCap) b.SB--;
     b.lds = BwdLds(NA, sp.L, sp.S, b.SB, b.nw, sp.dim, b.p_lds).total + table_lds(sp);
-    return b;
+    return own && !(b.p_lds && b.SB == sp.S) ? bwd_plan(sp, false, split) : b;
 }
 
 // What a model's descriptors are admitted by (the size a level-by-level adjoint with its
@@ -1053,17 +1071,27 @@ bool launch_soap_fwd_fast(const SoapDev &sp, int nc, const int *centres, const i
     if (!soap_fast_supported(sp.n, sp.L)) return false;
     ensure_soap_constants();
     if (nc <= 0) return true;
+    // More species than two keep the harmonics together up to l = 4, where m >= 4 is one pair of
+    // groups and would run the recursions again (22118 centres of five species at 6/4: 1007 -> 886
+    // us; at 6/6, four species: 1259 together, 1190 apart).
     // Two wavefronts per centre (m < 4, m >= 4) while a wavefront per centre would not fill the
     // GPU (si4055: 44 -> 30 us), and where the accumulators of all groups (2 x 29 x 3 registers
     // at 12/8) leave too few registers; one otherwise (no recursion is run twice).
-    const FwdPlan f = fwd_plan(sp, sp.n > 8 || sp.L > 6 || nc < 4096);
+    const FwdPlan f = fwd_plan(sp, wave_per_species(sp, nc), sp.n > 8 || sp.L > 6 || nc < 4096);
     const int cpb = centres_per_block(nc), nblk = (nc + cpb - 1) / cpb;
 #define GO(NN, LL, NW, SPLIT, SP)                                                                                  \
     hipLaunchKernelGGL((k_soap_fwd_x<NN, LL, NW, SPLIT, SP>), dim3(nblk), dim3(64 * NW), f.lds, s, sp, nc, cpb,    \
                        centres, Z, nb_off, nb_j, nb_r, nb_d, X, norm, cbuf, (int)f.p_lds, (int)f.c_lds)
 #define LAUNCH(NN, LL)                                                                                             \
     if (sp.n == NN && sp.L == LL) {                                                                                \
-        if (sp.S > 2 || !f.p_lds || !f.c_lds) GO(NN, LL, 4, true, 0);                                              \
+        if constexpr (NN <= 8 && LL <= 6)                                                                          \
+            if (f.own) {                                                                                           \
+                if (sp.S == 2) GO(NN, LL, 2, false, 2);                                                            \
+                else if (sp.S == 3) GO(NN, LL, 3, false, 3);                                                       \
+                else GO(NN, LL, 4, false, 4);                                                                      \
+                return true;                                                                                       \
+            }                                                                                                      \
+        if (sp.S > 2 || !f.p_lds || !f.c_lds) GO(NN, LL, 4, (LL > 4), 0);                                          \
         else if (sp.S == 2) GO(NN, LL, 4, true, 2);                                                                \
         else if (f.split) GO(NN, LL, 2, true, 1);                                                                  \
         else if constexpr (NN <= 8 && LL <= 6) GO(NN, LL, 1, false, 1);                                            \
@@ -1081,13 +1109,20 @@ bool launch_soap_bwd_fast(const SoapDev &sp, int nc, const int *centres, const i
     if (!soap_fast_supported(sp.n, sp.L)) return false;
     ensure_soap_constants();
     if (nc <= 0) return true;
-    const BwdPlan b = bwd_plan(sp, sp.n > 8 || sp.L > 6 || nc < 4096);
+    const BwdPlan b = bwd_plan(sp, wave_per_species(sp, nc), sp.n > 8 || sp.L > 6 || nc < 4096);
     const int cpb = centres_per_block(nc), nblk = (nc + cpb - 1) / cpb;
 #define GO(NN, LL, NW, SP)                                                                                         \
     hipLaunchKernelGGL((k_soap_bwd_x<NN, LL, NW, SP>), dim3(nblk), dim3(64 * NW), b.lds, s, sp, nc, cpb, centres,  \
                        Z, nb_off, nb_j, nb_r, nb_d, X, G, norm, cbuf, pairF, (int)b.p_lds, b.SB, (int)add)
 #define LAUNCH(NN, LL)                                                                                             \
     if (sp.n == NN && sp.L == LL) {                                                                                \
+        if constexpr (NN <= 8 && LL <= 6)                                                                          \
+            if (b.own) {                                                                                           \
+                if (sp.S == 2) GO(NN, LL, 2, 2);                                                                   \
+                else if (sp.S == 3) GO(NN, LL, 3, 3);                                                              \
+                else GO(NN, LL, 4, 4);                                                                             \
+                return true;                                                                                       \
+            }                                                                                                      \
         if (sp.S > 2 || !b.p_lds || b.SB < sp.S) GO(NN, LL, 4, 0);                                                 \
         else if (sp.S == 2) GO(NN, LL, 4, 2);                                                                      \
         else if (b.nw == 2) GO(NN, LL, 2, 1);                                                                      \
