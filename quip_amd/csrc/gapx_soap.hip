@@ -649,9 +649,12 @@ struct BwdLds {
 // centres at 8/6: 1.09 -> 0.63 ms against a lane per neighbour reading dE/dc' from LDS (VALU issue
 // 44%, matrix pipe 26% of it); 32768 SiC centres at 12/8: 3.80 -> 0.90 ms.  A wavefront per centre and
 // 2 wavefronts per SIMD: with spills at 3 the reloads queue behind the data on their way (1.07 ms).
-// Two species up to l = 4 take 3, with 183 to 190 registers cut to 168: 55296 centres at 5/4 868 -> 798 us.
-// SP: the number of species where it is fixed at compile time, else 0.
-constexpr int bwd_waves(int L, int SP) { return L <= 4 && SP == 2 ? 3 : 2; }
+// Up to l = 4, two species (183 to 190 registers cut to 168: 55296 centres at 5/4 868 -> 798 us)
+// and those not fixed at compile time (13440 centres of five at 5/4 1240 -> 928 us) take 3.
+// SP: the number of species where it is fixed at compile time, else 0; then X, G and c are
+// fetched several at a time, c a species ahead of its product (22400 centres of three
+// species at 12/6: 3346 -> 2347 us).
+constexpr int bwd_waves(int L, int SP) { return L <= 4 && (SP == 0 || SP == 2) ? 3 : 2; }
 template <int N, int L, int NW, int SP>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(bwd_waves(L, SP), 8))) void k_soap_bwd_x(
     SoapDev sp, int nc, int cpb, const int *__restrict__ centres, const int *__restrict__ Z,
@@ -728,6 +731,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(bwd_wav
 #pragma unroll
             for (int i = 0; i < QR; i++) dot += xr[i] * gr[i];
         } else {
+#pragma unroll 4
             for (int q = threadIdx.x; q < d; q += 64 * NW) dot += x[q] * gg[q];
         }
         dot = wave_sum_s(dot);
@@ -746,6 +750,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(bwd_wav
                 if (q < d - 1) P[q] = gr[i] - xr[i] * dot;
             }
         } else if (p_lds) {
+#pragma unroll 4
             for (int q = threadIdx.x; q < d - 1; q += 64 * NW) P[q] = gg[q] - x[q] * dot;
         }
         block_lds_sync<NW>();
@@ -807,12 +812,25 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(bwd_wav
                     double D1[NA];
 #pragma unroll
                     for (int u = 0; u < NA; u++) D1[u] = 0.0;
+                    double cn[NA];   // a column of c ahead of its product
+                    auto load_col = [&](int sj) {
+#pragma unroll
+                        for (int kk = 0; kk < NA; kk++) {
+                            const int aj = 4 * kk + k4;
+                            cn[kk] = sj < S && (N % 4 == 0 || aj < N) && pos != 0xffff ? cg[(sj * N + aj) * LM + pos] : 0.0;
+                        }
+                    };
+                    load_col(0);
                     for (int sj = 0; sj < S; sj++) {
+                        double cc[NA];
+#pragma unroll
+                        for (int kk = 0; kk < NA; kk++) cc[kk] = cn[kk];
+                        load_col(sj + 1);
 #pragma unroll
                         for (int kk = 0; kk < NA; kk++) {
                             const int aj = 4 * kk + k4, jb = sj * N + aj;
                             const bool okj = N % 4 == 0 || aj < N;
-                            const double cb = okj && pos != 0xffff ? cg[jb * LM + pos] : 0.0;
+                            const double cb = cc[kk];
 #pragma unroll
                             for (int u = 0; u < NA; u++) {
                                 const int ai = 4 * u + i4, ia = s * N + ai;

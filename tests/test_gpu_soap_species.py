@@ -1,5 +1,5 @@
 """GPU: the SOAP kernels that give each species a wavefront (bases up to 8/6, two to four
-species; two species from 513 centres on) against the oracle: partial tiles, a species that is
+species; two species from 513 centres on), and five species beside them, against the oracle: partial tiles, a species that is
 absent, centres without neighbours and with more than one staging pass of them, and batches
 with 512 and 513 centres."""
 import numpy as np
@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("described,present", [((14, 6), (14, 6)), ((14, 6, 1), (14, 1, 6)), ((14, 6, 1), (14, 6)),
-                                               ((1, 6, 8, 14), (14, 6, 1, 8)), ((1, 6, 8, 14), (14, 8, 9))])
+                                               ((1, 6, 8, 14), (14, 6, 1, 8)), ((1, 6, 8, 14), (14, 8, 9)),
+                                               ((1, 6, 7, 8, 14), (14, 6, 1, 8, 7))])
 @pytest.mark.parametrize("n,lm", [(4, 4), (5, 4), (8, 4), (6, 6), (8, 6)])
 def test_species_match_oracle(described, present, n, lm, tmp_path):
     shapes = [_gas(21, present, 30, 6.5), _gas(22, present, 25, 9.0), _gas(23, present, 6, 24.0)]
