@@ -2349,19 +2349,12 @@ extern "C" int gapx_calc_device_ex(gapx_model *m, int N, const double *d_pos, co
 // in the reference's instance order (print_gap_variance, IPModel_GAP.f95:506-516):
 // soap, one per centre atom (atoms[2k] = centre, atoms[2k+1] = -1, cutoff_sq = 1);
 // distance_2b, one per directed pair (i, j) with i ascending and j in i's neighbour order.
-// Read from the device, whose lists are still that calc's.
-static int read_instances(gapx_model *m, Engine &eg, int coord, VarInstances &out) {
+// put(variance, cutoff_sq, a, b) for each, read from the device, whose lists are still that calc's.
+template <class F> static int each_instance(gapx_model *m, Engine &eg, int coord, F put) {
     HIPCHK(hipSetDevice(m->device));
     HIPCHK(hipStreamSynchronize(eg.stream));
     Workspace &w = eg.ws;
-    out = VarInstances();
     if (!eg.var_has[coord]) return GAPX_OK;   // a coordinate the last calc skipped (only_descriptor)
-    auto put = [&](double var, double c2, int a, int b) {
-        out.var.push_back(var);
-        out.cut2.push_back(c2);
-        out.atoms.push_back(a);
-        out.atoms.push_back(b);
-    };
     if (m->coords[coord]->kind == 1) {
         const auto &cen = eg.h_centres[coord];
         std::vector<double> v(cen.size());
@@ -2392,14 +2385,19 @@ extern "C" int gapx_descriptor_variances(gapx_model *m, int coord, int max_entri
     if (coord < 0 || coord >= (int)m->coords.size()) return fail(GAPX_E_ARG, "coordinate %d out of range", coord);
     Engine &eg = *m->eng;
     if (!eg.var_valid) return fail(GAPX_E_ARG, "no variance formed by the last calc (ask for GAPX_WANT_VARIANCE)");
-    VarInstances read;
-    if (eg.var_kept.empty()) CHK(read_instances(m, eg, coord, read));
-    const VarInstances &vi = eg.var_kept.empty() ? read : eg.var_kept[coord];
-    const int n = (int)vi.var.size();
-    for (int k = 0; k < std::min(n, max_entries); k++) {
-        if (variance) variance[k] = vi.var[k];
-        if (cutoff_sq) cutoff_sq[k] = vi.cut2[k];
-        if (atoms) { atoms[2 * k] = vi.atoms[2 * k]; atoms[2 * k + 1] = vi.atoms[2 * k + 1]; }
+    int n = 0;
+    auto put = [&](double var, double c2, int a, int b) {
+        if (n < max_entries) {
+            if (variance) variance[n] = var;
+            if (cutoff_sq) cutoff_sq[n] = c2;
+            if (atoms) { atoms[2 * n] = a; atoms[2 * n + 1] = b; }
+        }
+        n++;
+    };
+    if (eg.var_kept.empty()) CHK(each_instance(m, eg, coord, put));
+    else {
+        const VarInstances &vi = eg.var_kept[coord];
+        for (size_t k = 0; k < vi.var.size(); k++) put(vi.var[k], vi.cut2[k], vi.atoms[2 * k], vi.atoms[2 * k + 1]);
     }
     *n_entries = n;
     return GAPX_OK;
@@ -2593,7 +2591,13 @@ extern "C" int gapx_descriptors(gapx_model *m, int coord, int N, const double *p
     if (N > 0 && !pos) return fail(GAPX_E_ARG, "positions are NULL");
     if (eg.var_valid && eg.var_kept.empty()) {   // the lists and centres of the last calc's variances go
         std::vector<VarInstances> kept(m->coords.size());
-        for (size_t k = 0; k < kept.size(); k++) CHK(read_instances(m, eg, (int)k, kept[k]));
+        for (size_t k = 0; k < kept.size(); k++)
+            CHK(each_instance(m, eg, (int)k, [&](double var, double c2, int a, int b) {
+                kept[k].var.push_back(var);
+                kept[k].cut2.push_back(c2);
+                kept[k].atoms.push_back(a);
+                kept[k].atoms.push_back(b);
+            }));
         eg.var_kept.swap(kept);
     }
     CHK(w.pos.ensure((size_t)N * 24 + 24));
