@@ -25,10 +25,11 @@ struct SoapDev {
     int n, S, K, LM, dim, L;
     int species_Z[kMaxSpecies];
     const double *rb;    // n grid points r_a = a dr
-    const double *rt;    // exp(-alpha r_a^2) / 2 and 1/a of a < 12 (zero for a = 0 and a >= n): 2 x 12
-    double dr, a2dr, ia2dr, ictw;   // grid spacing, 2 alpha dr, its inverse, 1 / ctw
     const double *T;     // n x n transform, T[a*n+b]
     const int *qmap;     // dim-1 entries: (ia<<16)|(jb<<8)|l
+    // the specialised kernels' (last: ahead of T they cost the general forward 32 bytes of scratch)
+    const double *rt;    // exp(-alpha r_a^2) / 2 and 1/a of a < 12 (zero for a = 0 and a >= n): 2 x 12
+    double dr, a2dr, ia2dr, ictw;   // grid spacing, 2 alpha dr, its inverse, 1 / ctw
 };
 
 // launchers (kernels.hip)
