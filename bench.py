@@ -340,23 +340,55 @@ def stage_counters():
 SINGLE_KERNEL_STAGES = ("soap_forward", "soap_adjoint", "gemm1")
 
 
-def stage_roofline(forms, model, n_si, nc_batch):
+def library_code():
+    """The built library's bytes (its kernels' mangled names among them)."""
+    with open(L.LIB_PATH, "rb") as fh:
+        return fh.read()
+
+
+def kernel_in_library(name, code):
+    """Whether the library holds the kernel that a counter summary names, as
+    k_soap_fwd_x<8,6,1,false,1> or k_gather."""
+    base, _, args = name.rstrip(">").partition("<")
+    sym = "N4gapx%d%s" % (len(base), base)
+    if args:
+        sym += "I%sE" % "".join("Lb%dE" % (a == "true") if a in ("true", "false") else "Li%sE" % a
+                                for a in args.replace(" ", "").split(","))
+    return (sym + "E").encode() in code
+
+
+def gp_products(kernel):
+    """How many of the GP's two products (2 nc M d flop each) one launch of `kernel` forms."""
+    return 2 if kernel.startswith(("k_gp_fused", "k_gp_tile")) else 1
+
+
+def stage_roofline(forms, model, n_si, nc_batch, gp_choice):
     """Achieved HBM GB/s and FP64-VALU fraction per descriptor stage.  Stages that are one
-    kernel (forward, adjoint, the GP kernel) divide the committed per-launch bytes and
-    flops by the stage time measured in this run with HIP events on the library's stream;
-    the neighbour-list and gather stages span several kernels, so their dominant kernel
-    is priced at its kernel-trace time and the live stage time is given beside it.  The
-    GP kernels also get their MFMA fraction (algorithmic 4 nc M d; the split form runs
-    three passes)."""
+    kernel (forward, adjoint, the GP kernel or its first product) divide the committed
+    per-launch bytes and flops by the stage time measured in this run with HIP events on the
+    library's stream; the other stages span several kernels, so their dominant kernel is
+    priced at its kernel-trace time and the live stage time is given beside it.  The GP
+    kernels also get their MFMA fraction, of the products that they form (the split form
+    runs three passes).  A summary of a kernel that the library no longer holds, or of a GP
+    form other than the one this run chose, is left out."""
     cnt = stage_counters()
     if not cnt:
         return None
+    code = library_code()
     live = {"si4096_fp64": forms.get("fp64", {}).get("stage_ms", {}),
             "batch512_bf16x3": forms.get("batch512_bf16x3", {}).get("stage_ms", {})}
     centres = {"si4096_fp64": n_si, "batch512_bf16x3": nc_batch}
     out = {}
     for (wl, stage), (kernel, nbytes, flops, avg_us) in sorted(cnt.items()):
         st_ms = live.get(wl, {}).get(stage)
+        gp = stage in ("gemm1", "gemm2")
+        if not kernel_in_library(kernel, code):
+            out.setdefault(wl, {})[stage] = dict(left_out="the library holds no %s" % kernel, stage_ms_live=st_ms)
+            continue
+        if gp and wl.endswith("fp64") and (gp_products(kernel) == 2) != (gp_choice[0] == "fused"):
+            out.setdefault(wl, {})[stage] = dict(left_out="this run chose %s, not %s" % (gp_choice[0], kernel),
+                                                 stage_ms_live=st_ms)
+            continue
         if stage in SINGLE_KERNEL_STAGES and st_ms:
             t, src = st_ms * 1e-3, "HIP events, this run"
         else:
@@ -365,9 +397,9 @@ def stage_roofline(forms, model, n_si, nc_batch):
                  kernel_ms=round(t * 1e3, 4), time_source=src, stage_ms_live=st_ms,
                  hbm_GBps=round(nbytes / t / 1e9, 1), hbm_frac=round(nbytes / t / HBM_PEAK, 4),
                  fp64_valu_TFps=round(flops / t / 1e12, 3), fp64_valu_frac=round(flops / t / VALU_FP64_PEAK, 4))
-        if stage == "gemm1":   # the GP kernel: MFMA is its roof
+        if gp:   # MFMA is its roof
             c = model.coords[0]
-            alg = 4.0 * centres[wl] * c.n_sparse * c.descriptor.dim
+            alg = 2.0 * gp_products(kernel) * centres[wl] * c.n_sparse * c.descriptor.dim
             if "split" in kernel:
                 e.update(bound="mfma", algorithmic_flops=alg, mfma_flops_executed=3 * alg,
                          mfma_frac_algorithmic=round(alg / t / MFMA_BF16_PEAK, 4),
@@ -562,8 +594,8 @@ def main():
                                        "copy-kernel calibration, profiles/k_gp_fused_f64_si4096_traffic.txt")
     else:
         gp_flops = 2.0 * nc * M * d
-        roofline = dict(bound="mfma", kernel="k_gemm_f64 GEMM 1 (K = X Xs^T, fused pow/alpha epilogue; FP64 MFMA "
-                        "16x16x4)", traffic=kernel_traffic("k_gemm_f64_gemm1_si4096_traffic.txt"),
+        roofline = dict(bound="mfma", kernel="k_gemm_f64_stream GEMM 1 (K = X Xs^T, fused pow/alpha epilogue; FP64 "
+                        "MFMA 16x16x4, tiles streamed into LDS)", traffic=kernel_traffic("k_gemm_f64_gemm1_si4096_traffic.txt"),
                         traffic_source="HBM bytes per launch: FETCH_SIZE + WRITE_SIZE of this kernel scaled by a "
                                        "copy-kernel calibration, profiles/k_gemm_f64_gemm1_si4096_traffic.txt")
     achieved = gp_flops / (st["gemm1"] * 1e-3)
@@ -588,7 +620,7 @@ def main():
         if a in forms and b in forms:
             same[key] = forms[a]["atoms_per_s"] / forms[b]["atoms_per_s"]
     nc_batch = sum(len(a) for a in frames)
-    stages_roof = stage_roofline(forms, model, N, nc_batch)
+    stages_roof = stage_roofline(forms, model, N, nc_batch, gp_choice)
     dev.free()
     fp = forms["fp64"]
     mixed = [k for k in forms if k.startswith("batch512_") and "fp64" not in k]
