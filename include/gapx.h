@@ -88,7 +88,11 @@ int gapx_model_info(const gapx_model *model, int *n_coord, int coord, int *dim, 
  * (IPModel_GAP.f95:233-605) including the calc_connect it relies on
  * (Potential.f95:844-859 -> Connection.f95:1035-1310).  `nl_cutoff` <= 0 uses the
  * model cutoff (QUIP's at%cutoff after set_cutoff).  Outputs not requested in
- * `want` may be NULL. */
+ * `want` may be NULL.  A call that asks for no force, virial or local virial leaves
+ * the descriptor's adjoint out, and in FP64 the second GP product too, whose form may
+ * then be another one: its energies agree with those of a call that asks for forces to
+ * 1e-12 eV/atom (FP64; 1e-7 in the split forms), not to the last bit.  A structure of no
+ * atoms has zero energy and virial. */
 int gapx_calc(gapx_model *model, int n_atoms, const double *pos, const int *Z, const double *lattice,
               const int *pbc, double nl_cutoff, unsigned want, double *e, double *local_e, double *f,
               double *virial, double *local_virial);
@@ -275,9 +279,13 @@ int gapx_descriptors(gapx_model *model, int coord, int n_atoms, const double *po
 /* FP64 GEMM autotuner (on by default).  No counterpart in the reference.  For
  * each gpCoordinate and centre-count bucket b (2^(b-1) < n_centres <= 2^b) the
  * first evaluation times every GEMM tile shape (tile 0: 128 x 128, 1: 64 x 128, 2: 64 x 64)
- * and every GEMM 2 split-K factor in {1,2,4,8} on its own operands, and keeps the fastest.
+ * and every GEMM 2 split-K factor in {1,2,4,8} on its own operands, and for descriptors of up to
+ * 256 components the fused kernel that forms both products, and keeps the fastest.  Buckets
+ * of up to 256 centres with up to 2048 sparse points keep the fused kernel whatever it took, so
+ * that models and runs do not differ there; calls for energies alone use GEMM 1.
  * gapx_model_tuning lists the choices (up to max_entries; n_entries gets the
- * count) with the measured milliseconds of one launch. */
+ * count) with the measured milliseconds of one launch; tile -1 is the fused kernel, with its
+ * sparse-point parts in the place of the split-K factor. */
 int gapx_model_set_autotune(gapx_model *model, int on);
 
 /* Split-form autotuner (on with gapx_model_set_autotune).  No counterpart in the reference.

@@ -1338,9 +1338,11 @@ int gapx::check_batch(int S, const int *atom_off, const int *Z, const double *la
 // GEMM autotuner.  For each coordinate and centre-count bucket (ceil log2 nc) the
 // first evaluation times every GEMM 1 tile and every GEMM 2 tile x split-K factor
 // (fastest of three launches after a warm-up) with HIP events on the engine's stream, on the
-// call's own operands (X is already computed), and keeps the fastest.  Later
-// calls in the bucket reuse the choice.  Without autotuning: 64 x 64 tiles,
-// GEMM 2 with the default split-K factor.
+// call's own operands (X is already computed), and the fused form (d <= 256), and keeps the
+// fastest of the tiles and of the two forms; calls of up to 256 centres and 2048 points take
+// the fused form whatever its time (energies alone their GEMM 1 tile).  Later
+// calls in the bucket reuse the choice.  Without autotuning: the fused form, else 64 x 64
+// tiles and GEMM 2 with the default split-K factor.
 static int gemm_tune(gapx_model *m, Engine &eg, Coord &c, int nc, GemmTune &out, bool cached_only = false) {
     out = GemmTune();
     out.parts = gemm2_parts(nc, c.dim);
@@ -1423,8 +1425,9 @@ static int gemm_tune(gapx_model *m, Engine &eg, Coord &c, int nc, GemmTune &out,
         }
         best.f64_ms = fbest;
         best.f64tile = tile;
-        // up to 256 centres and 2048 points the form for few centres is the faster by a third or
-        // more (216 x 2000: 29 us against 46): a rule, so that every model takes the same
+        // up to 256 centres and 2048 points the form for few centres is the faster by 7 to 70% (3 to
+        // 253 components, 1 to 256 centres, 10 to 2048 points; 216 x 2048 of 253: 29.5 us against 31.6,
+        // 8 x 500: 13 against 21): a rule, so that every model takes the same
         const bool sure = tile && nc <= 256 && c.M <= 2048;
         best.f64parts = (st == GAPX_OK && (sure || fbest < best.g1_ms + best.g2_ms)) ? fparts : 0;
     }

@@ -292,10 +292,11 @@ __global__ __launch_bounds__(256, 2) void k_gp_tile_f64(int nc, int M, int d, in
 
 bool gp_f64_fused_supported(int d) { return d >= 1 && d <= 256; }
 
-// The 16-centre form serves up to 512 centres: on 253 components and 500 points it took 13 us
-// against 27 for 8 centres, 17 against 30 for 216 and 22 against 35 for 500; on 2000 points 21
-// against 76 (two GEMMs and their sums: 45) for 8, 36 against 81 (46) for 288, but at 997 62
-// against the GEMMs' 58.  Its parts are sums of 16 points, at most 32 of them (the partial G
+// The 16-centre form serves up to 512 centres: on 253 components and 500 points it takes 13 us
+// against 27 (and 21 of the fastest two GEMMs with their sums) for 8 centres, 16 against 30 (23)
+// for 216 and 19 against 32 (25) for 512; on 2000 points 21 against 76 (27) for 8, 31 against
+// 80 (32) for 288 and 45 against 82 (37) for 512, where the tuner takes the GEMMs; at 997 centres
+// it would take 79 against 84 (51).  Its parts are sums of 16 points, at most 32 of them (the partial G
 // rows are written and read once: 64 parts took longer at every size).
 bool gp_f64_tile_serves(int nc) { return nc <= 512; }
 int gp_f64_tile_parts_valid(int parts, int M) {

@@ -363,8 +363,8 @@ struct FwdLds {
 // which are the operands of 4x4x4 products whose four blocks are four quarters of the tile.
 // The quarters are summed through LDS once per centre, T and the power spectrum follow as
 // further 4x4x4 products.  135612 Si centres at 8/6: 1.10 -> 0.46 ms against lanes accumulating
-// c' from levels staged in LDS (700 MB of X and c written at 1.5 TB/s; VALU issue 47% and the
-// matrix pipe 21% of it); 32768 SiC centres at 12/8: 3.19 -> 0.77 ms.  SP: the number of species where it is fixed at compile time, else 0.
+// c' from levels staged in LDS (945 MB moved at 2.0 TB/s; VALU issue 50% and the matrix pipe 22%
+// of it); 32768 SiC centres at 12/8: 3.19 -> 0.77 ms.  SP: the number of species where it is fixed at compile time, else 0.
 template <int N, int L, int NW, bool SPLIT, int SP>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(N <= 8 && L <= 6 ? 3 : 2, 8))) void k_soap_fwd_x(
     SoapDev sp, int nc, int cpb, const int *__restrict__ centres, const int *__restrict__ Z,
@@ -647,7 +647,7 @@ struct BwdLds {
 // The sums over l are kept per m with the Legendre factors only; (x + i y)^m enters once at
 // the end, and a last product with unit rows sums the lanes of a neighbour.  135612 Si
 // centres at 8/6: 1.09 -> 0.63 ms against a lane per neighbour reading dE/dc' from LDS (VALU issue
-// 44%, matrix pipe 26% of it); 32768 SiC centres at 12/8: 3.80 -> 0.90 ms.  A wavefront per centre and
+// 47%, matrix pipe 27% of it); 32768 SiC centres at 12/8: 3.80 -> 0.90 ms.  A wavefront per centre and
 // 2 wavefronts per SIMD: with spills at 3 the reloads queue behind the data on their way (1.07 ms).
 // Up to l = 4, two species (183 to 190 registers cut to 168: 55296 centres at 5/4 868 -> 798 us)
 // and those not fixed at compile time (13440 centres of five at 5/4 1240 -> 928 us) take 3.
@@ -1080,7 +1080,11 @@ size_t soap_fast_lds_bytes(const SoapDev &sp) {
 
 // Centres a block takes in turn: several once the launch has many more blocks than the GPU
 // holds (2048 to 3072 wavefronts), so that a centre's data arrive while the one before is
-// worked on (batch512 adjoint: 1.73 ms without, 0.63 ms with; the tables then in LDS).
+// worked on and the tables are filled once; fewer blocks leave a longer last round.  Forward +
+// adjoint in us with 1, 2, 4 and 8: 8/6 of one species 53, 52, 65, 108 (4096 centres), 136, 132,
+// 147, 165 (13824), 292, 281, 277, 287 (32768), 580, 557, 543, 543 (64000), 1218, 1151, 1114, 1112
+// (135200); 12/8 of two 718, 712, 744, 811 (6912), 1623, 1621, 1613, 1669 (16384).  2 from 4096
+// centres on would gain 1 to 4% there in one species and lose as much in two.
 static int centres_per_block(int nc) { return nc >= 65536 ? 8 : nc >= 16384 ? 4 : 1; }
 
 bool launch_soap_fwd_fast(const SoapDev &sp, int nc, const int *centres, const int *Z, const int *nb_off,
